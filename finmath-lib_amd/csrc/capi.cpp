@@ -135,7 +135,7 @@ struct fm_lmm {
     bool uniform_dt = false;            // all simulation steps have the same length
     std::vector<std::vector<double>> berm_fixing;   // fixing dates of the Bermudans of the last pass
 
-    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_Y0cap, d_sqrt_dt, d_lvb, d_svs;
+    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_Y0cap, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
     DevBuf d_states, d_poly, d_dw, d_row_of, d_paths, d_num;
     DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib, d_out, d_swapmeta, d_scale;
     DevBuf d_ckpt, d_ckpt_first, d_seg, d_adj_num, d_kcur, d_fsig, d_sig, d_cdiag, d_wave_grad, d_grad_out;
@@ -167,6 +167,17 @@ struct fm_lmm {
     // spot measure, functional (or equivalent) Euler, loadings without local volatility:
     // the kernel the adjoint differentiates
     bool plain_euler() const { return !terminal() && !pc() && !carry_matters() && !has_lv && !has_sv; }
+    // FP64_LOGSTATE takes EULER without a cap as the functional scheme too: the log-state kernel
+    // caps log-states, so EULER with a finite cap, which caps only the value, is left to the
+    // general kernel
+    bool logstate() const {
+        return cfg.precision == FM_PRECISION_FP64_LOGSTATE && cfg.state_space == FM_STATE_SPACE_LOGNORMAL && !terminal() &&
+               !pc() && (!carry() || std::isinf(cfg.libor_cap)) && !has_lv && !has_sv;
+    }
+    // the FP64 spot kernel (lmm_spot64.hpp): base-2 log-forwards, its own record layout
+    bool spot64() const { return !fp32() && (plain_euler() || logstate()); }
+    // records per time step: the FP64 spot kernel reads them in pairs
+    int rec_n() const { return spot64() ? n() + (n() & 1) : n(); }
     size_t real_size() const { return fp32() ? sizeof(float) : sizeof(double); }
     int process_time_index(double t) const { return jsearch(times, round_tick(t)); }
     int libor_index(double t) const { return jsearch(tenor, round_tick(t)); }
@@ -269,14 +280,40 @@ void prepare_model(fm_lmm* c) {
     // records per (step i, component j): lambda_j.(t_i) zero-padded to the factor capacity,
     // variance*(-0.5) (0 in the normal state space), d/d and 1/d
     const int fcap = fcap_of(F), rs = rec_size_of(fcap);
-    std::vector<double> rec((size_t)nT * n * rs, 0.0);
+    // the FP64 spot kernel's records (lmm_spot64.hpp) scale each forward by its initial value (where
+    // that is an ordinary positive number) and hold no loadings for the forwards fixed at t_i
+    const bool spot64 = c->spot64();
+    const int rec_n = c->rec_n();
+    // (the spot kernel touches the records of the pair after the last one)
+    std::vector<double> rec(((size_t)nT * rec_n + 4) * rs, 0.0), lead((size_t)2 * n, 1.0), z0((size_t)n, 0.0);
+    std::vector<double> zcap((size_t)n, c->cfg.libor_cap);
+    for (int j = 0; j < n; j++) {
+        if (!lognormal) continue;
+        const double v = c->L0[(size_t)j];
+        if (v >= 1e-12 && v <= 1e12) { lead[(size_t)j] = v; lead[(size_t)(n + j)] = 1.0 / v; }
+        // log2(0) is a finite number whose power underflows to zero
+        else z0[(size_t)j] = v > 0.0 ? std::log2(v) : -1.0e9;
+        if (!std::isinf(c->cfg.libor_cap)) zcap[(size_t)j] = std::log2(c->cfg.libor_cap / lead[(size_t)j]);
+        z0[(size_t)j] = std::min(z0[(size_t)j], zcap[(size_t)j]);
+    }
     for (int i = 0; i < nT; i++)
-        for (int j = 0; j < n; j++) {
-            double* r = rec.data() + ((size_t)i * n + j) * rs;
-            for (int k = 0; k < F; k++) r[k] = c->lam[((size_t)i * n + j) * F + k];
-            r[fcap] = lognormal ? c->var[(size_t)i * n + j] * (-0.5) : 0.0;
+        for (int j = 0; j < rec_n; j++) {
+            double* r = rec.data() + ((size_t)i * rec_n + j) * rs;
+            if (j == n) { r[fcap + 1] = HUGE_VAL; r[fcap + 2] = 1.0; continue; }     // absent forward of the last pair
+            const bool fixed = spot64 && j < c->first_alive[(size_t)i];
+            if (!fixed) {
+                for (int k = 0; k < F; k++) r[k] = c->lam[((size_t)i * n + j) * F + k];
+                r[fcap] = lognormal ? c->var[(size_t)i * n + j] * (-0.5) : 0.0;
+            }
+            const double d = delta[(size_t)j];
+            if (spot64) {
+                r[fcap] *= (c->times[(size_t)i + 1] - c->times[(size_t)i]) * kLog2E;
+                r[fcap + 1] = zcap[(size_t)j];
+                r[fcap + 2] = 1.0 / d * lead[(size_t)(n + j)];
+                continue;
+            }
             // Scalar.of(+-d).discount(L, d) = 1/(L (d/(+-d)) + 1/(+-d)) (LMM:1145,1167)
-            const double d = delta[(size_t)j], m = c->terminal() ? -d : d;
+            const double m = c->terminal() ? -d : d;
             r[fcap + 1] = d / m;
             r[fcap + 2] = 1.0 / m;
         }
@@ -313,6 +350,10 @@ void prepare_model(fm_lmm* c) {
     if (!std::isinf(c->cfg.libor_cap))
         for (double& y : y0c) y = std::min(y, std::log(c->cfg.libor_cap));
     upload(c->d_Y0cap, y0c, s);
+    if (!lognormal) z0 = c->init_value;
+    z0.resize(80, 0.0);         // the register array's capacity
+    upload(c->d_z0, z0, s);
+    upload(c->d_lead, lead, s);
     // terminal measure N(T_0): the Scalar chain of the time-0 values (LMM:1028-1042,
     // stochastic/Scalar.java:320-328)
     c->n0_terminal = 1.0;
@@ -385,6 +426,7 @@ struct Lowered {
     std::vector<int> slot_k;                  // slot -> numeraire tenor index (single-date)
     std::vector<int32_t> swap_col0, swap_ncol, swap_slot;
     std::vector<int> contrib_k;               // contribution column -> numeraire tenor index
+    std::vector<double> walk;                 // walk tables of swaption groups, rows of eight (FP64 spot kernel)
 };
 
 // kcur of the kernel after the numeraire advance at time index ti
@@ -451,6 +493,41 @@ static void group_swaptions(Lowered& L) {
             }
         }
         i = e;
+    }
+}
+
+// Walk tables of the FP64 spot kernel (SwaptionWalk, lmm_spot64.hpp): at each time index the first
+// group whose periods are discounted over their tenor periods is valued by that index's Euler step.
+// A second group, and one exercised at the last time index (which has no step), keep a walk of
+// their own. The period lengths are tick-rounded dates' differences, hence the tolerance.
+static void make_walks(const fm_lmm* c, Lowered& L) {
+    for (KProduct& k : L.kp) k.walk = -1;
+    if (!c->spot64()) return;
+    int last = -1;          // time index of the last group that got a walk
+    for (size_t i = 0; i < L.kp.size(); i += 1 + (size_t)(L.kp[i].type == FM_PRODUCT_SWAPTION ? L.kp[i].pad2 : 0)) {
+        KProduct& k = L.kp[i];
+        if (k.type != FM_PRODUCT_SWAPTION || k.eval_index >= c->nT() || k.eval_index == last) continue;
+        bool tenor_periods = true;
+        for (int q = 0; q < k.num_periods; q++) {
+            const size_t j = (size_t)(k.first_j + q);
+            const double d = c->tenor[j + 1] - c->tenor[j];
+            if (!(std::fabs(L.per[(size_t)(k.param_off + q)].tau - d) <= 1e-14 * d)) tenor_periods = false;
+        }
+        if (!tenor_periods) continue;
+        last = k.eval_index;
+        k.walk = (int32_t)(L.walk.size() / 8);
+        double adj = 1.0;
+        for (int q = 0; q < k.num_periods; q++) {
+            const KPeriod& pe = L.per[(size_t)(k.param_off + q)];
+            const double v = c->L0[(size_t)(k.first_j + q)];
+            const bool scaled = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL && v >= 1e-12 && v <= 1e12;
+            const double s = scaled ? v : 1.0;
+            adj *= pe.adj;
+            double row[8] = {s * pe.period_length * adj, 0, 0, 0, 0, 0, 0, 0};
+            for (int g = 0; g < kSwaptionGroup; g++)
+                row[1 + g] = g <= k.pad2 ? L.per[(size_t)(L.kp[i + (size_t)g].param_off + q)].strike / s : 0.0;
+            L.walk.insert(L.walk.end(), row, row + 8);
+        }
     }
 }
 
@@ -666,6 +743,7 @@ Lowered lower_products(fm_lmm* c, const fm_product* prods, int count) {
     }
     std::stable_sort(L.kp.begin(), L.kp.end(), [](const KProduct& a, const KProduct& b) { return a.eval_index < b.eval_index; });
     group_swaptions(L);
+    make_walks(c, L);
     return L;
 }
 
@@ -862,6 +940,7 @@ size_t external_scratch_bytes(const fm_lmm* c, const Lowered& L) {
     const size_t num_waves = ((size_t)c->P() + 63) / 64, stride = (size_t)L.num_slots + c->n() + 1;
     return 2 * ExternalScratch::piece(num_waves * stride * sizeof(double)) +
            ExternalScratch::piece(L.kp.size() * sizeof(KProduct)) + ExternalScratch::piece(L.per.size() * sizeof(KPeriod)) +
+           ExternalScratch::piece(L.walk.size() * sizeof(double)) +
            ExternalScratch::piece(stride * 2 * sizeof(double));
 }
 
@@ -929,16 +1008,15 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.ckpt_stride = ckpt ? ckpt_stride : 1;
     a.ckpt_first = ckpt_first;
     tm.mark(2);
+    const bool lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL;
     // kernel variant: the spot-measure Euler kernels, else the general kernel (terminal
     // measure, carried state, predictor-corrector)
-    // the log-forward kernel caps the log-state, as EULER_FUNCTIONAL does up to rounding;
-    // EULER with a finite cap caps only the value and runs on the general kernel
-    const bool logstate_kernel = c->cfg.precision == FM_PRECISION_FP64_LOGSTATE &&
-        c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL && !c->terminal() && !c->pc() &&
-        (!c->carry() || std::isinf(c->cfg.libor_cap)) && !c->has_lv && !c->has_sv;
-    if (logstate_kernel) {
-        a.Y0 = c->d_Y0cap.as<double>();
-        launch_lmm_step_fp64_logstate(a, s);
+    a.rec_n = c->rec_n();
+    if (c->spot64()) {
+        a.Y0 = c->d_z0.as<double>();
+        a.lead = c->d_lead.as<double>();
+        a.walk = xs ? xs->upload(L.walk, s) : upload(c->d_walk, L.walk, s);
+        launch_lmm_step_fp64(a, s);
     } else if (c->has_lv || c->has_sv) {
         a.lv_alpha = c->lv_alpha;
         a.lvb = c->has_lv ? c->d_lvb.p : nullptr;
@@ -946,12 +1024,8 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
         if (c->fp32()) launch_lmm_step_lv_fp32(a, s);
         else launch_lmm_step_lv_fp64(a, s);
     } else if (c->plain_euler()) {
-        // the spot kernel's initial states: FP64 log-normal the log-forwards capped at log(cap),
-        // otherwise the capped initial forwards
-        a.Y0 = (!c->fp32() && c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL) ? c->d_Y0cap.as<double>()
-                                                                               : c->d_L0.as<double>();
-        if (c->fp32()) launch_lmm_step_fp32(a, s);
-        else launch_lmm_step_fp64(a, s);
+        a.Y0 = c->d_L0.as<double>();            // the capped initial forwards
+        launch_lmm_step_fp32(a, s);
     } else {
         // the general kernel: FP64 log-normal functional schemes carry the log-forwards, capped
         // at log(cap), like the spot kernel
@@ -1570,6 +1644,8 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
     a.capped = std::isinf(c->cfg.libor_cap) ? 0 : 1;
     a.delta = c->d_delta.as<double>();
     a.L0 = c->d_L0.as<double>(); a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
+    a.rec_n = c->rec_n();
+    a.lead = c->d_lead.as<double>();
     a.num_products = (int)kp.size();
     a.products = upload(c->d_products, kp, s);
     a.periods = upload(c->d_periods, L.per, s);

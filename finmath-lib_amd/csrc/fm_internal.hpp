@@ -12,6 +12,8 @@
 
 namespace fm {
 
+constexpr double kLog2E = 1.4426950408889634074;      // 1 / ln 2
+
 // Error carried to the C ABI as a status code plus message.
 struct FmError : std::runtime_error {
     int code;
@@ -76,6 +78,8 @@ struct KProduct {
     int32_t param_off;    // offset into the per-period parameter table
     int32_t pad2;         // swaption: number of following swaptions valued with it (pricing);
                           // adjoint Bermudan period: the Bermudan's index
+    int32_t walk;         // FP64 spot kernel: first row of the group's walk table (lmm_spot64.hpp), or -1
+    int32_t pad3;
 };
 
 // Swaptions valued together by one walk over their shared periods (KProduct.pad2 of the first
@@ -98,13 +102,16 @@ struct StepArgs {
     const int32_t* first_alive;  // device nT
     const int32_t* tenor_time_index; // device n+1: process time index of T_k (rounded up)
     const void* rec;             // device [nT][n][rec_size_of(fcap_of(F))] records (double or float)
+    int rec_n;                   // records per time step (n, or n rounded up to even for the FP64 spot kernel)
     int lognormal, capped;       // state space is LOGNORMAL; the liborCap applies
     const double* delta;         // device n: T_{j+1}-T_j
     const double* L0;            // device n: initial forwards in value space
+    const double* lead;          // FP64 spot kernel, device [2][n]: the forwards' scales s_j and 1/s_j
+    const double* walk;          // FP64 spot kernel, device [rows][8]: walk tables of swaption groups
     const double* Y0;            // device n: initial states (log(max(L0, 0)) or L0) of the carried schemes;
                                  // for the log-forward and spot kernels kept below log(cap)
                                  // (the spot kernel in the normal state space: the capped forwards)
-    double logcap;               // log(cap) for the log-forward kernel
+    double logcap;               // the cap of a carried log-value: log(cap), log2(cap) for the FP64 spot kernel
     int terminal;                // TERMINAL measure (general kernel)
     int carry;                   // EULER / PREDICTOR_CORRECTOR: the state is carried (general kernel)
     int pc;                      // predictor-corrector (general kernel)
@@ -134,7 +141,6 @@ struct StepArgs {
 };
 void launch_lmm_step_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_fp32(const StepArgs& a, void* stream);
-void launch_lmm_step_fp64_logstate(const StepArgs& a, void* stream);
 // General variant (terminal measure, carried state, predictor-corrector), see lmm_step.hpp.
 void launch_lmm_step_general_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_general_fp32(const StepArgs& a, void* stream);

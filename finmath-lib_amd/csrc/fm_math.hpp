@@ -71,4 +71,43 @@ __device__ __forceinline__ double fm_div_nr_r(double a, double b, double r) {
 
 __device__ __forceinline__ double fm_div_nr(double a, double b) { return fm_div_nr_r(a, b, fm_rcp_nr(b)); }
 
+// The coefficients of fm_exp2 in scalar registers, made once before a kernel's loops (an FP64 operand
+// cannot be a literal on this target). The empty asm hides their values: as known constants the
+// compiler copies each into vector registers for an accumulating multiply-add, two moves more per
+// Horner step.
+struct Exp2Coef {
+    double c1, c2, c3, c4, c5, c6, c7, c8, c9, c10, c11;
+    __device__ __forceinline__ Exp2Coef()
+        : c1(0x1.62e42fefa39f3p-1), c2(0x1.ebfbdff82c598p-3), c3(0x1.c6b08d7048f31p-5), c4(0x1.3b2ab6fba1e1cp-7),
+          c5(0x1.5d87fe7bbbe09p-10), c6(0x1.43091309610fcp-13), c7(0x1.ffcbee3b0a61cp-17), c8(0x1.62bfd49ededd3p-20),
+          c9(0x1.b54167a1b0034p-24), c10(0x1.e605f964b639dp-28), c11(0x1.c063841f3a21dp-32) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm("" : "+s"(c1), "+s"(c2), "+s"(c3), "+s"(c4), "+s"(c5), "+s"(c6));
+        asm("" : "+s"(c7), "+s"(c8), "+s"(c9), "+s"(c10), "+s"(c11));
+#endif
+    }
+};
+
+// 2^x. x = n + r with n the nearest integer (both exact), 2^r = 1 + r q(r) with q the minimax
+// polynomial of degree 10 on [-1/2, 1/2] (relative error below 1.8e-17, Remez exchange in 60-digit
+// arithmetic), scaled by ldexp, which also gives the underflow to zero and the overflow to
+// infinity: within one unit in the last place. NaN propagates; an infinite x gives NaN, so a state
+// that stands for log2(0) is held as the lowest finite number instead.
+__device__ __forceinline__ double fm_exp2(double x, const Exp2Coef& k) {
+    const double n = __builtin_rint(x);
+    const double r = x - n;
+    double p = fma(k.c11, r, k.c10);
+    p = fma(p, r, k.c9);
+    p = fma(p, r, k.c8);
+    p = fma(p, r, k.c7);
+    p = fma(p, r, k.c6);
+    p = fma(p, r, k.c5);
+    p = fma(p, r, k.c4);
+    p = fma(p, r, k.c3);
+    p = fma(p, r, k.c2);
+    p = fma(p, r, k.c1);
+    p = fma(p, r, 1.0);
+    return __builtin_amdgcn_ldexp(p, (int)n);
+}
+
 } // namespace fm

@@ -188,7 +188,7 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
     const Variant<real> var{lognormal, capped, carry, cap, (real)a.logcap, (real)a.lv_alpha,
                             LV ? (const real*)a.lvb : nullptr, LV ? (const real*)a.svs : nullptr};
     // the array holds log-values, states (carried schemes) or values; val gives the value
-    auto val = [&](real x) -> real {
+    auto val = [&](real x, int) -> real {
         return LOGCARRY ? dev_exp<real>(x) : (carry ? to_value<real>(x, lognormal, capped, cap) : x);
     };
 
@@ -213,7 +213,7 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
             const size_t base = (size_t)(ti / a.ckpt_stride) * n;
             static_for<0, W * NCH>([&](auto J) {
                 constexpr int j = decltype(J)::value;
-                if (j < n) ckpt[(base + j) * P + p] = val(X.template at<j>());
+                if (j < n) ckpt[(base + j) * P + p] = val(X.template at<j>(), j);
             });
         }
         if constexpr (TERMINAL) {
@@ -229,7 +229,7 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
                     const int l1 = n < W * q + W ? n : W * q + W;
 #pragma unroll 1
                     for (int l = l0; l < l1; l++) {
-                        const double Ll = (double)val(X.template ch<q>()[l - W * q]);
+                        const double Ll = (double)val(X.template ch<q>()[l - W * q], l);
                         const double dl = delta[l];
                         if (ti == 0) Nn = 1.0 / (Ll * (dl / Nn) + 1.0 / Nn);
                         else if (l == kcur) Nn = 1.0 / (Ll * dl + 1.0);
@@ -246,7 +246,7 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
         } else {
             // ---- N(T_{k+1}) = N(T_k).accrue(L_k(T_k), d_k) once L_k is final (LMM:1050-1066)
             while (kcur < n && tenor_ti[kcur] <= ti) {
-                const double Lk = (double)val(X.get(kcur));
+                const double Lk = (double)val(X.get(kcur), kcur);
                 const double dk = delta[kcur];
                 double Nn;
                 if (kcur == 0)      Nn = Lk * (dk * 1.0) + 1.0;      // Scalar.accrue of Scalar 1.0
@@ -263,8 +263,9 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
         // terminal and predictor-corrector kernels (measured 4-5% faster there; slower in FP32
         // and in the spot Euler kernel)
         constexpr bool group = sizeof(real) == 8 && (TERMINAL || PC);
-        eval_products_at<group, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
-                                           active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P);
+        int walk = -1;
+        eval_products_at<group, false, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
+                                                  active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P, walk);
 
         if (ti == nT) break;
 

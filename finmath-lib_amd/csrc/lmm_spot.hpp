@@ -27,20 +27,10 @@
 // step's model records are read through the scalar cache, one 64-byte record per component.
 #pragma once
 
-#include <type_traits>
-
 #include "lmm_step.hpp"
 #include "hip_check.hpp"
 
 namespace fm {
-
-template <int I, int N, typename Fn>
-__device__ __forceinline__ void static_for(Fn&& fn) {
-    if constexpr (I < N) {
-        fn(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(fn);
-    }
-}
 
 // Forwards per chunk: a chunk is sixteen VGPRs, eight FP64 or sixteen FP32 forwards. At this
 // width the compiler reads and writes an element at a uniform run-time index with one indexed
@@ -124,7 +114,6 @@ __device__ __forceinline__ void spot_step(ChunkedForwards<NCH, real>& Y, int n, 
                                           const real (&dW)[FCAP], const real* __restrict__ rec,
                                           bool capped, real ycap, real* __restrict__ paths,
                                           const int32_t* __restrict__ row_next, int64_t p, int P, bool active) {
-    constexpr bool LOGCARRY = carries_log<real>();
     constexpr int W = chunk_width<real>();
     real S[FCAP];
 #pragma unroll
@@ -137,7 +126,7 @@ __device__ __forceinline__ void spot_step(ChunkedForwards<NCH, real>& Y, int n, 
         for (int j = j0; j < j1; j++) {
             const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, n, i, j);
             const real x = Y.template ch<q>()[j - W * q];
-            const real Lj = (LOGCARRY && lognormal) ? dev_exp<real>(x) : x;
+            const real Lj = x;
             real w = spot_div<real>((real)1.0, Lj * R.c1() + R.c2());
             if (lognormal) w = w * Lj;
 #pragma unroll
@@ -146,42 +135,44 @@ __device__ __forceinline__ void spot_step(ChunkedForwards<NCH, real>& Y, int n, 
 #pragma unroll
             for (int k = 1; k < FCAP; k++) mu = mu + S[k] * R.lam(k);
             mu = mu + R.hv();
-            real y = (!LOGCARRY && lognormal) ? dev_log<real>(Lj) : x;
+            real y = lognormal ? dev_log<real>(Lj) : x;
             y = y + mu * dt;
 #pragma unroll
             for (int k = 0; k < FCAP; k++) y = y + dW[k] * R.lam(k);
-            if (LOGCARRY) {
-                if (capped) y = jmin(y, ycap);
-                Y.template ch<q>()[j - W * q] = y;
-                if (paths && active) paths[(size_t)row_next[j] * P + p] = lognormal ? dev_exp<real>(y) : y;
-            } else {
-                real v = lognormal ? dev_exp<real>(y) : y;
-                if (capped) v = jmin(v, ycap);
-                Y.template ch<q>()[j - W * q] = v;
-                if (paths && active) paths[(size_t)row_next[j] * P + p] = v;
-            }
+            real v = lognormal ? dev_exp<real>(y) : y;
+            if (capped) v = jmin(v, ycap);
+            Y.template ch<q>()[j - W * q] = v;
+            if (paths && active) paths[(size_t)row_next[j] * P + p] = v;
         }
     });
 }
 
 // Products evaluated at time index ti, in the order they were lowered (qp advances over them):
 // swaptions and caplets are reduced into their wave partials, swap periods and Bermudan
-// regression bases go to per-path contribution columns. Y holds the path's states and val(y)
+// regression bases go to per-path contribution columns. Y holds the path's states and val(y, j)
 // gives the forward L_j(t_ti) of state y; N and Nprev are the numeraires N(T_knum) and the one
 // before it. GROUP values a swaption group in one walk; without it every member walks its own
 // copy of the periods (the FP32 kernels: the shared walk measured slower there).
-template <bool GROUP, int NCH, typename real, typename Val>
-__device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_products, const KProduct* __restrict__ products,
-                                                 const KPeriod* __restrict__ periods, const double* __restrict__ delta,
+// WALK: a swaption group with a walk table is left to the step (its index is returned in walk).
+template <bool GROUP, bool WALK, int NCH, typename real, typename Val, typename Products, typename Periods, typename Doubles>
+__device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_products, Products products,
+                                                 Periods periods, Doubles delta,
                                                  double N, double Nprev, int knum, ChunkedForwards<NCH, real>& Y,
                                                  Val&& val, bool active, int cnt, int lane, int64_t wave,
                                                  double* __restrict__ wave_sum, double* __restrict__ wave_m2,
-                                                 int stride, double* __restrict__ contrib, int64_t p, int P) {
+                                                 int stride, double* __restrict__ contrib, int64_t p, int P, int& walk) {
     constexpr int W = chunk_width<real>();
-    auto value_of = [&](int j) -> real { return val(Y.get(j)); };
+    auto value_of = [&](int j) -> real { return val(Y.get(j), j); };
     while (qp < num_products && products[qp].eval_index == ti) {
         const KProduct pr = products[qp];
         qp++;
+        if constexpr (WALK) {
+            if (pr.walk >= 0) {         // valued by the step's own walk (SwaptionWalk)
+                walk = qp - 1;
+                qp += pr.pad2;
+                continue;
+            }
+        }
         const double Nsel = (pr.num_k == knum) ? N : Nprev;
         if (pr.type == FM_PRODUCT_SWAPTION) {
             // Swaption.java:150-190: the periods backwards, value = (value + payoff) / (1 + L tau) * adj.
@@ -202,7 +193,7 @@ __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_produc
 #pragma unroll 1
                 for (int j = jb - 1; j >= ja; j--) {
                     const KPeriod pe = periods[pr.param_off + (j - j0)];
-                    const real Lj = val(Y.template ch<q>()[j - W * q]);
+                    const real Lj = val(Y.template ch<q>()[j - W * q], j);
                     const real b = (real)1.0 + Lj * (real)pe.tau;
                     const real r = spot_rcp<real>(b);
                     // every member's strike and notional are read up front (indices clamped to the
@@ -290,11 +281,7 @@ __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_produc
     }
 }
 
-// BUILD tells apart instantiations compiled with different floating-point flags (0: without
-// contraction, the FP64 and FP32-mixed builds; 1: with fused multiply-add, FP64_LOGSTATE). Two
-// translation units that instantiated one kernel under one name with different flags would
-// give one definition to both: the linker keeps a single copy of a template instantiation.
-template <int NCH, int FCAP, typename real, bool lognormal, int BUILD = 0>
+template <int NCH, int FCAP, typename real, bool lognormal>
 __global__ void __launch_bounds__(kStepThreads)
 lmm_spot_kernel(const StepArgs a, const real* __restrict__ rec, const double* __restrict__ delta,
                 const double* __restrict__ times, const int32_t* __restrict__ first_alive,
@@ -315,10 +302,9 @@ lmm_spot_kernel(const StepArgs a, const real* __restrict__ rec, const double* __
     const int cnt = (int)((int64_t)P - wave * 64 > 64 ? 64 : ((int64_t)P - wave * 64));
     const int stride = a.num_slots + n + 1;
     const bool capped = a.capped != 0;
-    constexpr bool LOGCARRY = carries_log<real>();
     constexpr int W = chunk_width<real>();
-    const real ycap = (LOGCARRY && lognormal) ? (real)a.logcap : (real)a.cap;
-    auto val = [&](real y) -> real { return (LOGCARRY && lognormal) ? dev_exp<real>(y) : y; };
+    const real ycap = (real)a.cap;
+    auto val = [&](real y, int) -> real { return y; };
 
     ChunkedForwards<NCH, real> Y;
     static_for<0, W * NCH>([&](auto J) {
@@ -343,7 +329,7 @@ lmm_spot_kernel(const StepArgs a, const real* __restrict__ rec, const double* __
         }
         // ---- N(T_{k+1}) = N(T_k).accrue(L_k(T_k), d_k) once L_k is final (LMM:1050-1066)
         while (kcur < n && tenor_ti[kcur] <= ti) {
-            const double Lk = (double)val(Y.get(kcur));
+            const double Lk = (double)Y.get(kcur);
             const double dk = delta[kcur];
             double Nn;
             if (kcur == 0)      Nn = Lk * (dk * 1.0) + 1.0;      // Scalar.accrue of Scalar 1.0
@@ -356,9 +342,9 @@ lmm_spot_kernel(const StepArgs a, const real* __restrict__ rec, const double* __
             if (numeraire_out && active) numeraire_out[(size_t)kcur * P + p] = N;
         }
         // ---- products evaluated at this time index
-        constexpr bool group = sizeof(real) == 8;
-        eval_products_at<group, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, Y, val,
-                                           active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P);
+        int walk = -1;
+        eval_products_at<false, false, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, Y, val,
+                                                  active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P, walk);
 
         if (ti == nT) break;
 
@@ -372,43 +358,40 @@ lmm_spot_kernel(const StepArgs a, const real* __restrict__ rec, const double* __
     }
 }
 
-template <int NCH, int FCAP, typename real, bool lognormal, int BUILD>
+template <int NCH, int FCAP, typename real, bool lognormal>
 void launch_spot_ss(const StepArgs& a, hipStream_t stream) {
     const int64_t blocks = ((int64_t)a.P + kStepThreads - 1) / kStepThreads;
-    hipLaunchKernelGGL((lmm_spot_kernel<NCH, FCAP, real, lognormal, BUILD>), dim3((unsigned)blocks), dim3(kStepThreads), 0,
+    hipLaunchKernelGGL((lmm_spot_kernel<NCH, FCAP, real, lognormal>), dim3((unsigned)blocks), dim3(kStepThreads), 0,
                        stream, a, (const real*)a.rec, a.delta, a.times, a.first_alive, a.tenor_time_index, a.products,
                        a.periods, (const real*)a.dw, a.wave_sum, a.wave_m2, a.contrib, (real*)a.paths, a.row_of,
                        a.numeraire, (real*)a.ckpt);
     HIP_CHECK(hipGetLastError());
 }
 
-template <int NCH, int FCAP, typename real, int BUILD>
+template <int NCH, int FCAP, typename real>
 void launch_spot_cap(const StepArgs& a, hipStream_t stream) {
-    if (a.lognormal) launch_spot_ss<NCH, FCAP, real, true, BUILD>(a, stream);
-    else launch_spot_ss<NCH, FCAP, real, false, BUILD>(a, stream);
+    if (a.lognormal) launch_spot_ss<NCH, FCAP, real, true>(a, stream);
+    else launch_spot_ss<NCH, FCAP, real, false>(a, stream);
 }
 
-template <int NCH, typename real, int BUILD>
+template <int NCH, typename real>
 void launch_spot_n(const StepArgs& a, hipStream_t stream) {
-    if (a.F <= 1) launch_spot_cap<NCH, 1, real, BUILD>(a, stream);
-    else if (a.F <= 3) launch_spot_cap<NCH, 3, real, BUILD>(a, stream);
-    else if (a.F <= 5) launch_spot_cap<NCH, 5, real, BUILD>(a, stream);
-    else if (a.F <= 10) launch_spot_cap<NCH, 10, real, BUILD>(a, stream);
+    if (a.F <= 1) launch_spot_cap<NCH, 1, real>(a, stream);
+    else if (a.F <= 3) launch_spot_cap<NCH, 3, real>(a, stream);
+    else if (a.F <= 5) launch_spot_cap<NCH, 5, real>(a, stream);
+    else if (a.F <= 10) launch_spot_cap<NCH, 10, real>(a, stream);
     else throw FmError(FM_ERR_UNSUPPORTED, "number of factors above 10 is not supported by the path kernel");
 }
 
-// The spot Euler kernel of the pricing and simulation passes. a.Y0 holds the initial states:
-// FP64 log-normal the log-forwards capped at log(cap) (a.logcap = log(cap)), otherwise the
-// capped initial forwards.
-template <typename real, int BUILD = 0>
+// The spot Euler kernel of the pricing and simulation passes, FP32-mixed; a.Y0 holds the capped
+// initial forwards.
+template <typename real>
 void launch_spot(const StepArgs& a, hipStream_t stream) {
-    // 1, 3, 5, 10 chunks of eight FP64 forwards; 1, 2, 3, 5 chunks of sixteen FP32 forwards
-    constexpr int W = chunk_width<real>();
-    constexpr int N2 = W == 8 ? 3 : 2, N3 = W == 8 ? 5 : 3, N4 = W == 8 ? 10 : 5;
-    if (a.n <= W) launch_spot_n<1, real, BUILD>(a, stream);
-    else if (a.n <= W * N2) launch_spot_n<N2, real, BUILD>(a, stream);
-    else if (a.n <= W * N3) launch_spot_n<N3, real, BUILD>(a, stream);
-    else if (a.n <= 80) launch_spot_n<N4, real, BUILD>(a, stream);
+    constexpr int W = chunk_width<real>();      // 1, 2, 3, 5 chunks of sixteen forwards
+    if (a.n <= W) launch_spot_n<1, real>(a, stream);
+    else if (a.n <= W * 2) launch_spot_n<2, real>(a, stream);
+    else if (a.n <= W * 3) launch_spot_n<3, real>(a, stream);
+    else if (a.n <= 80) launch_spot_n<5, real>(a, stream);
     else throw FmError(FM_ERR_UNSUPPORTED, "more than 80 forward rates are not supported by the path kernel");
 }
 

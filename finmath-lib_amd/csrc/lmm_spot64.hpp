@@ -1,0 +1,309 @@
+// The Euler step of the FP64 spot kernel (lmm_spot.hpp), also run by its reverse sweep.
+//
+// The state of a forward is z_j = log2(L_j / s_j) with the scale s_j its initial value (1 where that
+// is not positive; in the normal state space the state is the forward itself and s_j = 1): the
+// exponential of a step needs no scaling of its argument, and a state near zero is rounded more
+// finely than a logarithm of the forward. With E_j = L_j / s_j and c = 1/ln 2 (E_j = z_j and c = 1 in
+// the normal state space) the step of an alive component is
+//   E_j = 2^z_j
+//   w   = c dt E_j / (E_j + e_j)               e_j = 1/(d_j s_j); c dt / (E_j + e_j) in the normal
+//   T_k = T_k + w lambda_jk                    ascending j, from T_k = c dW_k
+//   z_j = z_j + (h_j + sum_k T_k lambda_jk)    h_j = -1/2 variance_j c dt, 0
+//   z_j = min(z_j, log2(cap / s_j))
+// which is the drift and the diffusion of lmm_spot.hpp taken together: sum_k (c dt S_k + c dW_k)
+// lambda_jk, with S_k the reference's factor sums. One pair of multiply-adds per factor replaces two
+// products and two sums in the drift and one of each in the diffusion, and the state takes one
+// rounding per step instead of one per factor. The record of (t_i, j) holds lambda_jk, h_j, the cap
+// of z_j and e_j.
+//
+// The components are processed in pairs, unrolled over the register array: a pair's two exponentials
+// and reciprocals are independent, which hides the latency of the FP64 pipeline and of the scalar
+// loads of the two records, and a constant register index needs no indexed moves. A pair holds a
+// fixed or absent forward beside an alive one where the alive range starts or ends at an odd
+// index: its record has no loadings, so it adds an exact zero to every sum and to its state.
+//
+// Swaptions that exercise at t_i over consecutive tenor periods are valued by the same walk
+// (SwaptionWalk): it has E_j and the reciprocal at hand, so a period of a swaption costs two
+// operations and three more that its group shares, where a walk of its own needs another
+// exponential and another reciprocal.
+//
+// The kernel is bound by the FP64 vector pipeline. At 40 forwards x 5 factors x 1,000,000 paths with 30
+// swaptions it issues 38,500 vector instructions per wavefront (80,400 with rolled component loops,
+// a general exponential and separate products and sums) and takes 1.65 ms (3.46 ms), the vector ALUs
+// 0.73 busy (0.67) at four wavefronts per SIMD (three): the registers are held to 128 by reading the
+// kernel's arguments where they are used and the increments when the step begins. Bringing the next
+// pair's records into the scalar cache took it from 1.88 to 1.79 ms at three wavefronts; two sets of
+// scalar registers for them instead spilled.
+#pragma once
+
+#include "lmm_spot.hpp"
+
+namespace fm {
+
+typedef const double __attribute__((address_space(4)))* RecPtr;
+
+// A record read whole into scalar registers (64-byte pieces).
+template <int FCAP>
+struct RecVec {
+    typedef double V __attribute__((ext_vector_type(8)));
+    static constexpr int size = rec_size_of(FCAP);
+    static constexpr int N = (size + 7) / 8;
+    V v[N];
+    // record j of a time step whose first record is at rec
+    __device__ __forceinline__ RecVec(RecPtr rec, int j) {
+        typedef const V __attribute__((address_space(4)))* P;
+#pragma unroll
+        for (int q = 0; q < N; q++) v[q] = *(P)(rec + j * size + 8 * q);
+    }
+    __device__ __forceinline__ double at(int e) const { return v[e / 8][e % 8]; }
+    __device__ __forceinline__ double lam(int k) const { return at(k); }
+    __device__ __forceinline__ double h() const { return at(FCAP); }
+    __device__ __forceinline__ double zcap() const { return at(FCAP + 1); }
+    __device__ __forceinline__ double e() const { return at(FCAP + 2); }
+};
+
+// Up to kSwaptionGroup swaptions exercised at one time index over the periods [j0, j0 + periods):
+//   V_g = sum_j P_j a_j (E_j - k_gj),   P_j = prod_{l <= j} 1/(1 + L_l d_l) = prod_{l <= j} e_l / (E_l + e_l)
+// with a_j = s_j x period length x the discounting adjustments up to j and k_gj = strike / s_j, one
+// table row {a, k_0 .. k_3, -, -, -} per period. V_g is the value of Swaption.java:150-190 for a
+// notional of 1, its backward recursion written out as a sum.
+struct SwaptionWalk {
+    RecPtr table;
+    int j0 = 0, periods = 0;
+    double P = 1.0, V[kSwaptionGroup] = {0.0, 0.0, 0.0, 0.0};
+    __device__ __forceinline__ void period(int j, double E, double e, double r) {
+        if ((unsigned)(j - j0) >= (unsigned)periods) return;
+        typedef double Row __attribute__((ext_vector_type(8)));
+        typedef const Row __attribute__((address_space(4)))* RowPtr;
+        const Row row = *(RowPtr)(table + 8 * (j - j0));
+        P = P * (e * r);
+        const double Pa = P * row[0];
+#pragma unroll
+        for (int g = 0; g < kSwaptionGroup; g++) V[g] = fma(E - row[1 + g], Pa, V[g]);
+    }
+};
+
+// One Euler step of the alive components [first, n), in place. WALK: the walk's swaptions are valued
+// on the states before the step, which also passes over their forwards that are fixed at t_i.
+template <int NCH, int FCAP, bool lognormal, bool WALK, typename Chunks>
+__device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, int first, double dt,
+                                            const double (&dW)[FCAP], const double* rec, const Exp2Coef& ke,
+                                            SwaptionWalk* sw) {
+    RecPtr recs = (RecPtr)(uintptr_t)(rec + (size_t)i * rec_n * RecVec<FCAP>::size);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(recs));      // one base address for the step's records
+#endif
+    const double cdt = lognormal ? dt * kLog2E : dt;
+    double T[FCAP];
+#pragma unroll
+    for (int k = 0; k < FCAP; k++) T[k] = lognormal ? dW[k] * kLog2E : dW[k];
+    // 1 / b by the hardware reciprocal r0 corrected to third order: with e = 1 - b r0,
+    // 1/b = r0 (1 + e + e^2 + ...); |e| < 2^-20, so the terms left out are below rounding
+    auto reciprocal = [&](double b) -> double {
+        const double r0 = __builtin_amdgcn_rcp(b);
+        const double e = fma(-b, r0, 1.0);
+        return fma(r0, fma(e, e, e), r0);
+    };
+    auto increment = [&](double w, const RecVec<FCAP>& R) -> double {
+#pragma unroll
+        for (int k = 0; k < FCAP; k++) T[k] = fma(w, R.lam(k), T[k]);
+        double inc = R.h();
+#pragma unroll
+        for (int k = 0; k < FCAP; k++) inc = fma(T[k], R.lam(k), inc);
+        return inc;
+    };
+    if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
+    const unsigned alive = (unsigned)(n - first + 1);
+    static_for<0, 4 * NCH>([&](auto Q) {
+        constexpr int j = 2 * decltype(Q)::value;
+        if ((unsigned)(j + 1 - first) < alive) {        // j + 1 >= first and j < n
+            const RecVec<FCAP> R0(recs, j), R1(recs, j + 1);
+            __builtin_amdgcn_sched_barrier(0);          // both records are requested before the exponentials
+            const double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
+            const double E0 = lognormal ? fm_exp2(x0, ke) : x0;
+            const double E1 = lognormal ? fm_exp2(x1, ke) : x1;
+            const double b0 = E0 + R0.e(), b1 = E1 + R1.e();
+            // the next pair's records are brought into the scalar cache while this one runs (the table
+            // of a model is several times that cache); a pair beyond the last reads its last record
+            __builtin_amdgcn_sched_barrier(0);
+            typedef const volatile uint32_t __attribute__((address_space(4)))* WordPtr;
+            constexpr int step = RecVec<FCAP>::size;
+            uint32_t t0 = *(WordPtr)(recs + (j + 2) * step), t1 = *(WordPtr)(recs + (j + 3) * step);
+            const double r0 = reciprocal(b0), r1 = reciprocal(b1);
+            if constexpr (WALK) {
+                if (sw->periods > 0) {
+                    sw->period(j, E0, R0.e(), r0);
+                    sw->period(j + 1, E1, R1.e(), r1);
+                }
+            }
+            double y0 = x0 + increment((lognormal ? cdt * E0 : cdt) * r0, R0);
+            double y1 = x1 + increment((lognormal ? cdt * E1 : cdt) * r1, R1);
+            // the cap seldom binds: one comparison each (min(y, cap) keeps NaN, as a comparison does)
+            if (__builtin_amdgcn_ballot_w64(y0 > R0.zcap() || y1 > R1.zcap()) != 0) {
+                asm volatile("");       // a branch, not selects
+                y0 = jmin(y0, R0.zcap());
+                y1 = jmin(y1, R1.zcap());
+            }
+            Y.template put<j>(y0);
+            Y.template put<j + 1>(y1);
+#if defined(__HIP_DEVICE_COMPILE__)
+            asm volatile("" :: "s"(t0), "s"(t1));
+#endif
+        }
+    });
+}
+
+// The spot kernel in FP64: one thread per path, its states in NCH chunks of eight doubles. Per time
+// index: checkpoints (the adjoint's forward pass), numeraire updates, the products evaluated there,
+// the Euler step with its swaption walk, and the new forwards when the process is stored.
+template <int NCH, int FCAP, bool lognormal>
+__global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(NCH <= 5 && FCAP <= 5 ? 4 : 1)))
+lmm_spot64_kernel(const StepArgs) {
+    constexpr int W = chunk_width<double>();
+    ArgPtr a = kernel_arguments();
+    const uint32_t p0 = blockIdx.x * (uint32_t)kStepThreads + threadIdx.x;      // P < 2^31
+    const int lane = threadIdx.x & 63;
+    // the wavefront index, uniform: kept in a scalar register
+    const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Exp2Coef ke;
+
+    ChunkedForwards<NCH, double> Y;
+    {
+        const ConstArray<double> z0{a->Y0};
+        static_for<0, W * NCH>([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            Y.template put<j>(z0[j]);           // zeros beyond the n forwards
+            if constexpr (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);    // a chunk's scalar loads at a time
+        });
+    }
+    double N = 1.0, Nprev = 1.0;   // unadjusted numeraire N(T_knum) and the one before it
+    int kcur = 0, knum = 0;
+    int qp = 0;
+    for (int ti = 0;; ti++) {
+        a = kernel_arguments();
+        const int P = a->P, n = a->n;
+        const int64_t p = p0;
+        const bool active = p < P;
+        const int64_t pc = active ? p : (int64_t)P - 1;
+        const int cnt = (int)((int64_t)P - wave * 64 > 64 ? 64 : ((int64_t)P - wave * 64));
+        const ConstArray<double> lead{a->lead};
+        auto val = [&](double z, int j) -> double {
+            if constexpr (lognormal) return lead[j] * fm_exp2(z, ke);
+            else return z;
+        };
+        // ---- the carried states every ckpt_stride steps, for the adjoint's reverse sweep:
+        // [ti / stride][j][P], stored non-temporal (read back only by the sweep, after this pass)
+        if (a->ckpt && (ti % a->ckpt_stride) == 0) {
+            const int c = ti / a->ckpt_stride, cfirst = ConstArray<int32_t>{a->ckpt_first}[c];
+            double* to = (double*)a->ckpt + (size_t)c * n * P + pc;
+            static_for<0, W * NCH>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                if ((unsigned)(j - cfirst) < (unsigned)(n - cfirst) && active)
+                    __builtin_nontemporal_store(Y.template at<j>(), to);
+                to += P;
+            });
+        }
+        // ---- N(T_{k+1}) = N(T_k).accrue(L_k(T_k), d_k) once L_k is final (LMM:1050-1066)
+        const int num_slots = a->num_slots, stride = num_slots + n + 1;
+        while (kcur < n && ConstArray<int32_t>{a->tenor_time_index}[kcur] <= ti) {
+            const double Lk = val(Y.get(kcur), kcur);
+            const double dk = ConstArray<double>{a->delta}[kcur];
+            double Nn;
+            if (kcur == 0)      Nn = Lk * (dk * 1.0) + 1.0;      // Scalar.accrue of Scalar 1.0
+            else if (kcur == 1) Nn = Lk * (dk * N) + N;          // Scalar.accrue of a stochastic rate
+            else                Nn = N * (1 + Lk * dk);          // RandomVariableFromDoubleArray.accrue
+            Nprev = N; N = Nn; kcur++; knum = kcur;
+            // sum of 1/N(T_k) over paths (numeraire adjustment average)
+            const double s = wave_reduce_sum(active ? (1.0 / N) * 1.0 : 0.0);
+            if (lane == 0 && cnt > 0) a->wave_sum[(size_t)wave * stride + num_slots + kcur] = s;
+            if (a->numeraire && active) a->numeraire[(size_t)kcur * P + p] = N;
+        }
+        // ---- products evaluated at this time index; walk: the swaption group that its step values
+        const ConstArray<KProduct> products{a->products};
+        int walk = -1;
+        eval_products_at<true, true, NCH, double>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
+                                                  ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, cnt, lane,
+                                                  wave, a->wave_sum, a->wave_m2, stride, a->contrib, p, P, walk);
+        const int nT = a->nT;
+        if (ti == nT) break;
+
+        // ---- Euler step ti -> ti+1
+        const ConstArray<double> times{a->times};
+        const double dt = times[ti + 1] - times[ti];
+        const int first = ConstArray<int32_t>{a->first_alive}[ti];
+        // the step's increments, and a touch of the last of the next step's, which brings its line into
+        // the L2 while this step runs
+        const int F = a->F;
+        const double* dwp = (const double*)a->dw + ((size_t)pc * nT + ti) * F;
+        double dW[FCAP];
+        if (F == FCAP) {
+#pragma unroll
+            for (int k = 0; k < FCAP; k++) dW[k] = dwp[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < FCAP; k++) dW[k] = k < F ? dwp[k] : 0.0;
+        }
+        const uint32_t touch = *(const volatile uint32_t*)(dwp + (ti + 1 < nT ? 2 * F - 1 : F - 1));
+        SwaptionWalk sw;
+        sw.table = (RecPtr)(uintptr_t)a->walk;
+        if (walk >= 0) {
+            const KProduct pr = products[walk];
+            sw.table += 8 * pr.walk;
+            sw.j0 = pr.first_j;
+            sw.periods = pr.num_periods;
+        }
+        spot64_step<NCH, FCAP, lognormal, true>(Y, n, a->rec_n, ti, first, dt, dW, (const double*)a->rec, ke, &sw);
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" :: "v"(touch));
+#endif
+        if (walk >= 0) {
+            const KProduct pr = products[walk];
+            const int m = 1 + pr.pad2;
+            const double invN = 1.0 / (pr.num_k == knum ? N : Nprev);
+            double x[4];
+            int slot[4];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const KProduct pg = products[walk + (g < m ? g : 0)];
+                x[g] = jmax0(sw.V[g] * pg.notional) * invN;
+                slot[g] = pg.out_slot;
+            }
+            reduce_slots4(x, m, active, cnt, cnt > 0 ? 1.0 / (double)cnt : 0.0, lane, wave, a->wave_sum, a->wave_m2,
+                          stride, slot);
+        }
+        if (a->paths) {
+            const ConstArray<int32_t> row{a->row_of + (size_t)(ti + 1) * n};
+            double* paths = (double*)a->paths + pc;
+            static_for<0, NCH>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                const int j1 = n < W * q + W ? n : W * q + W;
+#pragma unroll 1
+                for (int j = first > W * q ? first : W * q; j < j1; j++) {
+                    const double v = val(Y.template ch<q>()[j - W * q], j);
+                    if (active) paths[(size_t)row[j] * P] = v;
+                }
+            });
+        }
+    }
+}
+
+template <int NCH, int FCAP>
+void launch_spot64_cap(const StepArgs& a, hipStream_t stream) {
+    const dim3 grid((unsigned)(((int64_t)a.P + kStepThreads - 1) / kStepThreads));
+    if (a.lognormal)
+        hipLaunchKernelGGL((lmm_spot64_kernel<NCH, FCAP, true>), grid, dim3(kStepThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL((lmm_spot64_kernel<NCH, FCAP, false>), grid, dim3(kStepThreads), 0, stream, a);
+    HIP_CHECK(hipGetLastError());
+}
+
+template <int NCH>
+void launch_spot64_n(const StepArgs& a, hipStream_t stream) {
+    if (a.F <= 1) launch_spot64_cap<NCH, 1>(a, stream);
+    else if (a.F <= 3) launch_spot64_cap<NCH, 3>(a, stream);
+    else if (a.F <= 5) launch_spot64_cap<NCH, 5>(a, stream);
+    else if (a.F <= 10) launch_spot64_cap<NCH, 10>(a, stream);
+    else throw FmError(FM_ERR_UNSUPPORTED, "number of factors above 10 is not supported by the path kernel");
+}
+
+} // namespace fm

@@ -25,7 +25,7 @@
 // weights of the induction's own adjoint (lmm_bermudan.hip) when given.
 #pragma once
 
-#include "lmm_spot.hpp"
+#include "lmm_spot64.hpp"
 #include "lmm_adjoint.hpp"
 
 namespace fm {
@@ -53,9 +53,15 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
     const int cnt = (int)((int64_t)P - wave * 64 > 64 ? 64 : ((int64_t)P - wave * 64));
     const int gstride = nT * n + n;
     const bool capped = a.capped != 0;
-    const real ycap = LOGCARRY ? (real)a.logcap : (real)a.cap;
+    const real ycap = (real)a.cap;
     const int stride = g.stride;
-    auto val = [&](real x) -> real { return LOGCARRY ? dev_exp<real>(x) : x; };
+    const Exp2Coef ke;
+    auto val = [&](real x, int j) -> real {
+        if constexpr (LOGCARRY) return a.lead[j] * fm_exp2(x, ke);
+        else return x;
+    };
+    constexpr bool D = sizeof(real) == 8;     // states and records of lmm_spot64.hpp
+    const int rec_n = D ? a.rec_n : n;
 
     ChunkedForwards<NCH, real> X;     // state at t
     ChunkedForwards<NCH, real> Lb;    // adjoint of the forwards L_j(t)
@@ -92,9 +98,13 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                 for (int s = c; s < t; s++) {
                     real dWs[FCAP];
                     load_increments<FCAP, real>(dWs, dw, pc, nT, s, F);
-                    spot_step<NCH, FCAP, real, lognormal>(X, n, s, first_alive[s], (real)(times[s + 1] - times[s]),
-                                                          dWs, rec, capped, ycap, (real*)nullptr,
-                                                          (const int32_t*)nullptr, p, P, active);
+                    const real dts = (real)(times[s + 1] - times[s]);
+                    if constexpr (D)
+                        spot64_step<NCH, FCAP, lognormal, false>(X, n, rec_n, s, first_alive[s], dts, dWs, rec, ke,
+                                                                 nullptr);
+                    else
+                        spot_step<NCH, FCAP, real, lognormal>(X, n, s, first_alive[s], dts, dWs, rec, capped, ycap,
+                                                              (real*)nullptr, (const int32_t*)nullptr, p, P, active);
                     if (s + 1 < hi && active) {
                         const size_t srow = (size_t)(s - c) * n;
                         static_for<0, W * NCH>([&](auto J) {
@@ -123,7 +133,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                     const int j1 = n < W * q + W ? n : W * q + W;
 #pragma unroll 1
                     for (int j = j0; j < j1; j++) {
-                        const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, n, t, j);
+                        const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, rec_n, t, j);
                         const real mb = Lb.template ch<q>()[j - W * q] * dt;
 #pragma unroll
                         for (int k = 0; k < FCAP; k++) Sb[k] = Sb[k] + mb * R.lam(k);
@@ -140,10 +150,22 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                     const int j1 = n < W * q + W ? n : W * q + W;
 #pragma unroll 1
                     for (int j = j0; j < j1; j++) {
-                        const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, n, t, j);
-                        const real Lj = val(X.template ch<q>()[j - W * q]);
-                        const real r = spot_div<real>((real)1.0, Lj * R.c1() + R.c2());
-                        const real w = lognormal ? r * Lj : r;
+                        const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, rec_n, t, j);
+                        const real xj = X.template ch<q>()[j - W * q];
+                        real Lj, w, dwdL;
+                        if constexpr (D) {
+                            // E_j = L_j / s_j; w = E/(E + e) (log-normal) and dw/dL = e/(E + e)^2 / s
+                            const double E = lognormal ? fm_exp2(xj, ke) : xj;
+                            const double r = fm_rcp_nr(E + R.c2());
+                            w = lognormal ? E * r : r;
+                            Lj = lognormal ? a.lead[j] * E : E;
+                            dwdL = lognormal ? R.c2() * r * r * a.lead[n + j] : -r * r;
+                        } else {
+                            Lj = xj;
+                            const real r = spot_div<real>((real)1.0, Lj * R.c1() + R.c2());
+                            w = lognormal ? r * Lj : r;
+                            dwdL = lognormal ? R.c2() * r * r : -R.c1() * r * r;
+                        }
                         const real Yb = Lb.template ch<q>()[j - W * q];     // adjoint of y_j(t+1)
                         const real mb = Yb * dt;
                         real wb = (real)0;
@@ -164,7 +186,6 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                         // variance sigma^2 c in the drift: d(-var/2)/dsigma = -sigma c
                         if (lognormal) sgb = sgb + mb * vterm[(size_t)t * n + j];
                         // y_j(t+1) = log L_j(t) + ... (or L_j(t) + ...), and w_j depends on L_j(t)
-                        const real dwdL = lognormal ? R.c2() * r * r : -R.c1() * r * r;
                         const real direct = lognormal ? Yb * adj_rcp<real>(Lj) : Yb;
                         Lb.template ch<q>()[j - W * q] = direct + wb * dwdL;
                         const real gs = active ? sgb : (real)0;
@@ -213,7 +234,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
 #pragma unroll 1
                         for (int j = jb - 1; j >= ja; j--) {
                             const KPeriod pe = periods[pr.param_off + (j - j0)];
-                            const real Lj = val(X.template ch<q>()[j - W * q]);
+                            const real Lj = val(X.template ch<q>()[j - W * q], j);
                             const real D = (real)pe.adj * adj_rcp<real>((real)1.0 + Lj * (real)pe.tau);
                             V = (V + ((Lj - (real)pe.strike) * (real)pe.period_length) * (real)pr.notional) * D;
                             Pc = Pc * D;
@@ -231,7 +252,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
 #pragma unroll 1
                         for (int j = jb - 1; j >= ja; j--) {
                             const KPeriod pe = periods[pr.param_off + (j - j0)];
-                            const real Lj = val(X.template ch<q>()[j - W * q]);
+                            const real Lj = val(X.template ch<q>()[j - W * q], j);
                             const real one = (real)1.0 + Lj * (real)pe.tau;
                             const real inv = adj_rcp<real>(one);
                             const real pj = ((Lj - (real)pe.strike) * (real)pe.period_length) * (real)pr.notional;
@@ -243,7 +264,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                     });
                 } else if (pr.type == FM_PRODUCT_CAPLET) {
                     const KPeriod pe = periods[pr.param_off];
-                    const real Lj = val(X.get(pr.first_j));
+                    const real Lj = val(X.get(pr.first_j), pr.first_j);
                     const real v = Lj - (real)pe.strike;
                     // floor(0.0) has derivative 1 for v >= 0, cap(0.0) has derivative 1 for v < 0
                     // (RandomVariableDifferentiableAAD.java:333-348)
@@ -269,7 +290,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                         }
                     }
                     const KPeriod pe = periods[pr.param_off];
-                    const real Lj = val(X.get(pr.first_j));
+                    const real Lj = val(X.get(pr.first_j), pr.first_j);
                     const double sgn = (pr.flags & 1) ? 1.0 : -1.0;
                     const double pay = sgn * (double)(((Lj - (real)pe.strike) * (real)pe.period_length) * (real)pe.notional);
                     xadd = (real)(pw * sgn * pe.period_length * pe.notional * wq / Nsel);
@@ -284,7 +305,7 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
             while (K > Kprev) {
                 const int k = K - 1;
                 const double Nk = (k == 0) ? 1.0 : numeraire[(size_t)k * P + pc];
-                const double Lk = (double)val(X.get(k));
+                const double Lk = (double)val(X.get(k), k);
                 const double dk = delta[k];
                 Lb.add(k, (real)(Nb_top * dk * Nk));
                 Nb_low += Nb_top * (1.0 + Lk * dk);
@@ -308,8 +329,10 @@ lmm_spot_adjoint_kernel(const StepArgs a, const AdjArgs g, const real* __restric
                     for (int j = j0; j < j1; j++) {
                         const real x = X.template ch<q>()[j - W * q];
                         const real lb = Lb.template ch<q>()[j - W * q];
-                        const real yb = lognormal ? lb * val(x) : lb;
-                        Lb.template ch<q>()[j - W * q] = (capped && x >= ycap) ? (real)0 : yb;
+                        const real yb = lognormal ? lb * val(x, j) : lb;
+                        real xcap = ycap;
+                        if constexpr (D) xcap = rec_at<FCAP, real>(rec, rec_n, t - 1, j).c1();
+                        Lb.template ch<q>()[j - W * q] = (capped && x >= xcap) ? (real)0 : yb;
                     }
                 });
             }

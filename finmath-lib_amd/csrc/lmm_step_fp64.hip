@@ -1,14 +1,20 @@
-// FP64 instantiations of the spot Euler path kernel and its reverse sweep. Compiled with
-// -ffp-contract=off: every product and sum is rounded separately, as the JVM evaluates the
-// reference.
-#include "lmm_spot.hpp"
-#include "lmm_spot_adjoint.hpp"
+// FP64 instantiations of the spot Euler path kernel up to 24 forwards, and the choice by size:
+// capacities of 8, 24, 40 and 80 forwards in chunks of eight. Compiled with -ffp-contract=off: the
+// multiply-adds are written where they are meant. The larger capacities are translation units of
+// their own, which compile side by side.
+#include "lmm_spot64.hpp"
 
 namespace fm {
-// Pricing, simulation and the adjoint's forward pass (with checkpoints) run the spot kernel;
-// the reverse sweep recomputes its steps from the checkpointed states.
+void launch_spot64_40(const StepArgs& a, hipStream_t stream);
+void launch_spot64_80(const StepArgs& a, hipStream_t stream);
+
+// Pricing, simulation and the adjoint's forward pass (with checkpoints); a.Y0 holds the initial states.
 void launch_lmm_step_fp64(const StepArgs& a, void* stream) {
-    launch_spot<double>(a, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    if (a.n <= 8) launch_spot64_n<1>(a, s);
+    else if (a.n <= 24) launch_spot64_n<3>(a, s);
+    else if (a.n <= 40) launch_spot64_40(a, s);
+    else if (a.n <= 80) launch_spot64_80(a, s);
+    else throw FmError(FM_ERR_UNSUPPORTED, "more than 80 forward rates are not supported by the path kernel");
 }
-void launch_lmm_adjoint_fp64(const StepArgs& a, const AdjArgs& g, void* stream) { launch_spot_adjoint<double>(a, g, (hipStream_t)stream); }
 }

@@ -1,0 +1,6 @@
+// FP64 instantiations of the spot Euler path kernel for up to 40 forwards.
+#include "lmm_spot64.hpp"
+
+namespace fm {
+void launch_spot64_40(const StepArgs& a, hipStream_t stream) { launch_spot64_n<5>(a, stream); }
+}
