@@ -35,11 +35,16 @@ NO_CONTRACT = ["-ffp-contract=off"]
 SOURCES = {
     "mt19937_gf2.cpp": NO_CONTRACT,
     "mt19937.hip": NO_CONTRACT,
+    "lmm_adjoint_fp64_80.hip": NO_CONTRACT,
+    "lmm_adjoint_fp64_40.hip": NO_CONTRACT,
+    "lmm_adjoint_fp32_80.hip": [],
+    "lmm_adjoint_fp32_48.hip": [],
     "lmm_adjoint_fp64.hip": NO_CONTRACT,
     "lmm_step_fp64_80.hip": NO_CONTRACT,
     "lmm_step_fp64_40.hip": NO_CONTRACT,
     "lmm_step_fp64.hip": NO_CONTRACT,
     "lmm_adjoint_fp32.hip": [],
+    "lmm_step_fp32_80.hip": [],
     "lmm_step_fp32.hip": [],
     "lmm_step_general_fp64.hip": NO_CONTRACT,
     "lmm_step_pc_fp64.hip": NO_CONTRACT,

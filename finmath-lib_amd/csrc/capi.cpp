@@ -176,8 +176,9 @@ struct fm_lmm {
     }
     // the FP64 spot kernel (lmm_spot64.hpp): base-2 log-forwards, its own record layout
     bool spot64() const { return !fp32() && (plain_euler() || logstate()); }
-    // records per time step: the FP64 spot kernel reads them in pairs
-    int rec_n() const { return spot64() ? n() + (n() & 1) : n(); }
+    bool spot32() const { return fp32() && plain_euler(); }
+    // records per time step: the spot kernels read them in pairs
+    int rec_n() const { return spot64() || spot32() ? n() + (n() & 1) : n(); }
     size_t real_size() const { return fp32() ? sizeof(float) : sizeof(double); }
     int process_time_index(double t) const { return jsearch(times, round_tick(t)); }
     int libor_index(double t) const { return jsearch(tenor, round_tick(t)); }
@@ -281,10 +282,10 @@ void prepare_model(fm_lmm* c) {
     // variance*(-0.5) (0 in the normal state space), d/d and 1/d
     const int fcap = fcap_of(F), rs = rec_size_of(fcap);
     // the FP64 spot kernel's records (lmm_spot64.hpp) scale each forward by its initial value (where
-    // that is an ordinary positive number) and hold no loadings for the forwards fixed at t_i
-    const bool spot64 = c->spot64();
+    // that is an ordinary positive number); the spot kernels' hold no loadings for the forwards fixed
+    // at t_i, and the FP64 one touches the records of the pair after the last one
+    const bool spot64 = c->spot64(), spot = spot64 || c->spot32();
     const int rec_n = c->rec_n();
-    // (the spot kernel touches the records of the pair after the last one)
     std::vector<double> rec(((size_t)nT * rec_n + 4) * rs, 0.0), lead((size_t)2 * n, 1.0), z0((size_t)n, 0.0);
     std::vector<double> zcap((size_t)n, c->cfg.libor_cap);
     for (int j = 0; j < n; j++) {
@@ -299,8 +300,8 @@ void prepare_model(fm_lmm* c) {
     for (int i = 0; i < nT; i++)
         for (int j = 0; j < rec_n; j++) {
             double* r = rec.data() + ((size_t)i * rec_n + j) * rs;
-            if (j == n) { r[fcap + 1] = HUGE_VAL; r[fcap + 2] = 1.0; continue; }     // absent forward of the last pair
-            const bool fixed = spot64 && j < c->first_alive[(size_t)i];
+            if (j == n) { r[fcap + 1] = spot64 ? HUGE_VAL : 1.0; r[fcap + 2] = 1.0; continue; }     // absent forward of the last pair
+            const bool fixed = spot && j < c->first_alive[(size_t)i];
             if (!fixed) {
                 for (int k = 0; k < F; k++) r[k] = c->lam[((size_t)i * n + j) * F + k];
                 r[fcap] = lognormal ? c->var[(size_t)i * n + j] * (-0.5) : 0.0;
@@ -350,7 +351,7 @@ void prepare_model(fm_lmm* c) {
     if (!std::isinf(c->cfg.libor_cap))
         for (double& y : y0c) y = std::min(y, std::log(c->cfg.libor_cap));
     upload(c->d_Y0cap, y0c, s);
-    if (!lognormal) z0 = c->init_value;
+    if (!spot64 || !lognormal) z0 = c->init_value;       // states that are the forwards themselves
     z0.resize(80, 0.0);         // the register array's capacity
     upload(c->d_z0, z0, s);
     upload(c->d_lead, lead, s);
@@ -427,6 +428,7 @@ struct Lowered {
     std::vector<int32_t> swap_col0, swap_ncol, swap_slot;
     std::vector<int> contrib_k;               // contribution column -> numeraire tenor index
     std::vector<double> walk;                 // walk tables of swaption groups, rows of eight (FP64 spot kernel)
+    std::vector<float> walk32;                // the FP32 spot kernel's
 };
 
 // kcur of the kernel after the numeraire advance at time index ti
@@ -468,7 +470,7 @@ static bool same_swaption_periods(const KProduct& a, const KProduct& b, const st
 
 static void group_swaptions(Lowered& L) {
     std::vector<KProduct>& kp = L.kp;
-    for (size_t i = 0; i < kp.size(); i++) kp[i].pad2 = 0;
+    for (KProduct& k : kp) k.pad2 = k.pad3 = 0;
     for (size_t i = 0; i < kp.size();) {
         size_t e = i + 1;
         if (kp[i].type == FM_PRODUCT_SWAPTION) {
@@ -479,6 +481,7 @@ static void group_swaptions(Lowered& L) {
                 e++;
             }
             kp[i].pad2 = (int32_t)(e - i - 1);
+            for (size_t f = i; f < e; f++) kp[f].pad3 = (int32_t)(f - i);
             if (e - i > 1) {
                 const int np = kp[i].num_periods;
                 const int base = (int)L.per.size();
@@ -496,12 +499,28 @@ static void group_swaptions(Lowered& L) {
     }
 }
 
-// Walk tables of the FP64 spot kernel (SwaptionWalk, lmm_spot64.hpp): at each time index the first
+// Walk tables of the spot kernels. FP64 (SwaptionWalk, lmm_spot64.hpp): at each time index the first
 // group whose periods are discounted over their tenor periods is valued by that index's Euler step.
 // A second group, and one exercised at the last time index (which has no step), keep a walk of
 // their own. The period lengths are tick-rounded dates' differences, hence the tolerance.
 static void make_walks(const fm_lmm* c, Lowered& L) {
     for (KProduct& k : L.kp) k.walk = -1;
+    if (c->spot32()) {
+        // FP32: every group, rows {tau, period length, adjustment, -, strikes} (swaption_walk32)
+        for (size_t i = 0; i < L.kp.size(); i += 1 + (size_t)(L.kp[i].type == FM_PRODUCT_SWAPTION ? L.kp[i].pad2 : 0)) {
+            KProduct& k = L.kp[i];
+            if (k.type != FM_PRODUCT_SWAPTION) continue;
+            k.walk = (int32_t)(L.walk32.size() / 8);
+            for (int q = 0; q < k.num_periods; q++) {
+                const KPeriod& pe = L.per[(size_t)(k.param_off + q)];
+                float row[8] = {(float)pe.tau, (float)pe.period_length, (float)pe.adj, 0, 0, 0, 0, 0};
+                for (int g = 0; g <= k.pad2; g++)
+                    row[4 + g] = (float)L.per[(size_t)(L.kp[i + (size_t)g].param_off + q)].strike;
+                L.walk32.insert(L.walk32.end(), row, row + 8);
+            }
+        }
+        return;
+    }
     if (!c->spot64()) return;
     int last = -1;          // time index of the last group that got a walk
     for (size_t i = 0; i < L.kp.size(); i += 1 + (size_t)(L.kp[i].type == FM_PRODUCT_SWAPTION ? L.kp[i].pad2 : 0)) {
@@ -940,7 +959,7 @@ size_t external_scratch_bytes(const fm_lmm* c, const Lowered& L) {
     const size_t num_waves = ((size_t)c->P() + 63) / 64, stride = (size_t)L.num_slots + c->n() + 1;
     return 2 * ExternalScratch::piece(num_waves * stride * sizeof(double)) +
            ExternalScratch::piece(L.kp.size() * sizeof(KProduct)) + ExternalScratch::piece(L.per.size() * sizeof(KPeriod)) +
-           ExternalScratch::piece(L.walk.size() * sizeof(double)) +
+           ExternalScratch::piece(L.walk.size() * sizeof(double)) + ExternalScratch::piece(L.walk32.size() * sizeof(float)) +
            ExternalScratch::piece(stride * 2 * sizeof(double));
 }
 
@@ -1015,6 +1034,7 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     if (c->spot64()) {
         a.Y0 = c->d_z0.as<double>();
         a.lead = c->d_lead.as<double>();
+    a.walk = c->d_walk.p;           // uploaded by the pricing pass
         a.walk = xs ? xs->upload(L.walk, s) : upload(c->d_walk, L.walk, s);
         launch_lmm_step_fp64(a, s);
     } else if (c->has_lv || c->has_sv) {
@@ -1024,7 +1044,8 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
         if (c->fp32()) launch_lmm_step_lv_fp32(a, s);
         else launch_lmm_step_lv_fp64(a, s);
     } else if (c->plain_euler()) {
-        a.Y0 = c->d_L0.as<double>();            // the capped initial forwards
+        a.Y0 = c->d_z0.as<double>();            // the capped initial forwards
+        a.walk = xs ? xs->upload(L.walk32, s) : upload(c->d_walk, L.walk32, s);
         launch_lmm_step_fp32(a, s);
     } else {
         // the general kernel: FP64 log-normal functional schemes carry the log-forwards, capped
@@ -1630,8 +1651,6 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
             k.weight = wq[(size_t)q] * sc / (double)P;
         }
     }
-    std::vector<double> kweights(kp.size());
-    for (size_t i = 0; i < kp.size(); i++) kweights[i] = kp[i].weight;
     std::vector<int32_t> kcur((size_t)nT + 1);
     for (int t = 0; t <= nT; t++) kcur[(size_t)t] = kcur_at(c, t);
     StepArgs a{};
@@ -1646,6 +1665,7 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
     a.L0 = c->d_L0.as<double>(); a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
     a.rec_n = c->rec_n();
     a.lead = c->d_lead.as<double>();
+    a.walk = c->d_walk.p;           // uploaded by the pricing pass
     a.num_products = (int)kp.size();
     a.products = upload(c->d_products, kp, s);
     a.periods = upload(c->d_periods, L.per, s);
@@ -1653,7 +1673,6 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
     AdjArgs ga{};
     ga.stride = stride;
     ga.kcur_at = upload(c->d_kcur, kcur, s);
-    ga.weight = upload(c->d_scale, kweights, s);
     ga.berm_ex = L.berm.empty() ? nullptr : c->d_berm_ex.as<int32_t>();
     ga.berm_weight = nullptr;
     if (berm_adjoint) {
@@ -1664,13 +1683,15 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
         ga.berm_weight = w;
     }
     ga.seg = c->d_seg.get((size_t)std::max(stride - 2, 1) * n * P * c->real_size());
-    // factor matrix padded to the factor capacity and -sigma_j(t_i) c_j, in the path precision
-    std::vector<double> fpad((size_t)n * fcap_of(c->F()), 0.0), vterm((size_t)nT * n, 0.0);
+    // factor matrix in rows of a record's size and -sigma_j(t_i) c_j in rows of rec_n, in the path
+    // precision (the sweep reads whole rows and one group of four ahead)
+    const int rs = rec_size_of(fcap_of(c->F())), rec_n = c->rec_n();
+    std::vector<double> fpad((size_t)(rec_n + 4) * rs, 0.0), vterm((size_t)nT * rec_n + 4, 0.0);
     for (int j = 0; j < n; j++)
-        for (int k = 0; k < c->F(); k++) fpad[(size_t)j * fcap_of(c->F()) + k] = c->vf_fac[(size_t)j * c->F() + k];
+        for (int k = 0; k < c->F(); k++) fpad[(size_t)j * rs + k] = c->vf_fac[(size_t)j * c->F() + k];
     if (c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL)
         for (int i = 0; i < nT; i++)
-            for (int j = 0; j < n; j++) vterm[(size_t)i * n + j] = -c->vf_sig[(size_t)i * n + j] * c->vf_c[(size_t)j];
+            for (int j = 0; j < n; j++) vterm[(size_t)i * rec_n + j] = -c->vf_sig[(size_t)i * n + j] * c->vf_c[(size_t)j];
     // host sources stay alive until the stream synchronisation at the end of this call
     const std::vector<float> fpad_f(fpad.begin(), fpad.end()), vterm_f(vterm.begin(), vterm.end());
     if (c->fp32()) {

@@ -78,8 +78,8 @@ struct KProduct {
     int32_t param_off;    // offset into the per-period parameter table
     int32_t pad2;         // swaption: number of following swaptions valued with it (pricing);
                           // adjoint Bermudan period: the Bermudan's index
-    int32_t walk;         // FP64 spot kernel: first row of the group's walk table (lmm_spot64.hpp), or -1
-    int32_t pad3;
+    int32_t walk;         // spot kernels: first row of the group's walk table (lmm_spot64.hpp, lmm_spot32.hpp), or -1
+    int32_t pad3;         // swaption: its index within its group
 };
 
 // Swaptions valued together by one walk over their shared periods (KProduct.pad2 of the first
@@ -102,12 +102,12 @@ struct StepArgs {
     const int32_t* first_alive;  // device nT
     const int32_t* tenor_time_index; // device n+1: process time index of T_k (rounded up)
     const void* rec;             // device [nT][n][rec_size_of(fcap_of(F))] records (double or float)
-    int rec_n;                   // records per time step (n, or n rounded up to even for the FP64 spot kernel)
+    int rec_n;                   // records per time step (n, or n rounded up to even for the spot kernels)
     int lognormal, capped;       // state space is LOGNORMAL; the liborCap applies
     const double* delta;         // device n: T_{j+1}-T_j
     const double* L0;            // device n: initial forwards in value space
     const double* lead;          // FP64 spot kernel, device [2][n]: the forwards' scales s_j and 1/s_j
-    const double* walk;          // FP64 spot kernel, device [rows][8]: walk tables of swaption groups
+    const void* walk;            // spot kernels, device [rows][8]: walk tables of swaption groups (path precision)
     const double* Y0;            // device n: initial states (log(max(L0, 0)) or L0) of the carried schemes;
                                  // for the log-forward and spot kernels kept below log(cap)
                                  // (the spot kernel in the normal state space: the capped forwards)
@@ -158,13 +158,12 @@ void launch_stochastic_volatility(const double* dw, int nT, int Fd, int fa, int 
 void launch_heston_volatility(const double* dw, int nT, int Fd, int fa, int P, const double* times, double kappa,
                               double theta, double xi, void* out, int out_fp32, void* stream);
 
-// Reverse sweep (lmm_adjoint.hpp): adjoint arguments and launchers.
+// Reverse sweep (lmm_spot_adjoint.hpp): adjoint arguments and launchers.
 struct AdjArgs {
     int stride;                      // checkpoint stride
     const int32_t* kcur_at;          // [nT+1] numeraire index after the advance at each time index
-    const double* weight;            // [num kernel products] objective weight of each lowered product
-    const void* fsig;                // [n][fcap_of(F)] factor matrix f_jk, zero padded (path precision)
-    const void* vterm;               // [nT][n] -sigma_j(t_i) c_j, d(variance * -1/2)/dsigma (path precision)
+    const void* fsig;                // [rec_n + 4][rec_size_of(fcap_of(F))] factor matrix f_jk, zero padded (path precision)
+    const void* vterm;               // [nT][rec_n] -sigma_j(t_i) c_j, d(variance * -1/2)/dsigma (path precision)
     void* seg;                       // [max(stride-2,1)][n][P] states inside a checkpoint segment (path precision)
     double* wave_grad;               // [num_waves][nT*n + n] partials of dV/dsigma and dV/dL(0)
     const int32_t* berm_ex;          // [num Bermudans][P] exercise period per path (-1: never), or NULL

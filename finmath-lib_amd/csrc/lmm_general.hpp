@@ -14,7 +14,7 @@
 // has no dynamically indexed private array and no scratch.
 #pragma once
 
-#include "lmm_spot.hpp"
+#include "lmm_chunks.hpp"
 
 namespace fm {
 
@@ -263,9 +263,9 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
         // terminal and predictor-corrector kernels (measured 4-5% faster there; slower in FP32
         // and in the spot Euler kernel)
         constexpr bool group = sizeof(real) == 8 && (TERMINAL || PC);
-        int walk = -1;
-        eval_products_at<group, false, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
-                                                  active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P, walk);
+        eval_products_at<group, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
+                                                  active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P,
+                                           [](int, const KProduct&) { return false; });
 
         if (ti == nT) break;
 

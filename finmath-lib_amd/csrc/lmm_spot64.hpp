@@ -36,7 +36,7 @@
 // scalar registers for them instead spilled.
 #pragma once
 
-#include "lmm_spot.hpp"
+#include "lmm_chunks.hpp"
 
 namespace fm {
 
@@ -151,159 +151,6 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
 #endif
         }
     });
-}
-
-// The spot kernel in FP64: one thread per path, its states in NCH chunks of eight doubles. Per time
-// index: checkpoints (the adjoint's forward pass), numeraire updates, the products evaluated there,
-// the Euler step with its swaption walk, and the new forwards when the process is stored.
-template <int NCH, int FCAP, bool lognormal>
-__global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(NCH <= 5 && FCAP <= 5 ? 4 : 1)))
-lmm_spot64_kernel(const StepArgs) {
-    constexpr int W = chunk_width<double>();
-    ArgPtr a = kernel_arguments();
-    const uint32_t p0 = blockIdx.x * (uint32_t)kStepThreads + threadIdx.x;      // P < 2^31
-    const int lane = threadIdx.x & 63;
-    // the wavefront index, uniform: kept in a scalar register
-    const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Exp2Coef ke;
-
-    ChunkedForwards<NCH, double> Y;
-    {
-        const ConstArray<double> z0{a->Y0};
-        static_for<0, W * NCH>([&](auto J) {
-            constexpr int j = decltype(J)::value;
-            Y.template put<j>(z0[j]);           // zeros beyond the n forwards
-            if constexpr (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);    // a chunk's scalar loads at a time
-        });
-    }
-    double N = 1.0, Nprev = 1.0;   // unadjusted numeraire N(T_knum) and the one before it
-    int kcur = 0, knum = 0;
-    int qp = 0;
-    for (int ti = 0;; ti++) {
-        a = kernel_arguments();
-        const int P = a->P, n = a->n;
-        const int64_t p = p0;
-        const bool active = p < P;
-        const int64_t pc = active ? p : (int64_t)P - 1;
-        const int cnt = (int)((int64_t)P - wave * 64 > 64 ? 64 : ((int64_t)P - wave * 64));
-        const ConstArray<double> lead{a->lead};
-        auto val = [&](double z, int j) -> double {
-            if constexpr (lognormal) return lead[j] * fm_exp2(z, ke);
-            else return z;
-        };
-        // ---- the carried states every ckpt_stride steps, for the adjoint's reverse sweep:
-        // [ti / stride][j][P], stored non-temporal (read back only by the sweep, after this pass)
-        if (a->ckpt && (ti % a->ckpt_stride) == 0) {
-            const int c = ti / a->ckpt_stride, cfirst = ConstArray<int32_t>{a->ckpt_first}[c];
-            double* to = (double*)a->ckpt + (size_t)c * n * P + pc;
-            static_for<0, W * NCH>([&](auto J) {
-                constexpr int j = decltype(J)::value;
-                if ((unsigned)(j - cfirst) < (unsigned)(n - cfirst) && active)
-                    __builtin_nontemporal_store(Y.template at<j>(), to);
-                to += P;
-            });
-        }
-        // ---- N(T_{k+1}) = N(T_k).accrue(L_k(T_k), d_k) once L_k is final (LMM:1050-1066)
-        const int num_slots = a->num_slots, stride = num_slots + n + 1;
-        while (kcur < n && ConstArray<int32_t>{a->tenor_time_index}[kcur] <= ti) {
-            const double Lk = val(Y.get(kcur), kcur);
-            const double dk = ConstArray<double>{a->delta}[kcur];
-            double Nn;
-            if (kcur == 0)      Nn = Lk * (dk * 1.0) + 1.0;      // Scalar.accrue of Scalar 1.0
-            else if (kcur == 1) Nn = Lk * (dk * N) + N;          // Scalar.accrue of a stochastic rate
-            else                Nn = N * (1 + Lk * dk);          // RandomVariableFromDoubleArray.accrue
-            Nprev = N; N = Nn; kcur++; knum = kcur;
-            // sum of 1/N(T_k) over paths (numeraire adjustment average)
-            const double s = wave_reduce_sum(active ? (1.0 / N) * 1.0 : 0.0);
-            if (lane == 0 && cnt > 0) a->wave_sum[(size_t)wave * stride + num_slots + kcur] = s;
-            if (a->numeraire && active) a->numeraire[(size_t)kcur * P + p] = N;
-        }
-        // ---- products evaluated at this time index; walk: the swaption group that its step values
-        const ConstArray<KProduct> products{a->products};
-        int walk = -1;
-        eval_products_at<true, true, NCH, double>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
-                                                  ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, cnt, lane,
-                                                  wave, a->wave_sum, a->wave_m2, stride, a->contrib, p, P, walk);
-        const int nT = a->nT;
-        if (ti == nT) break;
-
-        // ---- Euler step ti -> ti+1
-        const ConstArray<double> times{a->times};
-        const double dt = times[ti + 1] - times[ti];
-        const int first = ConstArray<int32_t>{a->first_alive}[ti];
-        // the step's increments, and a touch of the last of the next step's, which brings its line into
-        // the L2 while this step runs
-        const int F = a->F;
-        const double* dwp = (const double*)a->dw + ((size_t)pc * nT + ti) * F;
-        double dW[FCAP];
-        if (F == FCAP) {
-#pragma unroll
-            for (int k = 0; k < FCAP; k++) dW[k] = dwp[k];
-        } else {
-#pragma unroll
-            for (int k = 0; k < FCAP; k++) dW[k] = k < F ? dwp[k] : 0.0;
-        }
-        const uint32_t touch = *(const volatile uint32_t*)(dwp + (ti + 1 < nT ? 2 * F - 1 : F - 1));
-        SwaptionWalk sw;
-        sw.table = (RecPtr)(uintptr_t)a->walk;
-        if (walk >= 0) {
-            const KProduct pr = products[walk];
-            sw.table += 8 * pr.walk;
-            sw.j0 = pr.first_j;
-            sw.periods = pr.num_periods;
-        }
-        spot64_step<NCH, FCAP, lognormal, true>(Y, n, a->rec_n, ti, first, dt, dW, (const double*)a->rec, ke, &sw);
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("" :: "v"(touch));
-#endif
-        if (walk >= 0) {
-            const KProduct pr = products[walk];
-            const int m = 1 + pr.pad2;
-            const double invN = 1.0 / (pr.num_k == knum ? N : Nprev);
-            double x[4];
-            int slot[4];
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const KProduct pg = products[walk + (g < m ? g : 0)];
-                x[g] = jmax0(sw.V[g] * pg.notional) * invN;
-                slot[g] = pg.out_slot;
-            }
-            reduce_slots4(x, m, active, cnt, cnt > 0 ? 1.0 / (double)cnt : 0.0, lane, wave, a->wave_sum, a->wave_m2,
-                          stride, slot);
-        }
-        if (a->paths) {
-            const ConstArray<int32_t> row{a->row_of + (size_t)(ti + 1) * n};
-            double* paths = (double*)a->paths + pc;
-            static_for<0, NCH>([&](auto Q) {
-                constexpr int q = decltype(Q)::value;
-                const int j1 = n < W * q + W ? n : W * q + W;
-#pragma unroll 1
-                for (int j = first > W * q ? first : W * q; j < j1; j++) {
-                    const double v = val(Y.template ch<q>()[j - W * q], j);
-                    if (active) paths[(size_t)row[j] * P] = v;
-                }
-            });
-        }
-    }
-}
-
-template <int NCH, int FCAP>
-void launch_spot64_cap(const StepArgs& a, hipStream_t stream) {
-    const dim3 grid((unsigned)(((int64_t)a.P + kStepThreads - 1) / kStepThreads));
-    if (a.lognormal)
-        hipLaunchKernelGGL((lmm_spot64_kernel<NCH, FCAP, true>), grid, dim3(kStepThreads), 0, stream, a);
-    else
-        hipLaunchKernelGGL((lmm_spot64_kernel<NCH, FCAP, false>), grid, dim3(kStepThreads), 0, stream, a);
-    HIP_CHECK(hipGetLastError());
-}
-
-template <int NCH>
-void launch_spot64_n(const StepArgs& a, hipStream_t stream) {
-    if (a.F <= 1) launch_spot64_cap<NCH, 1>(a, stream);
-    else if (a.F <= 3) launch_spot64_cap<NCH, 3>(a, stream);
-    else if (a.F <= 5) launch_spot64_cap<NCH, 5>(a, stream);
-    else if (a.F <= 10) launch_spot64_cap<NCH, 10>(a, stream);
-    else throw FmError(FM_ERR_UNSUPPORTED, "number of factors above 10 is not supported by the path kernel");
 }
 
 } // namespace fm

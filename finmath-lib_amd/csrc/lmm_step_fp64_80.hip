@@ -1,6 +1,6 @@
 // FP64 instantiations of the spot Euler path kernel for up to 80 forwards.
-#include "lmm_spot64.hpp"
+#include "lmm_spot.hpp"
 
 namespace fm {
-void launch_spot64_80(const StepArgs& a, hipStream_t stream) { launch_spot64_n<10>(a, stream); }
+void launch_spot64_80(const StepArgs& a, hipStream_t stream) { launch_spot_n<10, double>(a, stream); }
 }
