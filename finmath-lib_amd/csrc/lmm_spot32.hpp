@@ -93,6 +93,7 @@ __device__ __forceinline__ void spot32_step(Chunks& Y, int n, int rec_n, int i, 
         for (int k = 0; k < FCAP; k++) y = fmaf(dW[k], R.lam(c, k), y);
         return lognormal ? dev_exp<float>(y) : y;
     };
+    n = opaque(n);
     const unsigned alive = (unsigned)(n - first + 1);
     // a pair's records are read while the pair before it runs: two sets of scalar registers, even pairs
     // in A and odd pairs in B (the pair after the last reads the table's padding)

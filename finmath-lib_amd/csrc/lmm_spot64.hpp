@@ -113,6 +113,7 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
         return inc;
     };
     if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
+    n = opaque(n);
     const unsigned alive = (unsigned)(n - first + 1);
     static_for<0, 4 * NCH>([&](auto Q) {
         constexpr int j = 2 * decltype(Q)::value;

@@ -25,7 +25,7 @@
 //
 // The two register arrays leave two wavefronts per SIMD at 80 FP32 or 40 FP64 forwards, so the sweep
 // waits on scalar loads and on the vector pipeline in turn. 80 forwards x 10 factors x 1,000,000 FP32
-// paths: 22.2 ms at 0.61 vector ALU busy (29.3 ms and 0.49 with rolled loops and every kernel argument
+// paths: 20.7 ms (22.2 ms at 0.61 vector ALU busy while the bounds of the unrolled loops were hoisted as masks and spilled;  29.3 ms and 0.49 with rolled loops and every kernel argument
 // held in spilled scalar registers); 40 x 5 x 100,001 FP64 paths with 30 swaptions: 1.21 ms (2.82 ms).
 //
 // Conventions of the reference's AAD (RandomVariableDifferentiableAAD.java:165-219): averages
@@ -280,7 +280,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
         const int hi = (c + stride - 1 < k->a.nT) ? c + stride - 1 : k->a.nT;
         for (int t = hi; t >= c; t--) {
             k = adjoint_arguments();
-            const int P = k->a.P, n = k->a.n, nT = k->a.nT, F = k->a.F, rec_n = k->a.rec_n;
+            const int P = k->a.P, n = k->a.n, nT = k->a.nT, rec_n = k->a.rec_n;
             const bool active = p0 < (uint32_t)P;
             const uint32_t pc = active ? p0 : (uint32_t)P - 1;
             const ConstArray<double> times{k->a.times};
@@ -297,13 +297,15 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
             {
                 const real* src = (t > c && t < hi) ? (const real*)k->g.seg + (size_t)(t - c - 1) * n * P
                                                     : (const real*)k->a.ckpt + (size_t)(c / stride) * n * P;
+                const int cf = opaque(cfirst);
                 static_for<0, W * NCH>([&](auto J) {
                     constexpr int j = decltype(J)::value;
-                    if ((unsigned)(j - cfirst) < held) X.template put<j>(__builtin_nontemporal_load(src + pc));
+                    if ((unsigned)(j - cf) < held) X.template put<j>(__builtin_nontemporal_load(src + pc));
                     src += P;
                 });
             }
             auto increments = [&](real (&dW)[FCAP], int s) {
+                const int F = opaque(k->a.F);
                 const real* dwp = (const real*)k->a.dw + ((size_t)pc * nT + s) * F;
                 if (F == FCAP) {
 #pragma unroll
@@ -326,9 +328,10 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                                                           (float)k->a.cap);
                     if (s + 1 < hi) {
                         real* to = (real*)k->g.seg + (size_t)(s - c) * n * P;
+                        const int cf = opaque(cfirst);
                         static_for<0, W * NCH>([&](auto J) {
                             constexpr int j = decltype(J)::value;
-                            if ((unsigned)(j - cfirst) < held && active)
+                            if ((unsigned)(j - cf) < held && active)
                                 __builtin_nontemporal_store(X.template at<j>(), to + pc);
                             to += P;
                         });

@@ -180,6 +180,15 @@ __device__ __forceinline__ ArgPtr kernel_arguments() {
     return a;
 }
 
+// A uniform value whose origin the compiler does not see: comparisons with it are made where they are
+// used, instead of being hoisted out of a loop as one mask per unrolled component and spilled.
+__device__ __forceinline__ int opaque(int x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(x));
+#endif
+    return x;
+}
+
 // Record of one (time step, component).
 template <int FCAP, typename real>
 struct Rec {
