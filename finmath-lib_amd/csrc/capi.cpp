@@ -135,7 +135,7 @@ struct fm_lmm {
     bool uniform_dt = false;            // all simulation steps have the same length
     std::vector<std::vector<double>> berm_fixing;   // fixing dates of the Bermudans of the last pass
 
-    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_Y0cap, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
+    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
     DevBuf d_states, d_poly, d_dw, d_row_of, d_paths, d_num;
     DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib, d_out, d_swapmeta, d_scale;
     DevBuf d_ckpt, d_ckpt_first, d_seg, d_adj_num, d_kcur, d_fsig, d_sig, d_cdiag, d_wave_grad, d_grad_out;
@@ -174,11 +174,14 @@ struct fm_lmm {
         return cfg.precision == FM_PRECISION_FP64_LOGSTATE && cfg.state_space == FM_STATE_SPACE_LOGNORMAL && !terminal() &&
                !pc() && (!carry() || std::isinf(cfg.libor_cap)) && !has_lv && !has_sv;
     }
-    // the FP64 spot kernel (lmm_spot64.hpp): base-2 log-forwards, its own record layout
+    // the FP64 spot kernel (lmm_spot64.hpp)
     bool spot64() const { return !fp32() && (plain_euler() || logstate()); }
     bool spot32() const { return fp32() && plain_euler(); }
-    // records per time step: the spot kernels read them in pairs
-    int rec_n() const { return spot64() || spot32() ? n() + (n() & 1) : n(); }
+    bool wrapped() const { return has_lv || has_sv; }
+    // records per time step: all kernels but the FP32 general one read them in pairs
+    int rec_n() const { return !fp32() || spot32() ? n() + (n() & 1) : n(); }
+    // factor capacity of the kernel that runs: the general ones start at three factors
+    int fcap() const { return spot64() || spot32() ? fcap_of(F()) : std::max(3, fcap_of(F())); }
     size_t real_size() const { return fp32() ? sizeof(float) : sizeof(double); }
     int process_time_index(double t) const { return jsearch(times, round_tick(t)); }
     int libor_index(double t) const { return jsearch(tenor, round_tick(t)); }
@@ -280,35 +283,45 @@ void prepare_model(fm_lmm* c) {
     const bool lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL;
     // records per (step i, component j): lambda_j.(t_i) zero-padded to the factor capacity,
     // variance*(-0.5) (0 in the normal state space), d/d and 1/d
-    const int fcap = fcap_of(F), rs = rec_size_of(fcap);
-    // the FP64 spot kernel's records (lmm_spot64.hpp) scale each forward by its initial value (where
-    // that is an ordinary positive number); the spot kernels' hold no loadings for the forwards fixed
-    // at t_i, and the FP64 one touches the records of the pair after the last one
-    const bool spot64 = c->spot64(), spot = spot64 || c->spot32();
+    // FP64 records (lmm_spot64.hpp, lmm_general64.hpp) scale each forward by its initial value where that is
+    // an ordinary positive number. Records read in pairs (all but the FP32 general kernel's) hold no loadings
+    // for the forwards fixed at t_i and an absent forward after an odd last one; the kernels read or
+    // touch up to four records past the last.
+    const bool fp64 = !c->fp32(), paired = fp64 || c->spot32();
+    const bool carried = fp64 && c->carry() && !c->spot64();    // the value is capped, not the state
+    const int fcap = c->fcap(), rs = rec_size_of(fcap);
     const int rec_n = c->rec_n();
+    const double cap = c->cfg.libor_cap;
     std::vector<double> rec(((size_t)nT * rec_n + 4) * rs, 0.0), lead((size_t)2 * n, 1.0), z0((size_t)n, 0.0);
-    std::vector<double> zcap((size_t)n, c->cfg.libor_cap);
+    std::vector<double> zcap((size_t)n, cap);
     for (int j = 0; j < n; j++) {
-        if (!lognormal) continue;
+        if (!lognormal) {
+            z0[(size_t)j] = carried ? c->L0[(size_t)j] : c->init_value[(size_t)j];
+            continue;
+        }
         const double v = c->L0[(size_t)j];
         if (v >= 1e-12 && v <= 1e12) { lead[(size_t)j] = v; lead[(size_t)(n + j)] = 1.0 / v; }
         // log2(0) is a finite number whose power underflows to zero
         else z0[(size_t)j] = v > 0.0 ? std::log2(v) : -1.0e9;
-        if (!std::isinf(c->cfg.libor_cap)) zcap[(size_t)j] = std::log2(c->cfg.libor_cap / lead[(size_t)j]);
-        z0[(size_t)j] = std::min(z0[(size_t)j], zcap[(size_t)j]);
+        if (std::isinf(cap)) continue;
+        zcap[(size_t)j] = carried ? cap / lead[(size_t)j] : std::log2(cap / lead[(size_t)j]);
+        if (!carried) z0[(size_t)j] = std::min(z0[(size_t)j], zcap[(size_t)j]);
     }
     for (int i = 0; i < nT; i++)
         for (int j = 0; j < rec_n; j++) {
             double* r = rec.data() + ((size_t)i * rec_n + j) * rs;
-            if (j == n) { r[fcap + 1] = spot64 ? HUGE_VAL : 1.0; r[fcap + 2] = 1.0; continue; }     // absent forward of the last pair
-            const bool fixed = spot && j < c->first_alive[(size_t)i];
-            if (!fixed) {
+            if (j == n) { r[fcap + 1] = fp64 ? HUGE_VAL : 1.0; r[fcap + 2] = 1.0; continue; }
+            if (!paired || j >= c->first_alive[(size_t)i]) {
                 for (int k = 0; k < F; k++) r[k] = c->lam[((size_t)i * n + j) * F + k];
                 r[fcap] = lognormal ? c->var[(size_t)i * n + j] * (-0.5) : 0.0;
             }
             const double d = delta[(size_t)j];
-            if (spot64) {
+            if (fp64) {
                 r[fcap] *= (c->times[(size_t)i + 1] - c->times[(size_t)i]) * kLog2E;
+                if (c->wrapped()) {                 // the wrappers' variance: the sum of squares of the loadings
+                    r[fcap] = 0.0;
+                    for (int k = 0; k < F; k++) r[fcap] += r[k] * r[k];
+                }
                 r[fcap + 1] = zcap[(size_t)j];
                 r[fcap + 2] = 1.0 / d * lead[(size_t)(n + j)];
                 continue;
@@ -318,6 +331,18 @@ void prepare_model(fm_lmm* c) {
             r[fcap + 1] = d / m;
             r[fcap + 2] = 1.0 / m;
         }
+    // FP64 wrappers: the local-volatility factor a_j E_j + b_ij as pairs {a_j, b_ij}, 1 without
+    std::vector<double> lvt;
+    if (fp64 && c->wrapped()) {
+        lvt.assign((size_t)nT * rec_n * 2, 0.0);
+        for (int i = 0; i < nT; i++)
+            for (int j = 0; j < n; j++) {
+                double* q = lvt.data() + ((size_t)i * rec_n + j) * 2;
+                q[0] = c->has_lv ? (c->lv_alpha == 0.0 ? 1.0 : 1.0 - c->lv_alpha) * lead[(size_t)j] : 0.0;
+                q[1] = c->has_lv ? c->lvb[(size_t)i * n + j] : 1.0;
+            }
+        upload(c->d_lvb, lvt, s);
+    }
     upload(c->d_times, c->times, s);
     upload(c->d_first, c->first_alive, s);
     upload(c->d_tenor_ti, c->tenor_ti, s);
@@ -327,34 +352,26 @@ void prepare_model(fm_lmm* c) {
     // host staging buffers stay alive until the stream synchronisation below
     std::vector<float> rf, lvf;
     std::vector<double> l0d;
-    if (c->has_lv) {
-        if (c->fp32()) { lvf.assign(c->lvb.begin(), c->lvb.end()); upload(c->d_lvb, lvf, s); }
-        else upload(c->d_lvb, c->lvb, s);
-    }
+    // initial state of the FP32 carried schemes (LMM.getInitialState:1081-1093): log(max(L_j(0), 0)) or
+    // L_j(0), uncapped
+    std::vector<double> y0((size_t)n);
     if (c->fp32()) {
+        if (c->has_lv) { lvf.assign(c->lvb.begin(), c->lvb.end()); upload(c->d_lvb, lvf, s); }
         rf.assign(rec.begin(), rec.end());
         upload(c->d_rec, rf, s);
         l0d.resize((size_t)n);                              // float-rounded initial state, passed as double
         for (int j = 0; j < n; j++) l0d[(size_t)j] = (double)(float)c->init_value[(size_t)j];
         upload(c->d_L0, l0d, s);
+        for (int j = 0; j < n; j++)
+            y0[(size_t)j] = lognormal ? std::log(std::max(c->L0[(size_t)j], 0.0)) : c->L0[(size_t)j];
+        upload(c->d_Y0, y0, s);
+        z0 = c->init_value;     // the FP32 spot kernel's states are the forwards
     } else {
         upload(c->d_rec, rec, s);
-        upload(c->d_L0, c->init_value, s);
+        upload(c->d_lead, lead, s);
     }
-    // initial state (LMM.getInitialState:1081-1093): log(max(L_j(0), 0)) or L_j(0), uncapped
-    std::vector<double> y0((size_t)n);
-    for (int j = 0; j < n; j++)
-        y0[(size_t)j] = lognormal ? std::log(std::max(c->L0[(size_t)j], 0.0)) : c->L0[(size_t)j];
-    upload(c->d_Y0, y0, s);
-    // the log-forward kernel caps its log-states (Y <= log(cap))
-    std::vector<double> y0c(y0);
-    if (!std::isinf(c->cfg.libor_cap))
-        for (double& y : y0c) y = std::min(y, std::log(c->cfg.libor_cap));
-    upload(c->d_Y0cap, y0c, s);
-    if (!spot64 || !lognormal) z0 = c->init_value;       // states that are the forwards themselves
     z0.resize(80, 0.0);         // the register array's capacity
     upload(c->d_z0, z0, s);
-    upload(c->d_lead, lead, s);
     // terminal measure N(T_0): the Scalar chain of the time-0 values (LMM:1028-1042,
     // stochastic/Scalar.java:320-328)
     c->n0_terminal = 1.0;
@@ -521,7 +538,7 @@ static void make_walks(const fm_lmm* c, Lowered& L) {
         }
         return;
     }
-    if (!c->spot64()) return;
+    if (c->fp32() || c->terminal()) return;
     int last = -1;          // time index of the last group that got a walk
     for (size_t i = 0; i < L.kp.size(); i += 1 + (size_t)(L.kp[i].type == FM_PRODUCT_SWAPTION ? L.kp[i].pad2 : 0)) {
         KProduct& k = L.kp[i];
@@ -1006,7 +1023,6 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.delta = c->d_delta.as<double>();
     a.L0 = c->d_L0.as<double>();
     a.Y0 = c->d_Y0.as<double>();
-    a.logcap = std::isinf(c->cfg.libor_cap) ? HUGE_VAL : std::log(c->cfg.libor_cap);
     a.terminal = c->terminal() ? 1 : 0;
     a.carry = c->carry() ? 1 : 0;
     a.pc = c->pc() ? 1 : 0;
@@ -1027,38 +1043,28 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.ckpt_stride = ckpt ? ckpt_stride : 1;
     a.ckpt_first = ckpt_first;
     tm.mark(2);
-    const bool lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL;
     // kernel variant: the spot-measure Euler kernels, else the general kernel (terminal
     // measure, carried state, predictor-corrector)
     a.rec_n = c->rec_n();
-    if (c->spot64()) {
+    a.lv_alpha = c->lv_alpha;
+    a.lvb = (c->fp32() ? c->has_lv : c->wrapped()) ? c->d_lvb.p : nullptr;
+    a.svs = c->has_sv ? c->d_svs.p : nullptr;
+    if (c->fp32()) {
+        a.walk = xs ? xs->upload(L.walk32, s) : upload(c->d_walk, L.walk32, s);
+        if (c->wrapped()) launch_lmm_step_lv_fp32(a, s);
+        else if (c->plain_euler()) {
+            a.Y0 = c->d_z0.as<double>();        // the capped initial forwards
+            launch_lmm_step_fp32(a, s);
+        } else if (c->pc()) launch_lmm_step_pc_fp32(a, s);
+        else launch_lmm_step_general_fp32(a, s);
+    } else {
         a.Y0 = c->d_z0.as<double>();
         a.lead = c->d_lead.as<double>();
-    a.walk = c->d_walk.p;           // uploaded by the pricing pass
         a.walk = xs ? xs->upload(L.walk, s) : upload(c->d_walk, L.walk, s);
-        launch_lmm_step_fp64(a, s);
-    } else if (c->has_lv || c->has_sv) {
-        a.lv_alpha = c->lv_alpha;
-        a.lvb = c->has_lv ? c->d_lvb.p : nullptr;
-        a.svs = c->has_sv ? c->d_svs.p : nullptr;
-        if (c->fp32()) launch_lmm_step_lv_fp32(a, s);
-        else launch_lmm_step_lv_fp64(a, s);
-    } else if (c->plain_euler()) {
-        a.Y0 = c->d_z0.as<double>();            // the capped initial forwards
-        a.walk = xs ? xs->upload(L.walk32, s) : upload(c->d_walk, L.walk32, s);
-        launch_lmm_step_fp32(a, s);
-    } else {
-        // the general kernel: FP64 log-normal functional schemes carry the log-forwards, capped
-        // at log(cap), like the spot kernel
-        if (!c->fp32() && c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL && !c->carry())
-            a.Y0 = c->d_Y0cap.as<double>();
-        if (c->pc()) {
-            if (c->fp32()) launch_lmm_step_pc_fp32(a, s);
-            else launch_lmm_step_pc_fp64(a, s);
-        } else {
-            if (c->fp32()) launch_lmm_step_general_fp32(a, s);
-            else launch_lmm_step_general_fp64(a, s);
-        }
+        if (c->spot64()) launch_lmm_step_fp64(a, s);
+        else if (c->wrapped()) launch_lmm_step_lv_fp64(a, s);
+        else if (c->pc()) launch_lmm_step_pc_fp64(a, s);
+        else launch_lmm_step_general_fp64(a, s);
     }
     tm.mark(3);
     // numeraire-adjustment averages first (the swap contributions need them)

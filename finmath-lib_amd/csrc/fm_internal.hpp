@@ -106,17 +106,17 @@ struct StepArgs {
     int lognormal, capped;       // state space is LOGNORMAL; the liborCap applies
     const double* delta;         // device n: T_{j+1}-T_j
     const double* L0;            // device n: initial forwards in value space
-    const double* lead;          // FP64 spot kernel, device [2][n]: the forwards' scales s_j and 1/s_j
+    const double* lead;          // FP64 kernels, device [2][n]: the forwards' scales s_j and 1/s_j
     const void* walk;            // spot kernels, device [rows][8]: walk tables of swaption groups (path precision)
     const double* Y0;            // device n: initial states (log(max(L0, 0)) or L0) of the carried schemes;
                                  // for the log-forward and spot kernels kept below log(cap)
                                  // (the spot kernel in the normal state space: the capped forwards)
-    double logcap;               // the cap of a carried log-value: log(cap), log2(cap) for the FP64 spot kernel
     int terminal;                // TERMINAL measure (general kernel)
     int carry;                   // EULER / PREDICTOR_CORRECTOR: the state is carried (general kernel)
     int pc;                      // predictor-corrector (general kernel)
     double lv_alpha;             // local-volatility factor (L - L alpha) + b_ij, or L + b_ij for alpha = 0
-    const void* lvb;             // device [nT][n] b_ij (double or float), or NULL; local-volatility kernels only
+    const void* lvb;             // wrapper kernels: FP32 device [nT][n] b_ij or NULL, FP64 device [nT][rec_n] pairs
+                                 // {s_j (1 - alpha), b_ij}
     const void* svs;             // device [nT][P] stochastic volatility scaling (double or float), or NULL
     const void* dw;              // device dW [P][nT][F]
     double cap;

@@ -77,9 +77,6 @@ template <typename real> __device__ __forceinline__ real spot_div_r(real a, real
 template <> __device__ __forceinline__ double spot_div_r<double>(double a, double b, double r) { return fm_div_nr_r(a, b, r); }
 template <> __device__ __forceinline__ float spot_div_r<float>(float a, float, float r) { return a * r; }
 
-// The path kernels carry log-forwards in FP64 and values in FP32.
-template <typename real> constexpr bool carries_log() { return std::is_same<real, double>::value; }
-
 // Products evaluated at time index ti, in the order they were lowered (qp advances over them):
 // swaptions and caplets are reduced into their wave partials, swap periods and Bermudan
 // regression bases go to per-path contribution columns. Y holds the path's states and val(y, j)

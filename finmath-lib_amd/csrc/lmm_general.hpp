@@ -1,6 +1,7 @@
-// General path kernel: the terminal or spot measure, the carried-state EULER and
-// PREDICTOR_CORRECTOR schemes and their functional forms, both state spaces, and the
-// local-volatility and stochastic-volatility wrappers of the covariance model.
+// General path kernel in FP32-mixed arithmetic: the terminal or spot measure, the carried-state EULER
+// and PREDICTOR_CORRECTOR schemes and their functional forms, both state spaces, and the
+// local-volatility and stochastic-volatility wrappers of the covariance model. (FP64:
+// lmm_general64.hpp.)
 //
 // Per time step t_i -> t_{i+1}, alive component j, in the order of
 // LIBORMarketModelFromCovarianceModel.getDrift (LMM:1132-1181) and
@@ -25,7 +26,6 @@ struct Variant {
     bool carry;        // EULER / PREDICTOR_CORRECTOR: the state is carried between steps
                        // (else the *_FUNCTIONAL schemes re-derive it from the value, Euler:234-237)
     real cap;
-    real logcap;       // log(cap), the cap of a carried log-value
     real lv_alpha;     // local-volatility factor f = (L - L alpha) + b_ij, or L + b_ij for alpha = 0
     const real* lvb;   // b_ij, [nT][n], or NULL: no local-volatility factor (LV kernels only)
     const real* svs;   // stochastic volatility scaling S(t_i) [nT][P], or NULL (LV kernels only)
@@ -77,12 +77,8 @@ __device__ __forceinline__ real drift_component(real (&S)[FCAP], const Rec<FCAP,
     return mu + R.hv();
 }
 
-// One step of all alive components, in place. X holds the value (functional schemes), the
-// state (carried schemes) or, LOGCARRY, the log-value of each component.
-// LOGCARRY (FP64, log-normal, functional schemes): the functional scheme takes the log of the
-// capped value, log(min(exp(Y), cap)) = min(Y, log(cap)) since log(exp(Y)) returns Y exactly at
-// the forwards' magnitudes (the spot kernel's argument, lmm_spot.hpp), so the log-value is
-// carried and capped at log(cap), and the step needs no logarithm.
+// One step of all alive components, in place. X holds the value (functional schemes) or the state
+// (carried schemes) of each component.
 // PC: the reference evaluates the predictor's drift of every component, then the predicted
 // values, then the corrector's drift on them, and adds ((mu_pred - mu) / 2) dt to the state
 // (Euler:292-314). Component j's two drifts depend only on the components before it in the
@@ -92,12 +88,9 @@ __device__ __forceinline__ real drift_component(real (&S)[FCAP], const Rec<FCAP,
 // LV: the loadings of the drift and the diffusion carry the local-volatility factor of the
 // value the drift is evaluated on (the start value; the predicted value in the corrector) and
 // the path's stochastic volatility scaling at t_i.
-// STAGE: the step's increments are read from this thread's LDS slots sdw[k * kStepThreads]
-// instead of registers (the FP64 predictor-corrector: it frees the registers a third wave per
-// SIMD needs).
-template <int NCH, int FCAP, typename real, bool TERMINAL, bool PC, bool LV, bool LOGCARRY, bool STAGE>
+template <int NCH, int FCAP, typename real, bool TERMINAL, bool PC, bool LV>
 __device__ __forceinline__ void general_step(ChunkedForwards<NCH, real>& X, int n, int i, int first, real dt,
-                                             const real (&dW)[FCAP], const real* sdw, const real* __restrict__ rec,
+                                             const real (&dW)[FCAP], const real* __restrict__ rec,
                                              const Variant<real>& v, real* __restrict__ paths,
                                              const int32_t* __restrict__ row_next, int64_t p, int P, bool active) {
     constexpr int W = chunk_width<real>();
@@ -115,23 +108,14 @@ __device__ __forceinline__ void general_step(ChunkedForwards<NCH, real>& X, int 
             const int j = TERMINAL ? j0 + j1 - 1 - jj : jj;
             const Rec<FCAP, real> R = rec_at<FCAP, real>(rec, n, i, j);
             const real x = X.template ch<q>()[j - W * q];
-            const real Lj = LOGCARRY ? dev_exp<real>(x) : (v.carry ? to_value<real>(x, v.lognormal, v.capped, v.cap) : x);
+            const real Lj = v.carry ? to_value<real>(x, v.lognormal, v.capped, v.cap) : x;
             const real f = LV ? local_vol_factor<real>(Lj, v, i, j, n) : (real)1;
             const real mu = drift_component<FCAP, real, TERMINAL, LV>(S, R, Lj, v.lognormal, f, sv);
-            real Y = (LOGCARRY || v.carry) ? x : (v.lognormal ? dev_log<real>(Lj) : Lj);
+            real Y = v.carry ? x : (v.lognormal ? dev_log<real>(Lj) : Lj);
             Y = Y + mu * dt;
 #pragma unroll
             for (int k = 0; k < FCAP; k++) {
-                real d = dW[k];
-                if constexpr (STAGE) {
-                    // read from LDS in the component loop: the empty asm keeps the loads there
-                    const real* q = sdw;
-#if defined(__HIP_DEVICE_COMPILE__)
-                    asm volatile("" : "+v"(q));
-#endif
-                    d = q[k * kStepThreads];
-                }
-                Y = Y + d * (LV ? (R.lam(k) * f) * sv : R.lam(k));
+                Y = Y + dW[k] * (LV ? (R.lam(k) * f) * sv : R.lam(k));
             }
             if constexpr (PC) {
                 const real Lp = to_value<real>(Y, v.lognormal, v.capped, v.cap);    // predicted value
@@ -139,26 +123,18 @@ __device__ __forceinline__ void general_step(ChunkedForwards<NCH, real>& X, int 
                 const real mup = drift_component<FCAP, real, TERMINAL, LV>(Sc, R, Lp, v.lognormal, fp, sv);
                 Y = Y + ((mup - mu) * (real)0.5) * dt;
             }
-            if constexpr (LOGCARRY) {
-                const real y = v.capped ? jmin(Y, v.logcap) : Y;
-                X.template ch<q>()[j - W * q] = y;
-                if (paths && active) paths[(size_t)row_next[j] * P + p] = dev_exp<real>(y);
-            } else {
-                const real Ln = to_value<real>(Y, v.lognormal, v.capped, v.cap);
-                X.template ch<q>()[j - W * q] = v.carry ? Y : Ln;
-                if (paths && active) paths[(size_t)row_next[j] * P + p] = Ln;
-            }
+            const real Ln = to_value<real>(Y, v.lognormal, v.capped, v.cap);
+            X.template ch<q>()[j - W * q] = v.carry ? Y : Ln;
+            if (paths && active) paths[(size_t)row_next[j] * P + p] = Ln;
         }
     });
 }
 
 // SS >= 0 fixes the state space and the scheme's state at compile time (bit 0: log-normal,
 // bit 1: carried state); SS = -1 reads them from the arguments (the volatility-wrapper kernels).
-// a.Y0 holds the initial states of the carried schemes and, FP64 log-normal functional, the
-// initial log-forwards capped at log(cap); a.L0 the initial forwards.
+// a.Y0 holds the initial states of the carried schemes, a.L0 the initial forwards.
 template <int NCH, int FCAP, typename real, bool TERMINAL, bool PC, bool LV, int SS>
 __global__ void __launch_bounds__(kStepThreads)
-__attribute__((amdgpu_waves_per_eu((!LV && sizeof(real) == 8 && NCH <= 5 && FCAP <= 5) ? 3 : 1)))
 lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double* __restrict__ delta,
                    const double* __restrict__ times, const int32_t* __restrict__ first_alive,
                    const int32_t* __restrict__ tenor_ti, const KProduct* __restrict__ products,
@@ -180,26 +156,19 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
     const int stride = a.num_slots + n + 1;
     const bool lognormal = SS >= 0 ? (SS & 1) != 0 : a.lognormal != 0;
     const bool carry = SS >= 0 ? (SS & 2) != 0 : a.carry != 0;
-    constexpr bool LOGCARRY = carries_log<real>() && SS == 1;
-    // the cap is applied always: an absent cap is +inf (log-cap +inf), and jmin(x, +inf) = x
-    // for every x, NaN included
+    // the cap is applied always: an absent cap is +inf, and jmin(x, +inf) = x for every x, NaN
+    // included
     constexpr bool capped = true;
     const real cap = (real)a.cap;
-    const Variant<real> var{lognormal, capped, carry, cap, (real)a.logcap, (real)a.lv_alpha,
+    const Variant<real> var{lognormal, capped, carry, cap, (real)a.lv_alpha,
                             LV ? (const real*)a.lvb : nullptr, LV ? (const real*)a.svs : nullptr};
-    // the array holds log-values, states (carried schemes) or values; val gives the value
-    auto val = [&](real x, int) -> real {
-        return LOGCARRY ? dev_exp<real>(x) : (carry ? to_value<real>(x, lognormal, capped, cap) : x);
-    };
+    // the array holds states (carried schemes) or values; val gives the value
+    auto val = [&](real x, int) -> real { return carry ? to_value<real>(x, lognormal, capped, cap) : x; };
 
-    // FP64 predictor-corrector: the increments in LDS, [k][thread]; each thread reads only its
-    // own slots, after writing them, so no barrier is needed
-    constexpr bool STAGE = PC && !LV && sizeof(real) == 8;
-    __shared__ real sdw[STAGE ? FCAP * kStepThreads : 1];
     ChunkedForwards<NCH, real> X;
     static_for<0, W * NCH>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        X.template put<j>((j < n) ? (real)((LOGCARRY || carry) ? a.Y0[j] : a.L0[j]) : (real)0);
+        X.template put<j>((j < n) ? (real)(carry ? a.Y0[j] : a.L0[j]) : (real)0);
     });
 
     double N = 1.0, Nprev = 1.0;   // unadjusted numeraire N(T_knum) and the one before it
@@ -259,11 +228,9 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
                 if (numeraire_out && active) numeraire_out[(size_t)kcur * P + p] = N;
             }
         }
-        // ---- products evaluated at this time index; swaption groups share one walk in the FP64
-        // terminal and predictor-corrector kernels (measured 4-5% faster there; slower in FP32
-        // and in the spot Euler kernel)
-        constexpr bool group = sizeof(real) == 8 && (TERMINAL || PC);
-        eval_products_at<group, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
+        // ---- products evaluated at this time index (each swaption in a walk of its own: shared walks
+        // measured slower here)
+        eval_products_at<false, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
                                                   active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P,
                                            [](int, const KProduct&) { return false; });
 
@@ -279,14 +246,9 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
         pcs = pcs < P ? pcs : (int64_t)P - 1;
         real dW[FCAP];
         load_increments<FCAP, real>(dW, dw, pcs, nT, ti, F);
-        if constexpr (STAGE) {
-#pragma unroll
-            for (int k = 0; k < FCAP; k++) sdw[k * kStepThreads + threadIdx.x] = dW[k];
-        }
         const real dt = (real)(times[ti + 1] - times[ti]);
         const int32_t* row_next = row_of + (size_t)(ti + 1) * n;
-        general_step<NCH, FCAP, real, TERMINAL, PC, LV, LOGCARRY, STAGE>(X, n, ti, first_alive[ti], dt, dW,
-                                                               sdw + threadIdx.x, rec, var, paths, row_next,
+        general_step<NCH, FCAP, real, TERMINAL, PC, LV>(X, n, ti, first_alive[ti], dt, dW, rec, var, paths, row_next,
                                                         p, P, active);
     }
 }
@@ -332,16 +294,13 @@ void launch_general_n(const StepArgs& a, hipStream_t stream) {
     else throw FmError(FM_ERR_UNSUPPORTED, "number of factors above 10 is not supported by the path kernel");
 }
 
-// The general path kernel. Capacities 24, 40 and 80 forwards (FP64: 3, 5, 10 chunks of eight;
-// FP32: 32, 48, 80 in 2, 3, 5 chunks of sixteen) and 3, 5, 10 factors: fewer instantiations than
-// the spot kernel, whose capacities are tighter.
+// The general path kernel: capacities 32, 48 and 80 forwards in chunks of sixteen and 3, 5, 10 factors,
+// fewer instantiations than the spot kernel.
 template <typename real, bool PC, bool LV>
 void launch_general(const StepArgs& a, hipStream_t stream) {
-    constexpr int W = chunk_width<real>();
-    constexpr int N2 = W == 8 ? 3 : 2, N3 = W == 8 ? 5 : 3, N4 = W == 8 ? 10 : 5;
-    if (a.n <= W * N2) launch_general_n<N2, real, PC, LV>(a, stream);
-    else if (a.n <= W * N3) launch_general_n<N3, real, PC, LV>(a, stream);
-    else if (a.n <= 80) launch_general_n<N4, real, PC, LV>(a, stream);
+    if (a.n <= 32) launch_general_n<2, real, PC, LV>(a, stream);
+    else if (a.n <= 48) launch_general_n<3, real, PC, LV>(a, stream);
+    else if (a.n <= 80) launch_general_n<5, real, PC, LV>(a, stream);
     else throw FmError(FM_ERR_UNSUPPORTED, "more than 80 forward rates are not supported by the path kernel");
 }
 

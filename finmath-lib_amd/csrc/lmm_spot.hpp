@@ -100,20 +100,6 @@ lmm_spot_kernel(const StepArgs) {
         // ---- products evaluated at this time index. A swaption group with a walk table is left to the
         // Euler step (FP64), or valued by an unrolled walk (FP32).
         const ConstArray<KProduct> products{a->products};
-        const double inv_cnt = cnt > 0 ? 1.0 / (double)cnt : 0.0;
-        auto reduce_group = [&](int i, const KProduct& pr, const real (&V)[kSwaptionGroup]) {
-            const double Nsel = pr.num_k == knum ? N : Nprev;
-            double x[kSwaptionGroup];
-            int slot[kSwaptionGroup];
-#pragma unroll
-            for (int g = 0; g < kSwaptionGroup; g++) {
-                const KProduct pg = products[i + (g <= pr.pad2 ? g : 0)];
-                if constexpr (D) x[g] = jmax0(V[g] * pg.notional) / Nsel;
-                else x[g] = (double)jmax0(V[g]) / Nsel;
-                slot[g] = pg.out_slot;
-            }
-            reduce_slots4(x, 1 + pr.pad2, active, cnt, inv_cnt, lane, wave, a->wave_sum, a->wave_m2, stride, slot);
-        };
         int walk = -1;
         auto walk_group = [&](int i, const KProduct& pr) -> bool {
             if (pr.walk < 0) return false;
@@ -126,7 +112,15 @@ lmm_spot_kernel(const StepArgs) {
                     notional[g] = (float)products[i + (g <= pr.pad2 ? g : 0)].notional;
                 swaption_walk32<NCH>(Y, (const float*)a->walk + 8 * pr.walk, pr.first_j, pr.num_periods, 1 + pr.pad2,
                                      notional, V);
-                reduce_group(i, pr, V);
+                double x[kSwaptionGroup];
+                int slot[kSwaptionGroup];
+#pragma unroll
+                for (int g = 0; g < kSwaptionGroup; g++) {
+                    x[g] = (double)jmax0(V[g]) / (pr.num_k == knum ? N : Nprev);
+                    slot[g] = products[i + (g <= pr.pad2 ? g : 0)].out_slot;
+                }
+                reduce_slots4(x, 1 + pr.pad2, active, cnt, cnt > 0 ? 1.0 / (double)cnt : 0.0, lane, wave, a->wave_sum,
+                              a->wave_m2, stride, slot);
             }
             return true;
         };
@@ -163,7 +157,9 @@ lmm_spot_kernel(const StepArgs) {
                 sw.periods = pr.num_periods;
             }
             spot64_step<NCH, FCAP, lognormal, true>(Y, n, a->rec_n, ti, first, dt, dW, (const double*)a->rec, ke, &sw);
-            if (walk >= 0) reduce_group(walk, products[walk], sw.V);
+            if (walk >= 0)
+                reduce_walk(products, walk, sw.V, products[walk].num_k == knum ? N : Nprev, active, cnt, lane, wave,
+                            a->wave_sum, a->wave_m2, stride);
         } else {
             spot32_step<NCH, FCAP, lognormal>(Y, n, a->rec_n, ti, first, dt, dW, (const float*)a->rec, (float)a->cap);
         }

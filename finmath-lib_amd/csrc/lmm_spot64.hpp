@@ -154,4 +154,20 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
     });
 }
 
+// The values of a walk's swaptions over Nsel, reduced into their slots.
+__device__ __forceinline__ void reduce_walk(ConstArray<KProduct> products, int head,
+                                            const double (&V)[kSwaptionGroup], double Nsel, bool active, int cnt,
+                                            int lane, int64_t wave, double* wave_sum, double* wave_m2, int stride) {
+    const int m = 1 + products[head].pad2;
+    double x[kSwaptionGroup];
+    int slot[kSwaptionGroup];
+#pragma unroll
+    for (int g = 0; g < kSwaptionGroup; g++) {
+        const KProduct pg = products[head + (g < m ? g : 0)];
+        x[g] = jmax0(V[g] * pg.notional) / Nsel;
+        slot[g] = pg.out_slot;
+    }
+    reduce_slots4(x, m, active, cnt, cnt > 0 ? 1.0 / (double)cnt : 0.0, lane, wave, wave_sum, wave_m2, stride, slot);
+}
+
 } // namespace fm

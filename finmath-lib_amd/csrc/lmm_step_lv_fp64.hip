@@ -1,11 +1,11 @@
-// FP64 instantiations of the general path kernel with a local-volatility covariance
-// wrapper, with and without the predictor-corrector. Compiled with -ffp-contract=off like
-// the FP64 kernel.
-#include "lmm_general.hpp"
+// FP64 instantiations of the general path kernel with the local- and stochastic-volatility wrappers.
+#include "lmm_general64.hpp"
 
 namespace fm {
+void launch_lmm_step_lvpc_fp64(const StepArgs& a, hipStream_t stream);
+
 void launch_lmm_step_lv_fp64(const StepArgs& a, void* stream) {
-    if (a.pc) launch_general<double, true, true>(a, (hipStream_t)stream);
-    else launch_general<double, false, true>(a, (hipStream_t)stream);
+    if (a.pc) launch_lmm_step_lvpc_fp64(a, (hipStream_t)stream);
+    else launch_general64<false, true>(a, (hipStream_t)stream);
 }
 }
