@@ -46,6 +46,7 @@ SOURCES = {
     "lmm_adjoint_fp32.hip": [],
     "lmm_step_fp32_80.hip": [],
     "lmm_step_fp32.hip": [],
+    "lmm_step_rows_fp64.hip": NO_CONTRACT,
     "lmm_step_general_fp64.hip": NO_CONTRACT,
     "lmm_step_pc_fp64.hip": NO_CONTRACT,
     "lmm_step_general_fp32.hip": [],

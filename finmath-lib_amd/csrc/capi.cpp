@@ -135,7 +135,7 @@ struct fm_lmm {
     bool uniform_dt = false;            // all simulation steps have the same length
     std::vector<std::vector<double>> berm_fixing;   // fixing dates of the Bermudans of the last pass
 
-    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
+    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_values, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
     DevBuf d_states, d_poly, d_dw, d_row_of, d_paths, d_num;
     DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib, d_out, d_swapmeta, d_scale;
     DevBuf d_ckpt, d_ckpt_first, d_seg, d_adj_num, d_kcur, d_fsig, d_sig, d_cdiag, d_wave_grad, d_grad_out;
@@ -1061,7 +1061,10 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
         a.Y0 = c->d_z0.as<double>();
         a.lead = c->d_lead.as<double>();
         a.walk = xs ? xs->upload(L.walk, s) : upload(c->d_walk, L.walk, s);
-        if (c->spot64()) launch_lmm_step_fp64(a, s);
+        if (c->spot64() && !ckpt && !xs && P <= kRowKernelPaths) {
+            a.values = (double*)c->d_values.get((size_t)(L.num_slots + n + 1) * P * sizeof(double));
+            launch_lmm_rows_fp64(a, s);
+        } else if (c->spot64()) launch_lmm_step_fp64(a, s);
         else if (c->wrapped()) launch_lmm_step_lv_fp64(a, s);
         else if (c->pc()) launch_lmm_step_pc_fp64(a, s);
         else launch_lmm_step_general_fp64(a, s);

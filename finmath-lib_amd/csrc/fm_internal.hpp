@@ -131,6 +131,7 @@ struct StepArgs {
     // outputs
     double* wave_sum;            // [num_waves][num_slots + n + 1]
     double* wave_m2;             // [num_waves][num_slots]
+    double* values;              // row kernel: [num_slots + n + 1][P] per-path values to be averaged
     void* paths;                 // device triangle rows [rows][P] (store_paths)
     const int32_t* row_of;       // device [(nT+1)*n] row index of (t,j), -1 = initial value
     double* numeraire;           // device [(n+1)][P] unadjusted numeraire (store_paths or adjoint)
@@ -140,6 +141,14 @@ struct StepArgs {
                                  // each checkpoint's segment on (lower rows are neither written nor read)
 };
 void launch_lmm_step_fp64(const StepArgs& a, void* stream);
+// Up to this many paths the row kernel (lmm_rows64.hpp) prices and simulates: two of its wavefronts of four paths
+// for each of the 1,024 SIMDs. Both give the same results. Whole calls, row kernel against the other, 40
+// forwards x 5 factors with 20 swaptions and a swap: 357 us against 425 at 2,000 paths, 404 against 424 at
+// 8,000, 534 against 415 at 12,000; 80 x 10: 640 against 1091, 1188 against 1467, 1623 against 1464; 20 x 3: 257
+// against 280, 278 against 278, 299 against 277. It does not write checkpoints, and its table of values is not
+// planned for in caller scratch.
+constexpr int kRowKernelPaths = 8192;
+void launch_lmm_rows_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_fp32(const StepArgs& a, void* stream);
 // General variant (terminal measure, carried state, predictor-corrector), see lmm_step.hpp.
 void launch_lmm_step_general_fp64(const StepArgs& a, void* stream);

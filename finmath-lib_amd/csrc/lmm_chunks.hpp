@@ -19,7 +19,7 @@ template <> struct VecCh<float> { typedef float t __attribute__((ext_vector_type
 template <int NCH, typename real>
 struct ChunkedForwards {
     using V = typename VecCh<real>::t;
-    static constexpr int W = chunk_width<real>();
+    static constexpr int W = chunk_width<real>(), chunks = NCH;
     static_assert(NCH >= 1 && NCH <= 10, "one to ten chunks of forwards");
     V c0, c1, c2, c3, c4, c5, c6, c7, c8, c9;
     template <int Q> __device__ __forceinline__ V& ch() {
@@ -30,6 +30,7 @@ struct ChunkedForwards {
     }
     template <int J> __device__ __forceinline__ real at() { return ch<J / W>()[J % W]; }
     template <int J> __device__ __forceinline__ void put(real v) { ch<J / W>()[J % W] = v; }
+    template <int Q> __device__ __forceinline__ real element(int e) { return ch<Q>()[e]; }
     // Element j for a uniform run-time j: one indexed register read in the chunk of j. The
     // empty asm keeps each chunk a register value, so the per-chunk reads are not merged into
     // a load from a memory copy of the forwards.
@@ -85,15 +86,14 @@ template <> __device__ __forceinline__ float spot_div_r<float>(float a, float, f
 // copy of the periods (the FP32 kernels: the shared walk measured slower there).
 // walk_group(i) takes over the swaption group at product i when it has a walk table of its own
 // (the spot kernels: valued by the Euler step or by an unrolled walk); it returns whether it did.
-template <bool GROUP, int NCH, typename real, typename Val, typename Products, typename Periods, typename Doubles,
-          typename Walk>
+// emit(x, slot) takes a per-path value for its reduction slot.
+template <bool GROUP, typename real, typename Chunks, typename Val, typename Products, typename Periods,
+          typename Doubles, typename Emit, typename Walk>
 __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_products, Products products,
-                                                 Periods periods, Doubles delta,
-                                                 double N, double Nprev, int knum, ChunkedForwards<NCH, real>& Y,
-                                                 Val&& val, bool active, int cnt, int lane, int64_t wave,
-                                                 double* __restrict__ wave_sum, double* __restrict__ wave_m2,
-                                                 int stride, double* __restrict__ contrib, int64_t p, int P, Walk&& walk_group) {
-    constexpr int W = chunk_width<real>();
+                                                 Periods periods, Doubles delta, double N, double Nprev, int knum,
+                                                 Chunks& Y, Val&& val, bool active, double* __restrict__ contrib,
+                                                 int64_t p, int P, Emit&& emit, Walk&& walk_group) {
+    constexpr int W = Chunks::W, NCH = Chunks::chunks;
     auto value_of = [&](int j) -> real { return val(Y.get(j), j); };
     while (qp < num_products && products[qp].eval_index == ti) {
         const KProduct pr = products[qp];
@@ -122,7 +122,7 @@ __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_produc
 #pragma unroll 1
                 for (int j = jb - 1; j >= ja; j--) {
                     const KPeriod pe = periods[pr.param_off + (j - j0)];
-                    const real Lj = val(Y.template ch<q>()[j - W * q], j);
+                    const real Lj = val(Y.template element<q>(j - W * q), j);
                     const real b = (real)1.0 + Lj * (real)pe.tau;
                     const real r = spot_rcp<real>(b);
                     // every member's strike and notional are read up front (indices clamped to the
@@ -148,8 +148,7 @@ __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_produc
 #pragma unroll
             for (int g = 0; g < G; g++)
                 if (g < m)
-                    reduce_slot((double)jmax0(V[g]) / Nsel, active, cnt, lane, wave, wave_sum, wave_m2, stride,
-                                products[qp - 1 + g].out_slot);
+                    emit((double)jmax0(V[g]) / Nsel, products[qp - 1 + g].out_slot);
             qp += m - 1;
         } else if (pr.type == FM_PRODUCT_CAPLET) {
             const KPeriod pe = periods[pr.param_off];
@@ -157,8 +156,7 @@ __device__ __forceinline__ void eval_products_at(int ti, int& qp, int num_produc
             real v = Lj - (real)pe.strike;
             if (!pr.is_floorlet) v = jmax0(v) * (real)pe.notional;
             else v = ((v != v) ? v : (v > (real)0 ? (real)0 : v)) * ((real)(-1.0) * (real)pe.notional);
-            const double x = (double)v / Nsel;
-            reduce_slot(x, active, cnt, lane, wave, wave_sum, wave_m2, stride, pr.out_slot);
+            emit((double)v / Nsel, pr.out_slot);
         } else if (pr.type == K_BERM_BASIS) {
             // raw regression basis of a Bermudan exercise date T_e (BermudanSwaption.java:215-252)
             if (pr.flags == FM_BASIS_REFERENCE) {

@@ -230,9 +230,12 @@ lmm_general_kernel(const StepArgs a, const real* __restrict__ rec, const double*
         }
         // ---- products evaluated at this time index (each swaption in a walk of its own: shared walks
         // measured slower here)
-        eval_products_at<false, NCH, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val,
-                                                  active, cnt, lane, wave, wave_sum, wave_m2, stride, contrib, p, P,
-                                           [](int, const KProduct&) { return false; });
+        eval_products_at<false, real>(ti, qp, a.num_products, products, periods, delta, N, Nprev, knum, X, val, active,
+                                      contrib, p, P,
+                                      [&](double x, int slot) {
+                                          reduce_slot(x, active, cnt, lane, wave, wave_sum, wave_m2, stride, slot);
+                                      },
+                                      [](int, const KProduct&) { return false; });
 
         if (ti == nT) break;
 

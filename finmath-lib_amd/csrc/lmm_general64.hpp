@@ -19,9 +19,8 @@
 // and state, the corrector's drift on the predicted value and the corrected state.
 // Carried schemes cap the value min(2^z, cap/s_j) where it is read; functional ones cap the state.
 //
-// The FP64 vector pipeline bounds it, as it does the spot kernel. Every option is a template argument:
-// with the schemes chosen at run time the step took 2.1 times the instructions. 200,000 paths, 40 forwards,
-// 5 factors, 40 steps, terminal measure, PREDICTOR_CORRECTOR: 0.93 ms at 0.56 of the vector issue slots
+// The FP64 vector pipeline bounds it, as it does the spot kernel. 200,000 paths, 40 forwards,
+// 5 factors, 40 steps, terminal measure, PREDICTOR_CORRECTOR: 0.93 ms
 // (1.86 ms for the kernel with natural exponentials, divisions and rolled components that this one replaces);
 // 150,000 paths, spot measure, normal, stochastic volatility: 0.42 ms (1.50 ms).
 #pragma once
@@ -265,9 +264,11 @@ lmm_general64_kernel(const StepArgs) {
             walk = i;
             return true;
         };
-        eval_products_at<true, NCH, double>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
-                                            ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, cnt, lane, wave,
-                                            a->wave_sum, a->wave_m2, stride, a->contrib, p, P, walk_group);
+        eval_products_at<true, double>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
+                                       ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, a->contrib, p, P,
+                                       [&](double x, int slot) {
+                                           reduce_slot(x, active, cnt, lane, wave, a->wave_sum, a->wave_m2, stride, slot);
+                                       }, walk_group);
         const int nT = a->nT;
         if (ti == nT) break;
 

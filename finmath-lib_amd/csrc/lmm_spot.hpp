@@ -124,9 +124,11 @@ lmm_spot_kernel(const StepArgs) {
             }
             return true;
         };
-        eval_products_at<D, NCH, real>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
-                                       ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, cnt, lane, wave,
-                                       a->wave_sum, a->wave_m2, stride, a->contrib, p, P, walk_group);
+        eval_products_at<D, real>(ti, qp, a->num_products, products, ConstArray<KPeriod>{a->periods},
+                                       ConstArray<double>{a->delta}, N, Nprev, knum, Y, val, active, a->contrib, p, P,
+                                       [&](double x, int slot) {
+                                           reduce_slot(x, active, cnt, lane, wave, a->wave_sum, a->wave_m2, stride, slot);
+                                       }, walk_group);
         const int nT = a->nT;
         if (ti == nT) break;
 
