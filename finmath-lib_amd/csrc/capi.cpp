@@ -58,6 +58,60 @@ static T* upload(DevBuf& b, const std::vector<T>& v, hipStream_t s) {
     return d;
 }
 
+// Grow-only pinned host memory.
+struct PinnedBuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() { if (p) (void)hipHostFree(p); }
+    void* get(size_t need) {
+        if (need > bytes) {
+            if (g_no_alloc)
+                throw FmError(FM_ERR_STATE, "the context would have to allocate host staging memory: call the allocating "
+                                            "entry point once with this model first");
+            if (p) { HIP_CHECK(hipHostFree(p)); p = nullptr; bytes = 0; }
+            HIP_CHECK(hipHostMalloc(&p, need, hipHostMallocDefault));
+            bytes = need;
+        }
+        return p;
+    }
+};
+
+// Several host tables sent to the device by one copy from pinned memory. A copy from pageable memory costs the
+// calling thread some 10 us, and the tables of a small pass are a few kilobytes each: a calibration pass
+// (2,000 paths, 40 forwards x 5 factors) spent 180 of its 397 us on eleven of them and the wait that kept their
+// sources alive. The staging memory outlives the call; the stream is waited for before it is written
+// again, unless its owner has done so since (pending).
+struct Staged {
+    struct Piece { const void* src; size_t bytes, at; };
+    DevBuf dev;
+    PinnedBuf host;
+    std::vector<Piece> pieces;
+    size_t total = 0;
+    bool pending = false;
+    void begin() { pieces.clear(); total = 0; }
+    // Adds a table, which has to live until send; returns its offset.
+    template <class T> size_t add(const std::vector<T>& v) {
+        const size_t at = total, bytes = v.size() * sizeof(T);
+        pieces.push_back({v.data(), bytes, at});
+        total += (std::max<size_t>(bytes, 8) + 255) & ~(size_t)255;
+        return at;
+    }
+    char* send(hipStream_t s) {
+        if (pending) HIP_CHECK(hipStreamSynchronize(s));
+        pending = false;
+        char* d = (char*)dev.get(total);
+        char* h = (char*)host.get(total);
+        for (const Piece& p : pieces)
+            if (p.bytes) std::memcpy(h + p.at, p.src, p.bytes);
+        HIP_CHECK(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, s));
+        pending = true;
+        return d;
+    }
+};
+
 // Device memory handed in by the caller for the per-call buffers of one pass (wave
 // partials, product tables, reduction output), taken in 256-byte aligned pieces.
 struct ExternalScratch {
@@ -135,9 +189,15 @@ struct fm_lmm {
     bool uniform_dt = false;            // all simulation steps have the same length
     std::vector<std::vector<double>> berm_fixing;   // fixing dates of the Bermudans of the last pass
 
-    DevBuf d_times, d_first, d_tenor_ti, d_rec, d_delta, d_L0, d_Y0, d_values, d_z0, d_lead, d_walk, d_sqrt_dt, d_lvb, d_svs;
+    DevBuf d_times, d_first, d_tenor_ti, d_delta, d_values, d_sqrt_dt, d_svs;
+    Staged model, tables, late;         // model records; product tables; swap tables of the finishing pass
+    PinnedBuf h_out;                    // averages of a pass, written by the reduction
+    // of the model and of the last pass's product tables, on the device
+    const void *m_rec = nullptr, *m_lvb = nullptr, *m_walk = nullptr;
+    const double *m_L0 = nullptr, *m_Y0 = nullptr, *m_z0 = nullptr, *m_lead = nullptr;
+    bool grid_ready = false;            // the tables of times and tenor dates are on the device
     DevBuf d_states, d_poly, d_dw, d_row_of, d_paths, d_num;
-    DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib, d_out, d_swapmeta, d_scale;
+    DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib;
     DevBuf d_ckpt, d_ckpt_first, d_seg, d_adj_num, d_kcur, d_fsig, d_sig, d_cdiag, d_wave_grad, d_grad_out;
     DevBuf d_berm_vals, d_berm_under, d_berm_ex, d_berm_part, d_berm_coef, d_berm_col, d_berm_scale;
     // the Bermudan induction's adjoint: triggers and choices recorded by the pricing pass
@@ -177,6 +237,7 @@ struct fm_lmm {
     // the FP64 spot kernel (lmm_spot64.hpp)
     bool spot64() const { return !fp32() && (plain_euler() || logstate()); }
     bool spot32() const { return fp32() && plain_euler(); }
+    void idle() { model.pending = tables.pending = late.pending = false; }      // the stream has been waited for
     bool wrapped() const { return has_lv || has_sv; }
     // records per time step: all kernels but the FP32 general one read them in pairs
     int rec_n() const { return !fp32() || spot32() ? n() + (n() & 1) : n(); }
@@ -200,6 +261,7 @@ int fail(const std::exception& e) {
 #define FM_CATCH } catch (const std::exception& e) { return fail(e); } catch (...) { set_last_error("unknown error"); return FM_ERR_INTERNAL; }
 
 void require(bool cond, int code, const std::string& msg) { if (!cond) throw FmError(code, msg); }
+void require(bool cond, int code, const char* msg) { if (!cond) throw FmError(code, msg); }   // no string unless it fails
 
 struct DeviceGuard {
     int prev = -1;
@@ -244,19 +306,39 @@ void prepare_model(fm_lmm* c) {
     if (!c->tables_dirty) return;
     const int n = c->n(), nT = c->nT(), F = c->F();
     hipStream_t s = c->stream;
-    // first alive component at each step (LMM.getDrift:1126-1130)
-    c->first_alive.assign((size_t)nT, 0);
-    for (int i = 0; i < nT; i++) {
-        int f = jsearch(c->tenor, round_tick(c->times[(size_t)i])) + 1;
-        if (f < 0) f = -f - 1 + 1;
-        c->first_alive[(size_t)i] = std::min(f, n);
-    }
-    // process time index of each tenor date, rounded up (LMM:1055-1058)
-    c->tenor_ti.assign((size_t)n + 1, nT + 1);
-    for (int k = 0; k <= n; k++) {
-        int ti = c->process_time_index(c->tenor[(size_t)k]);
-        if (ti < 0) ti = -ti - 1;
-        c->tenor_ti[(size_t)k] = ti;
+    std::vector<double> delta((size_t)n);
+    for (int j = 0; j < n; j++) delta[(size_t)j] = c->tenor[(size_t)j + 1] - c->tenor[(size_t)j];
+    if (!c->grid_ready) {       // times and tenor dates are those the context was made with
+        // first alive component at each step (LMM.getDrift:1126-1130)
+        c->first_alive.assign((size_t)nT, 0);
+        for (int i = 0; i < nT; i++) {
+            int f = jsearch(c->tenor, round_tick(c->times[(size_t)i])) + 1;
+            if (f < 0) f = -f - 1 + 1;
+            c->first_alive[(size_t)i] = std::min(f, n);
+        }
+        // process time index of each tenor date, rounded up (LMM:1055-1058)
+        c->tenor_ti.assign((size_t)n + 1, nT + 1);
+        for (int k = 0; k <= n; k++) {
+            int ti = c->process_time_index(c->tenor[(size_t)k]);
+            if (ti < 0) ti = -ti - 1;
+            c->tenor_ti[(size_t)k] = ti;
+        }
+        // materialised-process row map
+        c->row_of.assign((size_t)(nT + 1) * n, -1);
+        int r = 0;
+        for (int ti = 1; ti <= nT; ti++)
+            for (int j = 0; j < n; j++) {
+                if (j >= c->first_alive[(size_t)ti - 1]) c->row_of[(size_t)ti * n + j] = r++;
+                else c->row_of[(size_t)ti * n + j] = c->row_of[(size_t)(ti - 1) * n + j];
+            }
+        c->num_rows = r;
+        upload(c->d_times, c->times, s);
+        upload(c->d_first, c->first_alive, s);
+        upload(c->d_tenor_ti, c->tenor_ti, s);
+        upload(c->d_delta, delta, s);
+        upload(c->d_row_of, c->row_of, s);
+        HIP_CHECK(hipStreamSynchronize(s));
+        c->grid_ready = true;
     }
     // time-0 process value: transform(initial state) (Euler:187-192, LMM:1081-1093,1200-1212)
     c->init_value.assign((size_t)n, 0.0);
@@ -267,19 +349,6 @@ void prepare_model(fm_lmm* c) {
         if (!std::isinf(c->cfg.libor_cap)) v = std::min(v, c->cfg.libor_cap);
         c->init_value[(size_t)j] = v;
     }
-    // materialised-process row map
-    c->row_of.assign((size_t)(nT + 1) * n, -1);
-    int r = 0;
-    for (int ti = 1; ti <= nT; ti++)
-        for (int j = 0; j < n; j++) {
-            if (j >= c->first_alive[(size_t)ti - 1]) c->row_of[(size_t)ti * n + j] = r++;
-            else c->row_of[(size_t)ti * n + j] = c->row_of[(size_t)(ti - 1) * n + j];
-        }
-    c->num_rows = r;
-    std::vector<double> delta((size_t)n), sq((size_t)nT);
-    for (int j = 0; j < n; j++) delta[(size_t)j] = c->tenor[(size_t)j + 1] - c->tenor[(size_t)j];
-    for (int i = 0; i < nT; i++) sq[(size_t)i] = std::sqrt(c->times[(size_t)i + 1] - c->times[(size_t)i]);
-    c->uniform_dt = std::all_of(sq.begin(), sq.end(), [&](double v) { return v == sq[0]; });
     const bool lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL;
     // records per (step i, component j): lambda_j.(t_i) zero-padded to the factor capacity,
     // variance*(-0.5) (0 in the normal state space), d/d and 1/d
@@ -341,37 +410,40 @@ void prepare_model(fm_lmm* c) {
                 q[0] = c->has_lv ? (c->lv_alpha == 0.0 ? 1.0 : 1.0 - c->lv_alpha) * lead[(size_t)j] : 0.0;
                 q[1] = c->has_lv ? c->lvb[(size_t)i * n + j] : 1.0;
             }
-        upload(c->d_lvb, lvt, s);
     }
-    upload(c->d_times, c->times, s);
-    upload(c->d_first, c->first_alive, s);
-    upload(c->d_tenor_ti, c->tenor_ti, s);
-    upload(c->d_delta, delta, s);
-    upload(c->d_sqrt_dt, sq, s);
-    upload(c->d_row_of, c->row_of, s);
-    // host staging buffers stay alive until the stream synchronisation below
     std::vector<float> rf, lvf;
-    std::vector<double> l0d;
-    // initial state of the FP32 carried schemes (LMM.getInitialState:1081-1093): log(max(L_j(0), 0)) or
-    // L_j(0), uncapped
-    std::vector<double> y0((size_t)n);
+    std::vector<double> l0d, y0;
+    Staged& up = c->model;
+    up.begin();
+    size_t at_lvb = 0, at_L0 = 0, at_Y0 = 0, at_lead = 0, at_rec;
     if (c->fp32()) {
-        if (c->has_lv) { lvf.assign(c->lvb.begin(), c->lvb.end()); upload(c->d_lvb, lvf, s); }
+        // initial state of the carried schemes (LMM.getInitialState:1081-1093): log(max(L_j(0), 0)) or
+        // L_j(0), uncapped
+        for (int j = 0; j < n; j++) {
+            y0.push_back(lognormal ? std::log(std::max(c->L0[(size_t)j], 0.0)) : c->L0[(size_t)j]);
+            l0d.push_back((double)(float)c->init_value[(size_t)j]);     // float-rounded, passed as double
+        }
+        lvf.assign(c->lvb.begin(), c->lvb.end());
         rf.assign(rec.begin(), rec.end());
-        upload(c->d_rec, rf, s);
-        l0d.resize((size_t)n);                              // float-rounded initial state, passed as double
-        for (int j = 0; j < n; j++) l0d[(size_t)j] = (double)(float)c->init_value[(size_t)j];
-        upload(c->d_L0, l0d, s);
-        for (int j = 0; j < n; j++)
-            y0[(size_t)j] = lognormal ? std::log(std::max(c->L0[(size_t)j], 0.0)) : c->L0[(size_t)j];
-        upload(c->d_Y0, y0, s);
         z0 = c->init_value;     // the FP32 spot kernel's states are the forwards
+        at_rec = up.add(rf);
+        at_lvb = up.add(lvf);
+        at_L0 = up.add(l0d);
+        at_Y0 = up.add(y0);
     } else {
-        upload(c->d_rec, rec, s);
-        upload(c->d_lead, lead, s);
+        at_rec = up.add(rec);
+        at_lvb = up.add(lvt);
+        at_lead = up.add(lead);
     }
     z0.resize(80, 0.0);         // the register array's capacity
-    upload(c->d_z0, z0, s);
+    const size_t at_z0 = up.add(z0);
+    const char* base = up.send(s);
+    c->m_rec = base + at_rec;
+    c->m_lvb = base + at_lvb;
+    c->m_L0 = (const double*)(base + at_L0);
+    c->m_Y0 = (const double*)(base + at_Y0);
+    c->m_lead = (const double*)(base + at_lead);
+    c->m_z0 = (const double*)(base + at_z0);
     // terminal measure N(T_0): the Scalar chain of the time-0 values (LMM:1028-1042,
     // stochastic/Scalar.java:320-328)
     c->n0_terminal = 1.0;
@@ -379,7 +451,6 @@ void prepare_model(fm_lmm* c) {
         const double v = c->n0_terminal;
         c->n0_terminal = 1.0 / (c->init_value[(size_t)j] * (delta[(size_t)j] / v) + 1.0 / v);
     }
-    HIP_CHECK(hipStreamSynchronize(s));
     c->tables_dirty = false;
 }
 
@@ -991,23 +1062,41 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     const int n = c->n(), P = c->P();
     if (xs) require(L.num_contrib == 0 && L.berm.empty() && !store && !ckpt, FM_ERR_INTERNAL,
                     "a pass in caller scratch takes single-date products only");
-    Timer tm(c);
-    tm.mark(0);
-    if (c->cfg.regenerate_increments) c->dw_ready = false;
-    const bool regen = !c->dw_ready;
-    ensure_brownian(c);
-    tm.mark(1);
     const int64_t num_waves = ((int64_t)P + 63) / 64;
     const int stride = L.num_slots + n + 1;
     const size_t wbytes = (size_t)num_waves * stride * sizeof(double);
     double* wsum = (double*)(xs ? xs->take(wbytes) : c->d_wave_sum.get(wbytes));
     double* wm2 = (double*)(xs ? xs->take(wbytes) : c->d_wave_m2.get(wbytes));
+    // the product tables
+    const KProduct* d_kp;
+    const KPeriod* d_per;
     if (xs) {
+        d_kp = xs->upload(L.kp, s);
+        d_per = xs->upload(L.per, s);
+        c->m_walk = c->fp32() ? (const void*)xs->upload(L.walk32, s) : (const void*)xs->upload(L.walk, s);
+    } else {
+        Staged& up = c->tables;
+        up.begin();
+        const size_t at_kp = up.add(L.kp), at_per = up.add(L.per), at_walk = c->fp32() ? up.add(L.walk32) : up.add(L.walk);
+        const char* base = up.send(s);
+        d_kp = (const KProduct*)(base + at_kp);
+        d_per = (const KPeriod*)(base + at_per);
+        c->m_walk = base + at_walk;
+    }
+    Timer tm(c);
+    tm.mark(0);
+    if (c->cfg.regenerate_increments) c->dw_ready = false;
+    const bool regen = !c->dw_ready;
+    ensure_brownian(c);
+    if (regen) tm.mark(1);
+    // The path kernel writes every partial but those of numeraires and products beyond the simulation and
+    // of swaps and Bermudans, which follow; partials that nothing writes are cleared.
+    bool unwritten = xs != nullptr;
+    for (int32_t ti : c->tenor_ti) unwritten = unwritten || ti > c->nT();
+    for (const KProduct& k : L.kp) unwritten = unwritten || k.eval_index < 0 || k.eval_index > c->nT();
+    if (unwritten) {
         launch_fill_zero(wsum, (size_t)num_waves * stride, s);
         launch_fill_zero(wm2, (size_t)num_waves * stride, s);
-    } else {
-        HIP_CHECK(hipMemsetAsync(wsum, 0, wbytes, s));
-        HIP_CHECK(hipMemsetAsync(wm2, 0, wbytes, s));
     }
     StepArgs a{};
     a.nT = c->nT(); a.n = n; a.F = c->F(); a.P = P;
@@ -1017,12 +1106,13 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.times = c->d_times.as<double>();
     a.first_alive = c->d_first.as<int32_t>();
     a.tenor_time_index = c->d_tenor_ti.as<int32_t>();
-    a.rec = c->d_rec.p;
+    a.rec = c->m_rec;
     a.lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL ? 1 : 0;
     a.capped = std::isinf(c->cfg.libor_cap) ? 0 : 1;
     a.delta = c->d_delta.as<double>();
-    a.L0 = c->d_L0.as<double>();
-    a.Y0 = c->d_Y0.as<double>();
+    a.L0 = c->m_L0;
+    a.Y0 = c->m_Y0;
+    a.walk = c->m_walk;
     a.terminal = c->terminal() ? 1 : 0;
     a.carry = c->carry() ? 1 : 0;
     a.pc = c->pc() ? 1 : 0;
@@ -1030,8 +1120,8 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.cap = c->cfg.libor_cap;
     a.scheme = c->cfg.scheme;
     a.num_products = (int)L.kp.size();
-    a.products = xs ? xs->upload(L.kp, s) : upload(c->d_products, L.kp, s);
-    a.periods = xs ? xs->upload(L.per, s) : upload(c->d_periods, L.per, s);
+    a.products = d_kp;
+    a.periods = d_per;
     a.num_slots = L.num_slots;
     a.num_contrib = L.num_contrib;
     a.contrib = L.num_contrib ? (double*)c->d_contrib.get((size_t)L.num_contrib * P * sizeof(double)) : nullptr;
@@ -1042,25 +1132,22 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.ckpt = ckpt;
     a.ckpt_stride = ckpt ? ckpt_stride : 1;
     a.ckpt_first = ckpt_first;
-    tm.mark(2);
     // kernel variant: the spot-measure Euler kernels, else the general kernel (terminal
     // measure, carried state, predictor-corrector)
     a.rec_n = c->rec_n();
     a.lv_alpha = c->lv_alpha;
-    a.lvb = (c->fp32() ? c->has_lv : c->wrapped()) ? c->d_lvb.p : nullptr;
+    a.lvb = (c->fp32() ? c->has_lv : c->wrapped()) ? c->m_lvb : nullptr;
     a.svs = c->has_sv ? c->d_svs.p : nullptr;
     if (c->fp32()) {
-        a.walk = xs ? xs->upload(L.walk32, s) : upload(c->d_walk, L.walk32, s);
         if (c->wrapped()) launch_lmm_step_lv_fp32(a, s);
         else if (c->plain_euler()) {
-            a.Y0 = c->d_z0.as<double>();        // the capped initial forwards
+            a.Y0 = c->m_z0;        // the capped initial forwards
             launch_lmm_step_fp32(a, s);
         } else if (c->pc()) launch_lmm_step_pc_fp32(a, s);
         else launch_lmm_step_general_fp32(a, s);
     } else {
-        a.Y0 = c->d_z0.as<double>();
-        a.lead = c->d_lead.as<double>();
-        a.walk = xs ? xs->upload(L.walk, s) : upload(c->d_walk, L.walk, s);
+        a.Y0 = c->m_z0;
+        a.lead = c->m_lead;
         if (c->spot64() && !ckpt && !xs && P <= kRowKernelPaths) {
             a.values = (double*)c->d_values.get((size_t)(L.num_slots + n + 1) * P * sizeof(double));
             launch_lmm_rows_fp64(a, s);
@@ -1072,12 +1159,21 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     tm.mark(3);
     // numeraire-adjustment averages first (the swap contributions need them)
     const int cols = L.num_slots + n + 1;
-    double* dout = (double*)(xs ? xs->take((size_t)cols * 2 * sizeof(double)) : c->d_out.get((size_t)cols * 2 * sizeof(double)));
+    // into pinned host memory, unless the caller's scratch is to hold them
+    double* dout = (double*)(xs ? xs->take((size_t)cols * 2 * sizeof(double)) : c->h_out.get((size_t)cols * 2 * sizeof(double)));
     launch_reduce_partials(wsum, wm2, (int)num_waves, stride, L.num_slots, n + 1, P, dout, dout + cols, s);
-    sums.assign((size_t)cols, 0.0); m2s.assign((size_t)cols, 0.0);
-    HIP_CHECK(hipMemcpyAsync(sums.data(), dout, cols * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(m2s.data(), dout + cols, cols * sizeof(double), hipMemcpyDeviceToHost, s));
+    std::vector<double> out;
+    if (xs) {
+        out.resize((size_t)cols * 2);
+        HIP_CHECK(hipMemcpyAsync(out.data(), dout, out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
+    const bool more = !L.swap_slot.empty() || !L.berm.empty();
+    if (!more) tm.mark(4);
     HIP_CHECK(hipStreamSynchronize(s));
+    c->idle();
+    const double* host = xs ? out.data() : dout;
+    sums.assign(host, host + cols);
+    m2s.assign(host + cols, host + 2 * cols);
     // zb_k = average of N(0)/N(T_k) (LMM:872)
     c->zb.assign((size_t)n + 1, 1.0);
     if (c->terminal()) {
@@ -1094,7 +1190,7 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
             c->zb[1] = (1.0 / N1) * 1.0;
         }
     }
-    if (!L.swap_slot.empty() || !L.berm.empty()) {
+    if (more) {
         const std::vector<double> adj = adjustment_chain(c);
         if (!L.swap_slot.empty()) {
             std::vector<double> scale((size_t)L.num_contrib, 1.0);
@@ -1102,12 +1198,16 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
                 const int k = L.contrib_k[(size_t)col];
                 if (k >= 0) scale[(size_t)col] = value_scale(c, k, adj);
             }
-            const double* dscale = upload(c->d_scale, scale, s);
             std::vector<int32_t> meta;
             meta.insert(meta.end(), L.swap_col0.begin(), L.swap_col0.end());
             meta.insert(meta.end(), L.swap_ncol.begin(), L.swap_ncol.end());
             meta.insert(meta.end(), L.swap_slot.begin(), L.swap_slot.end());
-            const int32_t* dmeta = upload(c->d_swapmeta, meta, s);
+            Staged& up = c->late;
+            up.begin();
+            const size_t at_scale = up.add(scale), at_meta = up.add(meta);
+            const char* base = up.send(s);
+            const double* dscale = (const double*)(base + at_scale);
+            const int32_t* dmeta = (const int32_t*)(base + at_meta);
             const int ns = (int)L.swap_slot.size();
             launch_swap_finalize(a.contrib, P, ns, dmeta, dmeta + ns, dmeta + 2 * ns, dscale, wsum, wm2, stride, s);
         }
@@ -1117,17 +1217,16 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
         for (size_t bi = 0; bi < L.berm.size(); bi++)
             run_bermudan(c, L.berm[bi], (int)bi, adj, a.contrib, wsum, wm2, stride);
         launch_reduce_partials(wsum, wm2, (int)num_waves, stride, L.num_slots, 0, P, dout, dout + cols, s);
-        std::vector<double> s2((size_t)cols), m2b((size_t)cols);
-        HIP_CHECK(hipMemcpyAsync(s2.data(), dout, L.num_slots * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipMemcpyAsync(m2b.data(), dout + cols, L.num_slots * sizeof(double), hipMemcpyDeviceToHost, s));
+        tm.mark(4);
         HIP_CHECK(hipStreamSynchronize(s));
+        c->idle();
+        const double *s2 = dout, *m2b = dout + cols;
         for (int ss : L.swap_slot) { sums[(size_t)ss] = s2[(size_t)ss]; m2s[(size_t)ss] = m2b[(size_t)ss]; }
         for (const BermPlan& b : L.berm) { sums[(size_t)b.slot] = s2[(size_t)b.slot]; m2s[(size_t)b.slot] = m2b[(size_t)b.slot]; }
     }
-    tm.mark(4);
     HIP_CHECK(hipEventSynchronize(c->ev[4]));
     c->timings[0] = regen ? tm.span(0, 1) : 0.0;
-    c->timings[1] = tm.span(2, 3);
+    c->timings[1] = tm.span(regen ? 1 : 0, 3);
     c->timings[2] = tm.span(3, 4);
     c->timings[4] = tm.span(0, 4);
 }
@@ -1667,14 +1766,14 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
     a.precision = c->cfg.precision; a.state_space = c->cfg.state_space;
     a.times = c->d_times.as<double>(); a.first_alive = c->d_first.as<int32_t>();
     a.tenor_time_index = c->d_tenor_ti.as<int32_t>();
-    a.rec = c->d_rec.p;
+    a.rec = c->m_rec;
     a.lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL ? 1 : 0;
     a.capped = std::isinf(c->cfg.libor_cap) ? 0 : 1;
     a.delta = c->d_delta.as<double>();
-    a.L0 = c->d_L0.as<double>(); a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
+    a.L0 = c->m_L0; a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
     a.rec_n = c->rec_n();
-    a.lead = c->d_lead.as<double>();
-    a.walk = c->d_walk.p;           // uploaded by the pricing pass
+    a.lead = c->m_lead;
+    a.walk = c->m_walk;           // uploaded by the pricing pass
     a.num_products = (int)kp.size();
     a.products = upload(c->d_products, kp, s);
     a.periods = upload(c->d_periods, L.per, s);
