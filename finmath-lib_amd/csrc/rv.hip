@@ -10,6 +10,12 @@
 // only the arithmetic of the program plus one load per input and one store: a program
 // of any length is one HBM pass. The inputs of an element are loaded together before
 // the program runs, so their latencies overlap, and each thread runs two elements.
+//
+// Sixteen registers and sixteen inputs of two elements fill the register file at two wavefronts per SIMD,
+// and the dispatch of a short program, loads and constants among its instructions, then takes longer
+// than its memory traffic. A program whose inputs, constants and intermediate values fit eight registers
+// runs on rv_compact_kernel: loads and constants are registers set before the program starts, and the
+// registers left let a thread run four elements per dispatch at large sizes.
 // Reductions (averages, variances) run the same program and sum the result with
 // compensated (Neumaier) partial sums in a fixed order, so they are reproducible.
 // Compiled with -ffp-contract=off: a + b * c rounds twice, as the JVM evaluates it.
@@ -45,7 +51,7 @@ constexpr int kRvMaxBlocks = 8192;              // reduction grid (fixed order o
 
 struct RvProg {
     int32_t n, nin, result, mode;               // mode: 0 store, 1 sum, 2 sum of squared deviations
-    double mean;                                // mode 2
+    const double* total;                        // mode 2: the mode 1 sum; its mean over size is subtracted
     int64_t size;
     const double* prob;                         // mode 1: weights (NULL: none)
     double prob_const;
@@ -54,6 +60,20 @@ struct RvProg {
     double cst[FM_RV_MAX_INPUTS];
 };
 static_assert(sizeof(RvProg) < 4000, "program must fit the kernel argument segment");
+
+// A program for eight registers: input i (or a constant) is in register i when it starts.
+constexpr int kRvCompact = 8;
+struct RvCompact {
+    int32_t n, nin, result, mode;
+    const double* total;
+    int64_t size;
+    const double* prob;
+    double prob_const;
+    uint32_t code[FM_RV_MAX_INSTRUCTIONS];      // opcode | dst << 8 | a << 12 | b << 16 | c << 20
+    double imm[FM_RV_MAX_INSTRUCTIONS];
+    const double* in[kRvCompact];
+    double cst[kRvCompact];
+};
 
 __host__ __device__ inline bool sign_bit(double x) {
     uint64_t u;
@@ -115,6 +135,31 @@ __host__ __device__ inline bool heavy_op(int op) {
     return op == FM_RV_POW || op == FM_RV_EXPM1 || op == FM_RV_SIN || op == FM_RV_COS;
 }
 
+// r[e] = op(a[e], b[e], c[e], imm) for a uniform opcode: one arm per launch-wide opcode.
+template <int E, bool FULL>
+__device__ __forceinline__ void run_op(int op, const double (&a)[E], const double (&b)[E], const double (&c)[E], double imm,
+                                       double (&r)[E]) {
+    switch (op) {
+#define FM_RV_OP(o) case o: for (int e = 0; e < E; e++) r[e] = apply_op(o, a[e], b[e], c[e], imm); break;
+    FM_RV_OP(FM_RV_CONST) FM_RV_OP(FM_RV_ADD) FM_RV_OP(FM_RV_SUB) FM_RV_OP(FM_RV_MULT) FM_RV_OP(FM_RV_DIV)
+    FM_RV_OP(FM_RV_CAP) FM_RV_OP(FM_RV_FLOOR) FM_RV_OP(FM_RV_EXP) FM_RV_OP(FM_RV_LOG)
+    FM_RV_OP(FM_RV_SQRT) FM_RV_OP(FM_RV_ABS) FM_RV_OP(FM_RV_INVERT) FM_RV_OP(FM_RV_SQUARED)
+    FM_RV_OP(FM_RV_ADD_PRODUCT) FM_RV_OP(FM_RV_ADD_RATIO) FM_RV_OP(FM_RV_SUB_RATIO) FM_RV_OP(FM_RV_ACCRUE)
+    FM_RV_OP(FM_RV_DISCOUNT) FM_RV_OP(FM_RV_CHOOSE) FM_RV_OP(FM_RV_ISNAN)
+    default:
+        if constexpr (FULL) {
+            switch (op) {
+            FM_RV_OP(FM_RV_POW) FM_RV_OP(FM_RV_EXPM1) FM_RV_OP(FM_RV_SIN) FM_RV_OP(FM_RV_COS)
+            default: for (int e = 0; e < E; e++) r[e] = a[e]; break;
+            }
+        } else {
+            for (int e = 0; e < E; e++) r[e] = a[e];
+        }
+        break;
+#undef FM_RV_OP
+    }
+}
+
 // Run the program on E elements (idx[e] < size when ok[e]); returns the result register.
 template <int E, bool FULL>
 __device__ __forceinline__ void run_program(const RvProg& g, const int64_t (&idx)[E], const bool (&ok)[E],
@@ -144,25 +189,7 @@ __device__ __forceinline__ void run_program(const RvProg& g, const int64_t (&idx
             double a[E], b[E], c[E];
 #pragma unroll
             for (int e = 0; e < E; e++) { a[e] = R[e][ia]; b[e] = R[e][ib]; c[e] = R[e][ic]; }
-            switch (op) {     // uniform: one arm per launch-wide opcode
-#define FM_RV_OP(o) case o: for (int e = 0; e < E; e++) r[e] = apply_op(o, a[e], b[e], c[e], in.imm); break;
-            FM_RV_OP(FM_RV_CONST) FM_RV_OP(FM_RV_ADD) FM_RV_OP(FM_RV_SUB) FM_RV_OP(FM_RV_MULT) FM_RV_OP(FM_RV_DIV)
-            FM_RV_OP(FM_RV_CAP) FM_RV_OP(FM_RV_FLOOR) FM_RV_OP(FM_RV_EXP) FM_RV_OP(FM_RV_LOG)
-            FM_RV_OP(FM_RV_SQRT) FM_RV_OP(FM_RV_ABS) FM_RV_OP(FM_RV_INVERT) FM_RV_OP(FM_RV_SQUARED)
-            FM_RV_OP(FM_RV_ADD_PRODUCT) FM_RV_OP(FM_RV_ADD_RATIO) FM_RV_OP(FM_RV_SUB_RATIO) FM_RV_OP(FM_RV_ACCRUE)
-            FM_RV_OP(FM_RV_DISCOUNT) FM_RV_OP(FM_RV_CHOOSE) FM_RV_OP(FM_RV_ISNAN)
-            default:
-                if constexpr (FULL) {
-                    switch (op) {
-                    FM_RV_OP(FM_RV_POW) FM_RV_OP(FM_RV_EXPM1) FM_RV_OP(FM_RV_SIN) FM_RV_OP(FM_RV_COS)
-                    default: for (int e = 0; e < E; e++) r[e] = a[e]; break;
-                    }
-                } else {
-                    for (int e = 0; e < E; e++) r[e] = a[e];
-                }
-                break;
-#undef FM_RV_OP
-            }
+            run_op<E, FULL>(op, a, b, c, in.imm, r);
         }
 #pragma unroll
         for (int e = 0; e < E; e++) R[e][id] = r[e];
@@ -179,6 +206,28 @@ __device__ __forceinline__ void neumaier_add(double& s, double& c, double x) {
     s = t;
 }
 
+// Fixed-order tree over the block: (sum, compensation) pairs.
+__device__ __forceinline__ void block_partial(double s, double comp, double* __restrict__ partials) {
+    __shared__ double ss[kRvThreads], sc[kRvThreads];
+    ss[threadIdx.x] = s;
+    sc[threadIdx.x] = comp;
+    __syncthreads();
+    for (int w = kRvThreads / 2; w >= 1; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            double a = ss[threadIdx.x], ca = sc[threadIdx.x];
+            neumaier_add(a, ca, ss[threadIdx.x + w]);
+            ca += sc[threadIdx.x + w];
+            ss[threadIdx.x] = a;
+            sc[threadIdx.x] = ca;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        partials[2 * blockIdx.x] = ss[0];
+        partials[2 * blockIdx.x + 1] = sc[0];
+    }
+}
+
 // Store mode: out[i] = program(i). Reduction modes: per-block (sum, compensation) of the
 // program's value (mode 1, times the weight), or of (value - mean)^2 (mode 2, times the
 // weight). Each thread visits its elements in increasing order (grid-stride) and the
@@ -191,6 +240,7 @@ __global__ void __launch_bounds__(kRvThreads) __attribute__((amdgpu_waves_per_eu
                                                                double* __restrict__ partials) {
     constexpr int E = kRvPerThread;
     const int64_t span = (int64_t)gridDim.x * kRvThreads * E;
+    const double mean = g.mode == 2 ? *g.total / (double)g.size : 0.0;
     double s = 0.0, comp = 0.0;
     for (int64_t base = (int64_t)blockIdx.x * kRvThreads * E; base < g.size; base += span) {
         int64_t idx[E];
@@ -210,32 +260,77 @@ __global__ void __launch_bounds__(kRvThreads) __attribute__((amdgpu_waves_per_eu
             for (int e = 0; e < E; e++) {
                 if (!ok[e]) continue;
                 double x = v[e];
-                if (g.mode == 2) { const double d = x - g.mean; x = d * d; }
+                if (g.mode == 2) { const double d = x - mean; x = d * d; }
                 if (g.prob || g.prob_const != 1.0) x = x * (g.prob ? g.prob[idx[e]] : g.prob_const);
                 neumaier_add(s, comp, x);
             }
         }
     }
     if (g.mode == 0) return;
-    // fixed-order tree over the block: (sum, compensation) pairs
-    __shared__ double ss[kRvThreads], sc[kRvThreads];
-    ss[threadIdx.x] = s;
-    sc[threadIdx.x] = comp;
-    __syncthreads();
-    for (int w = kRvThreads / 2; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            double a = ss[threadIdx.x], ca = sc[threadIdx.x];
-            neumaier_add(a, ca, ss[threadIdx.x + w]);
-            ca += sc[threadIdx.x + w];
-            ss[threadIdx.x] = a;
-            sc[threadIdx.x] = ca;
+    block_partial(s, comp, partials);
+}
+
+// The same for a compact program, E elements per thread: the elements of E / 2 consecutive trips of
+// rv_eval_kernel's loop, taken in its order, so the sums are the same. E = 4 where its grid makes more
+// than one trip. Bound by memory: x * y + z, discounted and capped, 16.8 million elements: 99 us stored
+// (0.54 GB, 5.4 TB/s; 225 us on sixteen registers).
+template <int E>
+__global__ void __launch_bounds__(kRvThreads) __attribute__((amdgpu_waves_per_eu(E == 4 ? 3 : 4)))
+rv_compact_kernel(const RvCompact g, double* __restrict__ out, double* __restrict__ partials) {
+    typedef double File __attribute__((ext_vector_type(kRvCompact)));
+    const int64_t span = (int64_t)gridDim.x * kRvThreads * 2;
+    const double mean = g.mode == 2 ? *g.total / (double)g.size : 0.0;
+    double s = 0.0, comp = 0.0;
+    for (int64_t base = (int64_t)blockIdx.x * kRvThreads * 2; base < g.size; base += span * (E / 2)) {
+        int64_t idx[E];
+        bool ok[E];
+        File R[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            idx[e] = base + (e / 2) * span + (int64_t)(e % 2) * kRvThreads + threadIdx.x;
+            ok[e] = idx[e] < g.size;
         }
-        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kRvCompact; i++) {
+            const double* src = i < g.nin ? g.in[i] : nullptr;      // uniform
+#pragma unroll
+            for (int e = 0; e < E; e++) R[e][i] = src != nullptr ? (ok[e] ? src[idx[e]] : 0.0) : g.cst[i];
+        }
+        uint32_t next = g.code[0];
+        double next_imm = g.imm[0];
+#pragma unroll 1
+        for (int k = 0; k < g.n; k++) {
+            const uint32_t code = next;
+            const double imm = next_imm;
+            const int k1 = k + 1 < FM_RV_MAX_INSTRUCTIONS ? k + 1 : k;      // read ahead of its dispatch
+            next = g.code[k1];
+            next_imm = g.imm[k1];
+            const int id = (code >> 8) & 15, ia = (code >> 12) & 15, ib = (code >> 16) & 15, ic = (code >> 20) & 15;
+            double a[E], b[E], c[E], r[E];
+#pragma unroll
+            for (int e = 0; e < E; e++) { a[e] = R[e][ia]; b[e] = R[e][ib]; c[e] = R[e][ic]; }
+            run_op<E, false>((int)(code & 255), a, b, c, imm, r);
+#pragma unroll
+            for (int e = 0; e < E; e++) R[e][id] = r[e];
+        }
+        double v[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = R[e][g.result];
+        if (g.mode == 0) {
+#pragma unroll
+            for (int e = 0; e < E; e++) if (ok[e]) out[idx[e]] = v[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                if (!ok[e]) continue;
+                double x = v[e];
+                if (g.mode == 2) { const double d = x - mean; x = d * d; }
+                if (g.prob || g.prob_const != 1.0) x = x * (g.prob ? g.prob[idx[e]] : g.prob_const);
+                neumaier_add(s, comp, x);
+            }
+        }
     }
-    if (threadIdx.x == 0) {
-        partials[2 * blockIdx.x] = ss[0];
-        partials[2 * blockIdx.x + 1] = sc[0];
-    }
+    if (g.mode != 0) block_partial(s, comp, partials);
 }
 
 // One workgroup: thread t merges the block partials of its contiguous chunk in order,
@@ -370,7 +465,103 @@ RvProg make_prog(int32_t nin, const fm_rv* const* inputs, int32_t nins, const fm
     return g;
 }
 
+// Operands that an opcode reads.
+int operands(int op) {
+    switch (op) {
+    case FM_RV_ADD: case FM_RV_SUB: case FM_RV_MULT: case FM_RV_DIV: case FM_RV_CAP: case FM_RV_FLOOR: case FM_RV_POW:
+    case FM_RV_ACCRUE: case FM_RV_DISCOUNT: return 2;
+    case FM_RV_ADD_PRODUCT: case FM_RV_ADD_RATIO: case FM_RV_SUB_RATIO: case FM_RV_CHOOSE: return 3;
+    default: return 1;
+    }
+}
+
+// The program on eight registers: inputs and constants become initial registers, intermediate values take
+// the registers whose last use has passed. False where eight do not suffice or a heavy opcode occurs.
+bool compact_program(const RvProg& g, RvCompact& c) {
+    struct Value { int kind, input; double constant; int last, slot; };     // kind: 0 input, 1 constant, 2 computed
+    std::vector<Value> vals;
+    struct Step { int op, v[3], out; double imm; };
+    std::vector<Step> steps;
+    vals.reserve(FM_RV_MAX_INSTRUCTIONS + FM_RV_REGISTERS);
+    steps.reserve(FM_RV_MAX_INSTRUCTIONS);
+    auto leaf = [&](int kind, int input, double constant) -> int {
+        for (size_t i = 0; i < vals.size(); i++)
+            if (vals[i].kind == kind && (kind == 0 ? vals[i].input == input
+                                                   : std::memcmp(&vals[i].constant, &constant, sizeof(double)) == 0)) return (int)i;
+        vals.push_back({kind, input, constant, -1, -1});
+        return (int)vals.size() - 1;
+    };
+    int cur[FM_RV_REGISTERS];
+    for (int& r : cur) r = -1;
+    auto read = [&](int r) -> int { if (cur[r] < 0) cur[r] = leaf(1, 0, 0.0); return cur[r]; };    // registers start at 0
+    for (int k = 0; k < g.n; k++) {
+        const fm_rv_instr& in = g.ins[k];
+        if (heavy_op(in.op)) return false;
+        if (in.op == FM_RV_LOAD) {
+            cur[in.dst] = g.in[in.a] ? leaf(0, in.a, 0.0) : leaf(1, 0, g.cst[in.a]);
+        } else if (in.op == FM_RV_CONST) {
+            cur[in.dst] = leaf(1, 0, in.imm);
+        } else {
+            Step st{in.op, {-1, -1, -1}, 0, in.imm};
+            const int m = operands(in.op), reg[3] = {in.a, in.b, in.c};
+            for (int i = 0; i < m; i++) st.v[i] = read(reg[i]);
+            vals.push_back({2, 0, 0.0, -1, -1});
+            st.out = cur[in.dst] = (int)vals.size() - 1;
+            steps.push_back(st);
+        }
+    }
+    const int result = read(g.result);
+    // last uses, from the end; a step whose value nothing uses has no effect and is dropped
+    vals[(size_t)result].last = (int)steps.size();
+    for (int k = (int)steps.size() - 1; k >= 0; k--) {
+        if (vals[(size_t)steps[(size_t)k].out].last < 0) continue;
+        for (int v : steps[(size_t)k].v)
+            if (v >= 0 && vals[(size_t)v].last < 0) vals[(size_t)v].last = k;
+    }
+    std::memset(&c, 0, sizeof(c));
+    unsigned used = 0;
+    for (Value& v : vals) {
+        if (v.kind == 2 || v.last < 0) continue;
+        if (c.nin == kRvCompact) return false;
+        v.slot = c.nin;
+        used |= 1u << c.nin;
+        c.in[c.nin] = v.kind == 0 ? g.in[v.input] : nullptr;
+        c.cst[c.nin++] = v.constant;
+    }
+    for (int k = 0; k < (int)steps.size(); k++) {
+        const Step& st = steps[(size_t)k];
+        Value& out = vals[(size_t)st.out];
+        if (out.last < 0) continue;
+        uint32_t code = (uint32_t)st.op;
+        for (int i = 0; i < 3; i++) {
+            if (st.v[i] < 0) continue;
+            const Value& v = vals[(size_t)st.v[i]];
+            code |= (uint32_t)v.slot << (12 + 4 * i);
+            if (v.last == k) used &= ~(1u << v.slot);
+        }
+        int slot = 0;
+        while (slot < kRvCompact && (used & (1u << slot))) slot++;
+        if (slot == kRvCompact) return false;
+        used |= 1u << slot;
+        out.slot = slot;
+        c.code[c.n] = code | (uint32_t)slot << 8;
+        c.imm[c.n++] = st.imm;
+    }
+    c.result = vals[(size_t)result].slot;
+    c.mode = g.mode; c.total = g.total; c.size = g.size; c.prob = g.prob; c.prob_const = g.prob_const;
+    return true;
+}
+
 void launch_eval(const RvProg& g, int blocks, hipStream_t s, double* out, double* partials) {
+    RvCompact c;
+    if (compact_program(g, c)) {
+        if (g.size > (int64_t)blocks * kRvThreads * kRvPerThread)
+            hipLaunchKernelGGL(rv_compact_kernel<4>, dim3(blocks), dim3(kRvThreads), 0, s, c, out, partials);
+        else
+            hipLaunchKernelGGL(rv_compact_kernel<2>, dim3(blocks), dim3(kRvThreads), 0, s, c, out, partials);
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     bool full = false;
     for (int k = 0; k < g.n; k++) full = full || heavy_op(g.ins[k].op);
     if (full) hipLaunchKernelGGL(rv_eval_kernel<true>, dim3(blocks), dim3(kRvThreads), 0, s, g, out, partials);
@@ -383,21 +574,25 @@ int reduce_blocks(int64_t size) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(kRvMaxBlocks, (size + per - 1) / per));
 }
 
-// Sum of the program's (mode 1) or squared-deviation (mode 2) values over the realisations.
-double reduce_program(RvProg g, int device) {
+// Sum of the program's values over the realisations (out[0]) and, with deviations, of the squared
+// deviations from their mean (out[1]): the second pass reads the first one's sum on the device.
+void reduce_program(RvProg g, int device, bool deviations, double* out) {
     DevGuard dg(device);
     hipStream_t s = lib_stream(device);
-    const int blocks = reduce_blocks(g.size);
+    const int blocks = reduce_blocks(g.size), passes = deviations ? 2 : 1;
     double* buf = nullptr;
-    HIP_CHECK(hipMallocAsync((void**)&buf, (size_t)(2 * blocks + 1) * sizeof(double), s));
-    launch_eval(g, blocks, s, nullptr, buf);
-    hipLaunchKernelGGL(rv_finish_kernel, dim3(1), dim3(kRvThreads), 0, s, buf, blocks, buf + 2 * blocks);
-    HIP_CHECK(hipGetLastError());
-    double r = 0.0;
-    HIP_CHECK(hipMemcpyAsync(&r, buf + 2 * blocks, sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMallocAsync((void**)&buf, (size_t)(2 * blocks + 2) * sizeof(double), s));
+    double* result = buf + 2 * blocks;
+    for (int pass = 0; pass < passes; pass++) {
+        g.mode = 1 + pass;
+        g.total = result;
+        launch_eval(g, blocks, s, nullptr, buf);
+        hipLaunchKernelGGL(rv_finish_kernel, dim3(1), dim3(kRvThreads), 0, s, buf, blocks, result + pass);
+        HIP_CHECK(hipGetLastError());
+    }
+    HIP_CHECK(hipMemcpyAsync(out, result, passes * sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipFreeAsync(buf, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    return r;
 }
 
 } // namespace
@@ -555,19 +750,15 @@ int fm_rv_evaluate_average(int32_t nin, const fm_rv* const* inputs, int32_t nins
         return FM_OK;
     }
     RvProg g = make_prog(nin, inputs, nins, prog, result, size);
-    g.mode = 1;
     g.prob = probabilities ? probabilities->d : nullptr;
     g.prob_const = probabilities ? probabilities->value : 1.0;
-    const double mean = reduce_program(g, dev) / (double)size;
-    *average = mean;
-    if (variance) {
-        // getVariance: sum((x - avg)^2) / P; getVariance(probabilities): sum((x - avg)^2 p)
-        if (size == 1 && !probabilities) { *variance = 0.0; return FM_OK; }
-        g.mode = 2;
-        g.mean = mean;
-        const double ss = reduce_program(g, dev);
-        *variance = probabilities ? ss : ss / (double)size;
-    }
+    // the variance of a single realisation without probabilities is 0
+    const bool deviations = variance && (size > 1 || probabilities);
+    double sums[2] = {0.0, 0.0};
+    reduce_program(g, dev, deviations, sums);
+    *average = sums[0] / (double)size;
+    // getVariance: sum((x - avg)^2) / P; getVariance(probabilities): sum((x - avg)^2 p)
+    if (variance) *variance = !deviations ? 0.0 : probabilities ? sums[1] : sums[1] / (double)size;
     return FM_OK;
     RV_CATCH
 }
