@@ -1107,6 +1107,10 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     a.first_alive = c->d_first.as<int32_t>();
     a.tenor_time_index = c->d_tenor_ti.as<int32_t>();
     a.rec = c->m_rec;
+    a.model = c->model.dev.p;
+    a.model_lines = (int)(c->model.total / 128);
+    a.tables = d_kp;
+    a.table_lines = (int)(((const char*)c->m_walk - (const char*)d_kp + L.walk.size() * sizeof(double)) / 128);
     a.lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL ? 1 : 0;
     a.capped = std::isinf(c->cfg.libor_cap) ? 0 : 1;
     a.delta = c->d_delta.as<double>();

@@ -102,6 +102,8 @@ struct StepArgs {
     const int32_t* first_alive;  // device nT
     const int32_t* tenor_time_index; // device n+1: process time index of T_k (rounded up)
     const void* rec;             // device [nT][n][rec_size_of(fcap_of(F))] records (double or float)
+    const void *model, *tables;  // FP64 kernels: the model's records and the products' tables, whole, and their
+    int model_lines, table_lines;   // sizes in lines of 128 bytes
     int rec_n;                   // records per time step (n, or n rounded up to even for the spot kernels)
     int lognormal, capped;       // state space is LOGNORMAL; the liborCap applies
     const double* delta;         // device n: T_{j+1}-T_j

@@ -187,6 +187,7 @@ lmm_general64_kernel(const StepArgs) {
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Exp2Coef ke;
+    touch_tables(a);
     ChunkedForwards<NCH, double> Y;
     {
         const ConstArray<double> z0{a->Y0};

@@ -81,13 +81,8 @@ __global__ void __launch_bounds__(64) lmm_rows64_kernel(const StepArgs) {
     {
         const int P = a->P, n = a->n, nT = a->nT, F = a->F, rec_n = a->rec_n;
         const double* dw = (const double*)a->dw + (size_t)(p0 < (uint32_t)P ? p0 : P - 1) * nT * F;
-        // The tables are small and have just been written: brought into each L2 once, by the workgroups that
-        // share it (consecutive ones lie on different dies), instead of missing it again at every step.
-        // So are the increments of these paths.
-        uint32_t touched = 0;
-        const int part = blockIdx.x >> 3, parts = (gridDim.x + 7) >> 3, lines = nT * rec_n * size / 16;
-        for (int l = part * 64 + lane; l < lines; l += parts * 64)
-            touched |= *(const volatile uint32_t*)((const double*)a->rec + 16 * (size_t)l);
+        touch_tables(a);
+        uint32_t touched = 0;       // and the increments of these paths
         for (int l = 16 * g; l < nT * F; l += 256) touched |= *(const volatile uint32_t*)(dw + l);
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("" :: "v"(touched));

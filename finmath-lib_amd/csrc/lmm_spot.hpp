@@ -45,6 +45,7 @@ lmm_spot_kernel(const StepArgs) {
     // the wavefront index, uniform: kept in a scalar register
     const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Exp2Coef ke;
+    if constexpr (D) touch_tables(a);
 
     ChunkedForwards<NCH, real> Y;
     {

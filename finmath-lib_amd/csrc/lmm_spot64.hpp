@@ -29,8 +29,8 @@
 //
 // The kernel is bound by the FP64 vector pipeline. At 40 forwards x 5 factors x 1,000,000 paths with 30
 // swaptions it issues 38,500 vector instructions per wavefront (80,400 with rolled component loops,
-// a general exponential and separate products and sums) and takes 1.65 ms (3.46 ms), the vector ALUs
-// 0.73 busy (0.67) at four wavefronts per SIMD (three): the registers are held to 128 by reading the
+// a general exponential and separate products and sums) and takes 1.59 ms (3.46 ms), the vector ALUs
+// 0.74 busy (0.67) at four wavefronts per SIMD (three): the registers are held to 128 by reading the
 // kernel's arguments where they are used and the increments when the step begins. Bringing the next
 // pair's records into the scalar cache took it from 1.88 to 1.79 ms at three wavefronts; two sets of
 // scalar registers for them instead spilled.
@@ -71,6 +71,12 @@ struct SwaptionWalk {
     RecPtr table;
     int j0 = 0, periods = 0;
     double P = 1.0, V[kSwaptionGroup] = {0.0, 0.0, 0.0, 0.0};
+    // brings component j's row (the nearest one where it has none) into the scalar cache
+    __device__ __forceinline__ uint32_t touch(int j) const {
+        typedef const volatile uint32_t __attribute__((address_space(4)))* WordPtr;
+        const int i = j < j0 ? 0 : j - j0 < periods ? j - j0 : periods - 1;
+        return *(WordPtr)(table + 8 * i);
+    }
     __device__ __forceinline__ void period(int j, double E, double e, double r) {
         if ((unsigned)(j - j0) >= (unsigned)periods) return;
         typedef double Row __attribute__((ext_vector_type(8)));
@@ -82,6 +88,22 @@ struct SwaptionWalk {
         for (int g = 0; g < kSwaptionGroup; g++) V[g] = fma(E - row[1 + g], Pa, V[g]);
     }
 };
+
+// Brings the tables of the launch into the L2 of each die, the workgroups of a die (consecutive ones lie on
+// different dies) touching a share of the lines each. The tables have just been written, and wavefronts
+// that walk them in step would all wait for each line as it first comes up: 100,000 paths, new tables of
+// 102 KB and 30 swaptions, 265 us against 312 without this and SwaptionWalk::touch.
+__device__ __forceinline__ void touch_tables(ArgPtr a) {
+    const int part = blockIdx.x >> 3, parts = (gridDim.x + 7) >> 3, width = blockDim.x;
+    uint32_t touched = 0;
+    for (int l = part * width + (int)threadIdx.x; l < a->model_lines; l += parts * width)
+        touched |= *(const volatile uint32_t*)((const char*)a->model + 128 * (size_t)l);
+    for (int l = part * width + (int)threadIdx.x; l < a->table_lines; l += parts * width)
+        touched |= *(const volatile uint32_t*)((const char*)a->tables + 128 * (size_t)l);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" :: "v"(touched));
+#endif
+}
 
 // One Euler step of the alive components [first, n), in place. WALK: the walk's swaptions are valued
 // on the states before the step, which also passes over their forwards that are fixed at t_i.
@@ -133,8 +155,12 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
             const double r0 = reciprocal(b0), r1 = reciprocal(b1);
             if constexpr (WALK) {
                 if (sw->periods > 0) {
+                    const uint32_t t2 = sw->touch(j + 2), t3 = sw->touch(j + 3);
                     sw->period(j, E0, R0.e(), r0);
                     sw->period(j + 1, E1, R1.e(), r1);
+#if defined(__HIP_DEVICE_COMPILE__)
+                    asm volatile("" :: "s"(t2), "s"(t3));
+#endif
                 }
             }
             double y0 = x0 + increment((lognormal ? cdt * E0 : cdt) * r0, R0);
