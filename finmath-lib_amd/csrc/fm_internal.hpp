@@ -101,7 +101,7 @@ struct StepArgs {
     const double* times;         // device nT+1
     const int32_t* first_alive;  // device nT
     const int32_t* tenor_time_index; // device n+1: process time index of T_k (rounded up)
-    const void* rec;             // device [nT][n][rec_size_of(fcap_of(F))] records (double or float)
+    const void* rec;             // device [nT][rec_n][rec_size_of(factor capacity)] records (double or float)
     const void *model, *tables;  // FP64 kernels: the model's records and the products' tables, whole, and their
     int model_lines, table_lines;   // sizes in lines of 128 bytes
     int rec_n;                   // records per time step (n, or n rounded up to even for the spot kernels)
@@ -144,11 +144,11 @@ struct StepArgs {
 };
 void launch_lmm_step_fp64(const StepArgs& a, void* stream);
 // Up to this many paths the row kernel (lmm_rows64.hpp) prices and simulates: two of its wavefronts of four paths
-// for each of the 1,024 SIMDs. Both give the same results. Whole calls, row kernel against the other, 40
-// forwards x 5 factors with 20 swaptions and a swap: 357 us against 425 at 2,000 paths, 404 against 424 at
-// 8,000, 534 against 415 at 12,000; 80 x 10: 640 against 1091, 1188 against 1467, 1623 against 1464; 20 x 3: 257
-// against 280, 278 against 278, 299 against 277. It does not write checkpoints, and its table of values is not
-// planned for in caller scratch.
+// for each of the 1,024 SIMDs. Both give the same results. Whole calls when a call took some 150 us more on the
+// host than it does now, row kernel against the other, 40 forwards x 5 factors with 20 swaptions and a swap:
+// 357 us against 425 at 2,000 paths, 404 against 424 at 8,000, 534 against 415 at 12,000; 80 x 10: 640
+// against 1091, 1188 against 1467, 1623 against 1464; 20 x 3: 257 against 280, 278 against 278, 299 against 277.
+// It does not write checkpoints, and its table of values is not planned for in caller scratch.
 constexpr int kRowKernelPaths = 8192;
 void launch_lmm_rows_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_fp32(const StepArgs& a, void* stream);
@@ -187,7 +187,7 @@ void launch_lmm_adjoint_fp32(const StepArgs& a, const AdjArgs& g, void* stream);
 // Deterministic reduction of per-wave partials: out_sum[col], out_m2[col] (Chan merge).
 // Zero count doubles with a kernel (no memset node: safe inside a captured stream).
 void launch_fill_zero(double* p, size_t count, void* stream);
-void launch_reduce_partials(const double* wave_sum, const double* wave_m2, int num_waves, int stride,
+void launch_reduce_partials(double* wave_sum, double* wave_m2, int num_waves, int stride,
                             int num_slots, int num_sums, int P, double* out_sum, double* out_m2, void* stream);
 
 // Column sums of a row-major table [num_rows][stride], first `cols` columns, in a fixed
