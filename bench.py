@@ -11,7 +11,7 @@ The headline line is the plain FP64 form at 40 semiannual forwards x 5 factors x
 1,000,000 paths. Beside it:
   fp32_mixed     the FP32-mixed form at 4,000,000 paths and its per-price difference to
                  the FP64 form on the same paths, in basis points
-  fp64_logstate  FP64 carrying the log-forwards between steps
+  fp64_logstate  the FP64_LOGSTATE precision (the FP64 kernels)
   variants       the general path kernels on the same workload: terminal measure with the
                  predictor-corrector, the displaced local-volatility and the stochastic
                  volatility wrappers (normal state space)
@@ -40,13 +40,13 @@ import numpy as np  # noqa: E402
 
 FP64_PEAK_TFLOPS = 78.6      # MI355X published FP64 peak (vector and matrix)
 HBM_PEAK_GBPS = 8000.0       # MI355X published HBM3E bandwidth
-# HBM bytes per launch of lmm_spot_kernel<5,5,double,true,0> on the 40 x 5 x 1,000,000-path strip:
+# HBM bytes per launch of lmm_spot_kernel<5,5,double,true> on the 40 x 5 x 1,000,000-path strip:
 # FETCH_SIZE and WRITE_SIZE counter passes scaled by a plain 1 GiB copy
 # (profiles/lmm_spot_fp64_c1_hbm_traffic.md)
-PATH_KERNEL_TRAFFIC_BYTES = 2.933e9
+PATH_KERNEL_TRAFFIC_BYTES = 4.691e9
 # VALU-busy fraction of the same kernel from its SQ counter pass: 4 SQ_ACTIVE_INST_VALU over
 # 1,024 SIMDs x GRBM_GUI_ACTIVE / 8 (profiles/lmm_spot_c1_sq_counters.md)
-PATH_KERNEL_VALU_BUSY = 0.673
+PATH_KERNEL_VALU_BUSY = 0.765
 FP32_PEAK_TFLOPS = 157.3     # MI355X published FP32 peak
 
 
@@ -323,7 +323,7 @@ def main():
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": PATH_KERNEL_TRAFFIC_BYTES,
                      "alu": "FP64 vector (MI355X FP64 vector and matrix peaks are both 78.6 TFLOP/s)",
                      "hbm_gbps_at_traffic": PATH_KERNEL_TRAFFIC_BYTES / (step_ms * 1e-3) / 1e9,
-                     "kernel": "lmm_spot_kernel<5,5,double,true,0>", "flops_per_launch": flops,
+                     "kernel": "lmm_spot_kernel<5,5,double,true>", "flops_per_launch": flops,
                      "valu_busy": PATH_KERNEL_VALU_BUSY,
                      "valu_busy_source": "SQ counter pass, profiles/lmm_spot_c1_sq_counters.md"},
     }
