@@ -285,8 +285,6 @@ lmm_general64_kernel(const StepArgs) {
 #pragma unroll
             for (int k = 0; k < FCAP; k++) dW[k] = k < F ? dwp[k] : 0.0;
         }
-        // the next step's line of increments is brought into the L2 while this step runs
-        const uint32_t touch = *(const volatile uint32_t*)(dwp + (ti + 1 < nT ? 2 * F - 1 : F - 1));
         General64 s;
         s.n = n;
         s.first = ConstArray<int32_t>{a->first_alive}[ti];
@@ -307,9 +305,6 @@ lmm_general64_kernel(const StepArgs) {
             sw.periods = pr.num_periods;
         }
         general64_step<NCH, FCAP, TERMINAL, PC, LV, lognormal>(Y, s, dW, ke, &sw);
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("" :: "v"(touch));
-#endif
         if (walk >= 0)
             reduce_walk(products, walk, sw.V, products[walk].num_k == knum ? N : Nprev, active, cnt, lane, wave,
                         a->wave_sum, a->wave_m2, stride);
