@@ -479,17 +479,16 @@ int operands(int op) {
 // the registers whose last use has passed. False where eight do not suffice or a heavy opcode occurs.
 bool compact_program(const RvProg& g, RvCompact& c) {
     struct Value { int kind, input; double constant; int last, slot; };     // kind: 0 input, 1 constant, 2 computed
-    std::vector<Value> vals;
+    Value vals[2 * FM_RV_MAX_INSTRUCTIONS + FM_RV_REGISTERS];   // an instruction makes one, the unwritten registers share one
     struct Step { int op, v[3], out; double imm; };
-    std::vector<Step> steps;
-    vals.reserve(FM_RV_MAX_INSTRUCTIONS + FM_RV_REGISTERS);
-    steps.reserve(FM_RV_MAX_INSTRUCTIONS);
+    Step steps[FM_RV_MAX_INSTRUCTIONS];
+    int nv = 0, ns = 0;
     auto leaf = [&](int kind, int input, double constant) -> int {
-        for (size_t i = 0; i < vals.size(); i++)
+        for (int i = 0; i < nv; i++)
             if (vals[i].kind == kind && (kind == 0 ? vals[i].input == input
-                                                   : std::memcmp(&vals[i].constant, &constant, sizeof(double)) == 0)) return (int)i;
-        vals.push_back({kind, input, constant, -1, -1});
-        return (int)vals.size() - 1;
+                                                   : std::memcmp(&vals[i].constant, &constant, sizeof(double)) == 0)) return i;
+        vals[nv] = {kind, input, constant, -1, -1};
+        return nv++;
     };
     int cur[FM_RV_REGISTERS];
     for (int& r : cur) r = -1;
@@ -505,22 +504,23 @@ bool compact_program(const RvProg& g, RvCompact& c) {
             Step st{in.op, {-1, -1, -1}, 0, in.imm};
             const int m = operands(in.op), reg[3] = {in.a, in.b, in.c};
             for (int i = 0; i < m; i++) st.v[i] = read(reg[i]);
-            vals.push_back({2, 0, 0.0, -1, -1});
-            st.out = cur[in.dst] = (int)vals.size() - 1;
-            steps.push_back(st);
+            vals[nv] = {2, 0, 0.0, -1, -1};
+            st.out = cur[in.dst] = nv++;
+            steps[ns++] = st;
         }
     }
     const int result = read(g.result);
     // last uses, from the end; a step whose value nothing uses has no effect and is dropped
-    vals[(size_t)result].last = (int)steps.size();
-    for (int k = (int)steps.size() - 1; k >= 0; k--) {
-        if (vals[(size_t)steps[(size_t)k].out].last < 0) continue;
-        for (int v : steps[(size_t)k].v)
-            if (v >= 0 && vals[(size_t)v].last < 0) vals[(size_t)v].last = k;
+    vals[result].last = ns;
+    for (int k = ns - 1; k >= 0; k--) {
+        if (vals[steps[k].out].last < 0) continue;
+        for (int v : steps[k].v)
+            if (v >= 0 && vals[v].last < 0) vals[v].last = k;
     }
     std::memset(&c, 0, sizeof(c));
     unsigned used = 0;
-    for (Value& v : vals) {
+    for (int i = 0; i < nv; i++) {
+        Value& v = vals[i];
         if (v.kind == 2 || v.last < 0) continue;
         if (c.nin == kRvCompact) return false;
         v.slot = c.nin;
@@ -528,14 +528,14 @@ bool compact_program(const RvProg& g, RvCompact& c) {
         c.in[c.nin] = v.kind == 0 ? g.in[v.input] : nullptr;
         c.cst[c.nin++] = v.constant;
     }
-    for (int k = 0; k < (int)steps.size(); k++) {
-        const Step& st = steps[(size_t)k];
-        Value& out = vals[(size_t)st.out];
+    for (int k = 0; k < ns; k++) {
+        const Step& st = steps[k];
+        Value& out = vals[st.out];
         if (out.last < 0) continue;
         uint32_t code = (uint32_t)st.op;
         for (int i = 0; i < 3; i++) {
             if (st.v[i] < 0) continue;
-            const Value& v = vals[(size_t)st.v[i]];
+            const Value& v = vals[st.v[i]];
             code |= (uint32_t)v.slot << (12 + 4 * i);
             if (v.last == k) used &= ~(1u << v.slot);
         }
@@ -547,7 +547,7 @@ bool compact_program(const RvProg& g, RvCompact& c) {
         c.code[c.n] = code | (uint32_t)slot << 8;
         c.imm[c.n++] = st.imm;
     }
-    c.result = vals[(size_t)result].slot;
+    c.result = vals[result].slot;
     c.mode = g.mode; c.total = g.total; c.size = g.size; c.prob = g.prob; c.prob_const = g.prob_const;
     return true;
 }
