@@ -14,9 +14,9 @@
 // unit and of the record loads. Where the alive range starts or ends at an odd index, the pair's other
 // forward has a record without loadings, which adds exact zeros to the sums, and keeps its value.
 //
-// The kernel is bound by vector issue: 40 forwards x 5 factors x 4,000,000 paths with 30 swaptions 3.9 ms
-// at 0.99 vector ALU busy (5.53 ms and 0.72 with rolled loops and one record read per component), 80 x 10 x
-// 1,000,000 paths 5.0 ms at 0.85 (7.20 ms, 0.60).
+// The kernel is bound by vector issue: 40 forwards x 5 factors x 4,000,000 paths with 30 swaptions 3.7 ms
+// at 1.0 vector ALU busy (5.53 ms and 0.72 with rolled loops and one record read per component), 80 x 10 x
+// 1,000,000 paths 4.7 ms (7.20 ms, 0.60).
 #pragma once
 
 #include "lmm_chunks.hpp"
