@@ -18,8 +18,9 @@
 // Per path the sweep holds two register arrays, the state at t and the adjoint B. In FP64 and the
 // log-normal state space B_j is the adjoint of ln L_j, into which the step's adjoint of its new state
 // goes unchanged and every sensitivity to L_j enters times L_j: no exponential or division is spent on
-// converting it. In FP32, and in the normal state space, B_j is the adjoint of L_j (the float arithmetic
-// is kept operation by operation, as in lmm_spot32.hpp).
+// converting it. In FP32, in the normal state space, and for the forwards that are fixed when the simulation
+// starts, B_j is the adjoint of L_j: the float arithmetic is kept operation by operation, as in
+// lmm_spot32.hpp, and a forward that no step moves may be zero, where ln L_j has no adjoint.
 // Components are unrolled over the register arrays in pairs, like the pricing pass's steps, except where
 // a component's code is long (reverse_step).
 //
@@ -39,6 +40,10 @@
 #include "lmm_spot64.hpp"
 
 namespace fm {
+
+// The forwards below this are moved by no step: the simulation and the tenor both start at time 0, which is the
+// fixing date of the first forward alone.
+constexpr int kFixedAtStart = 1;
 
 struct AdjKernelArgs {
     StepArgs a;
@@ -195,11 +200,12 @@ __device__ __forceinline__ void reverse_step(Chunks& X, Chunks& B, int n, int re
 // The sensitivities of a swaption group with a walk table in FP64 (SwaptionWalk, lmm_spot64.hpp). With c_g
 // the adjoint of V_g, C = sum_g c_g and G_j = P_j a_j (C E_j - sum_g c_g k_gj),
 //   dV/dE_j = P_j a_j C - r_j sum_{m >= j} G_m,   r_j = 1/(E_j + e_j),
-// in two ascending passes: the values, then the sensitivities. weight(V, c) turns the values into c.
-template <int NCH, int FCAP, bool lognormal, typename Chunks, typename Weight>
+// in two ascending passes: the values, then the sensitivities. weight(V, c) turns the values into c;
+// dB_dE(E, j) is what B_j gets for a sensitivity to E_j.
+template <int NCH, int FCAP, bool lognormal, typename Chunks, typename Weight, typename ToB>
 __device__ __forceinline__ void walk_adjoint64(Chunks& X, Chunks& B, const double* rec, int rec_n, int t,
                                                const double* table, int j0, int periods, const Exp2Coef& ke,
-                                               Weight&& weight) {
+                                               Weight&& weight, ToB&& dB_dE) {
     constexpr int RS = rec_size_of(FCAP);
     RecPtr recs = (RecPtr)(uintptr_t)(rec + (size_t)t * rec_n * RS);
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -245,7 +251,7 @@ __device__ __forceinline__ void walk_adjoint64(Chunks& X, Chunks& B, const doubl
             for (int g = 0; g < kSwaptionGroup; g++) kc = fma(c[g], row[1 + g], kc);
             const double dE = fma(Pa, C, -(r * rest));
             rest = fma(-Pa, fma(C, E, -kc), rest);
-            B.template ch<q>()[j - W * q] = fma(lognormal ? E : 1.0, dE, B.template ch<q>()[j - W * q]);
+            B.template ch<q>()[j - W * q] = fma(dB_dE(E, j), dE, B.template ch<q>()[j - W * q]);
         }
     });
 }
@@ -343,8 +349,10 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                 if constexpr (D && lognormal) return lead[j] * fm_exp2(x, ke);
                 else return x;
             };
-            // a sensitivity to L_j as a part of B_j
-            auto scale = [&](real Lj) -> real { return D && lognormal ? Lj : (real)1; };
+            // a sensitivity to L_j as a part of B_j; 1/s_0 is read here, since a read within the walk spilled 90
+            // scalar registers more (40 x 5 x 100,001 FP64 paths: 1.76 ms a call against 1.72)
+            const double inv_scale0 = D ? lead[n] : 0.0;
+            auto scale = [&](real Lj, int j) -> real { return D && lognormal && j >= kFixedAtStart ? Lj : (real)1; };
 
             // ---- 1. reverse the Euler step t -> t+1
             if (t < nT) {
@@ -391,6 +399,9 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                                         cg[g] = itm ? pg.weight * pg.notional / Nsel : 0.0;
                                         nb += itm ? -pg.weight * v / (Nsel * Nsel) : 0.0;
                                     }
+                                },
+                                [&](double E, int j) -> double {        // L_j = s_j E_j
+                                    return !lognormal ? 1.0 : j >= kFixedAtStart ? E : inv_scale0;
                                 });
                         }
                         qp -= m - 1;
@@ -432,7 +443,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                             U = U + pj * Pc;
                             const real dV = (real)pe.period_length * (real)pr.notional * Pc - ((real)pe.tau * inv) * U;
                             if constexpr (D && lognormal)
-                                B.template ch<q>()[j - W * q] = fma(Vb * Lj, dV, B.template ch<q>()[j - W * q]);
+                                B.template ch<q>()[j - W * q] = fma(Vb * scale(Lj, j), dV, B.template ch<q>()[j - W * q]);
                             else
                                 B.template ch<q>()[j - W * q] = B.template ch<q>()[j - W * q] + (real)Vb * dV;
                             Pc = Pc * (one * (real)pe.inv_adj);      // P_{j-1} = P_j / D_j
@@ -447,7 +458,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                     const bool itm = pr.is_floorlet ? (v < (real)0) : (v >= (real)0);
                     const double dcf = pe.notional;
                     const double x = pr.is_floorlet ? -(double)v * dcf : (double)v * dcf;
-                    xadd = itm ? (real)((pr.is_floorlet ? -dcf : dcf) * pr.weight / Nsel) * scale(Lj) : (real)0;
+                    xadd = itm ? (real)((pr.is_floorlet ? -dcf : dcf) * pr.weight / Nsel) * scale(Lj, pr.first_j) : (real)0;
                     nb = itm ? -pr.weight * x / (Nsel * Nsel) : 0.0;
                 } else if (pr.type == K_BERM_BASIS) {
                     // regression basis: not differentiated (the reference's conditional
@@ -469,7 +480,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                     const real Lj = val(X.get(pr.first_j), pr.first_j);
                     const double sgn = (pr.flags & 1) ? 1.0 : -1.0;
                     const double pay = sgn * (double)(((Lj - (real)pe.strike) * (real)pe.period_length) * (real)pe.notional);
-                    xadd = (real)(pw * sgn * pe.period_length * pe.notional * pr.weight / Nsel) * scale(Lj);
+                    xadd = (real)(pw * sgn * pe.period_length * pe.notional * pr.weight / Nsel) * scale(Lj, pr.first_j);
                     nb = -pw * pr.weight * pay / (Nsel * Nsel);
                 }
                 qp--;
@@ -485,7 +496,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
                 const real Lr = val(X.get(i), i);
                 const double Lk = (double)Lr;
                 const double dk = ConstArray<double>{k->a.delta}[i];
-                B.add(i, (real)(Nb_top * dk * Nk) * scale(Lr));
+                B.add(i, (real)(Nb_top * dk * Nk) * scale(Lr, i));
                 Nb_low += Nb_top * (1.0 + Lk * dk);
                 Nb_top = Nb_low;
                 Nb_low = 0.0;
@@ -541,7 +552,7 @@ lmm_spot_adjoint_kernel(const AdjKernelArgs)
         constexpr int j = decltype(J)::value;
         if (j < n) {
             double b = (double)B.template at<j>();
-            if constexpr (D && lognormal)
+            if constexpr (D && lognormal && j >= kFixedAtStart)
                 b = b / (ConstArray<double>{k->a.lead}[j] * fm_exp2(X.template at<j>(), ke));
             const double s = wave_sum_dpp(active ? b : 0.0);
             if (lane == 63) row[j] = s;
