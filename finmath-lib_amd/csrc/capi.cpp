@@ -299,6 +299,9 @@ void validate_config(const fm_lmm_config* c) {
             "the fused kernel holds at most 80 forward rates and 10 factors");
 }
 
+// Stands for log2(0) in the FP64 kernels' states: a finite number whose power underflows to zero.
+constexpr double kLog2Zero = -1.0e9;
+
 // Rebuild derived host tables and upload the model (on the context stream).
 void prepare_model(fm_lmm* c) {
     require(c->has_L0, FM_ERR_STATE, "initial forwards not set");
@@ -370,10 +373,9 @@ void prepare_model(fm_lmm* c) {
         }
         const double v = c->L0[(size_t)j];
         if (v >= 1e-12 && v <= 1e12) { lead[(size_t)j] = v; lead[(size_t)(n + j)] = 1.0 / v; }
-        // log2(0) is a finite number whose power underflows to zero
-        else z0[(size_t)j] = v > 0.0 ? std::log2(v) : -1.0e9;
+        else z0[(size_t)j] = v > 0.0 ? std::log2(v) : kLog2Zero;
         if (std::isinf(cap)) continue;
-        zcap[(size_t)j] = carried ? cap / lead[(size_t)j] : std::log2(cap / lead[(size_t)j]);
+        zcap[(size_t)j] = carried ? cap / lead[(size_t)j] : std::max(std::log2(cap / lead[(size_t)j]), kLog2Zero);
         if (!carried) z0[(size_t)j] = std::min(z0[(size_t)j], zcap[(size_t)j]);
     }
     for (int i = 0; i < nT; i++)

@@ -39,3 +39,25 @@ def test_gradient_of_a_fixed_forward_at_zero(precision, tol):
         assert np.max(np.abs(eL - dL)) <= tol * np.max(np.abs(dL))
         assert np.max(np.abs(esig - dsig)) <= tol * np.max(np.abs(dsig))
     assert abs(dL[0]) > 0.1 * np.max(np.abs(dL))
+
+
+# ---- a cap at zero: every log-normal forward is zero ------------------------------------------------
+
+@pytest.mark.parametrize("P", [300, 9000])
+@pytest.mark.parametrize("measure,scheme", [("SPOT", "EULER_FUNCTIONAL"), ("SPOT", "PREDICTOR_CORRECTOR_FUNCTIONAL"),
+                                            ("TERMINAL", "EULER_FUNCTIONAL"), ("SPOT", "EULER")])
+@pytest.mark.parametrize("precision", ["FP64", "FP64_LOGSTATE"])
+def test_cap_at_zero(precision, measure, scheme, P):
+    """Every forward and every rate is zero and every numeraire one: a floorlet pays its strike times its daycount
+    fraction on every path, exactly."""
+    say(f"case cap at zero {precision} {measure} {scheme} P={P}")
+    wl = workload(9, 3)
+    t = O.ModelTables(wl)
+    ctx = _abi.LmmContext(t.times, t.tenor, 3, P, wl.seed, precision=precision, measure=measure, scheme=scheme, libor_cap=0.0)
+    ctx.set_initial_forwards(t.L0)
+    ctx.set_covariance(t.lam, t.var)
+    products = [_abi.Product.caplet(T, 0.5, 0.03125, is_floorlet=True) for T in (0.5, 2.0, 4.0)]
+    products += to_products([s for s in wl.products if s["type"] == "swaption" and s["exercise"] > 0])
+    v, e = ctx.value_products(products)
+    assert np.array_equal(v[:3], np.full(3, 0.5 * 0.03125)) and np.array_equal(v[3:], np.zeros(len(v) - 3))
+    assert np.array_equal(e, np.zeros(len(e)))
