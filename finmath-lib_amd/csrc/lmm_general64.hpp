@@ -131,6 +131,8 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
         }
         return zn;
     };
+    const int moved = opaque(first);        // the forwards below are fixed
+    const int special = opaque(WALK && sw->periods > 0 ? n : first);    // pairs below walk or have a fixed forward
     if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
     const unsigned alive = (unsigned)(n - first + 1);
     static_for<0, 4 * NCH>([&](auto Q) {
@@ -143,13 +145,24 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
             V4 l = {0.0, 1.0, 0.0, 1.0};
             if constexpr (LV) l = *(P4)(s.lv + 2 * j);
             __builtin_amdgcn_sched_barrier(0);          // the records are requested before the exponentials
-            const double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
-            const double E0 = value(x0, R0.zcap()), E1 = value(x1, R1.zcap());
-            const double r0 = reciprocal(E0 + R0.e()), r1 = reciprocal(E1 + R1.e());
-            if constexpr (WALK) {
+            double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
+            double E0 = value(x0, R0.zcap()), E1 = value(x1, R1.zcap());
+            double r0 = reciprocal(E0 + R0.e()), r1 = reciprocal(E1 + R1.e());
+            if (WALK && j < special) {
+                asm volatile("");       // a branch, not selects
                 if (sw->periods > 0) {
                     sw->period(j, E0, R0.e(), r0);
                     sw->period(j + 1, E1, R1.e(), r1);
+                }
+                // a fixed forward has no weights: an infinite one times no loading is NaN (under the terminal
+                // measure it comes last)
+                if (j < moved) {
+                    E0 = r0 = 0.0;
+                    if constexpr (PC) x0 = 0.0;
+                    if (j + 1 < moved) {
+                        E1 = r1 = 0.0;
+                        if constexpr (PC) x1 = 0.0;
+                    }
                 }
             }
             double y0, y1;
@@ -165,6 +178,11 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
                 asm volatile("");       // a branch, not selects
                 y0 = jmin(y0, R0.zcap());
                 y1 = jmin(y1, R1.zcap());
+            }
+            if (PC && WALK && j < moved) {
+                asm volatile("");
+                y0 = Y.template at<j>();
+                if (j + 1 < moved) y1 = Y.template at<j + 1>();
             }
             Y.template put<j>(y0);
             Y.template put<j + 1>(y1);

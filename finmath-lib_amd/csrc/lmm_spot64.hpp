@@ -20,7 +20,8 @@
 // and reciprocals are independent, which hides the latency of the FP64 pipeline and of the scalar
 // loads of the two records, and a constant register index needs no indexed moves. A pair holds a
 // fixed or absent forward beside an alive one where the alive range starts or ends at an odd
-// index: its record has no loadings, so it adds an exact zero to every sum and to its state.
+// index: its record has no loadings, and a fixed one has no weight either (it may have overflowed), so it
+// adds an exact zero to every sum and to its state.
 //
 // Swaptions that exercise at t_i over consecutive tenor periods are valued by the same walk
 // (SwaptionWalk): it has E_j and the reciprocal at hand, so a period of a swaption costs two
@@ -134,6 +135,8 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
         for (int k = 0; k < FCAP; k++) inc = fma(T[k], R.lam(k), inc);
         return inc;
     };
+    const int moved = opaque(first);        // the forwards below are fixed
+    const int special = opaque(WALK && sw->periods > 0 ? n : first);    // pairs below walk or have a fixed forward
     if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
     n = opaque(n);
     const unsigned alive = (unsigned)(n - first + 1);
@@ -143,8 +146,8 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
             const RecVec<FCAP> R0(recs, j), R1(recs, j + 1);
             __builtin_amdgcn_sched_barrier(0);          // both records are requested before the exponentials
             const double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
-            const double E0 = lognormal ? fm_exp2(x0, ke) : x0;
-            const double E1 = lognormal ? fm_exp2(x1, ke) : x1;
+            double E0 = lognormal ? fm_exp2(x0, ke) : x0;
+            double E1 = lognormal ? fm_exp2(x1, ke) : x1;
             const double b0 = E0 + R0.e(), b1 = E1 + R1.e();
             // the next pair's records are brought into the scalar cache while this one runs (the table
             // of a model is several times that cache); a pair beyond the last reads its last record
@@ -152,8 +155,9 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
             typedef const volatile uint32_t __attribute__((address_space(4)))* WordPtr;
             constexpr int step = RecVec<FCAP>::size;
             uint32_t t0 = *(WordPtr)(recs + (j + 2) * step), t1 = *(WordPtr)(recs + (j + 3) * step);
-            const double r0 = reciprocal(b0), r1 = reciprocal(b1);
-            if constexpr (WALK) {
+            double r0 = reciprocal(b0), r1 = reciprocal(b1);
+            if (WALK && j < special) {
+                asm volatile("");       // a branch, not selects
                 if (sw->periods > 0) {
                     const uint32_t t2 = sw->touch(j + 2), t3 = sw->touch(j + 3);
                     sw->period(j, E0, R0.e(), r0);
@@ -162,9 +166,19 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
                     asm volatile("" :: "s"(t2), "s"(t3));
 #endif
                 }
+                if (j < moved) {        // no weight: an infinite one times no loading is NaN
+                    E0 = r0 = 0.0;
+                    if (j + 1 < moved) E1 = r1 = 0.0;
+                }
             }
-            double y0 = x0 + increment((lognormal ? cdt * E0 : cdt) * r0, R0);
-            double y1 = x1 + increment((lognormal ? cdt * E1 : cdt) * r1, R1);
+            double w0 = (lognormal ? cdt * E0 : cdt) * r0;
+            const double w1 = (lognormal ? cdt * E1 : cdt) * r1;
+            if (!WALK && j < moved) {
+                asm volatile("");
+                w0 = 0.0;
+            }
+            double y0 = x0 + increment(w0, R0);
+            double y1 = x1 + increment(w1, R1);
             // the cap seldom binds: one comparison each (min(y, cap) keeps NaN, as a comparison does)
             if (__builtin_amdgcn_ballot_w64(y0 > R0.zcap() || y1 > R1.zcap()) != 0) {
                 asm volatile("");       // a branch, not selects

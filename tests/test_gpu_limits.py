@@ -61,3 +61,42 @@ def test_cap_at_zero(precision, measure, scheme, P):
     v, e = ctx.value_products(products)
     assert np.array_equal(v[:3], np.full(3, 0.5 * 0.03125)) and np.array_equal(v[3:], np.zeros(len(v) - 3))
     assert np.array_equal(e, np.zeros(len(e)))
+
+
+# ---- a forward that overflows as it is fixed ---------------------------------------------------------
+
+@pytest.mark.parametrize("P", [300, 9001])
+@pytest.mark.parametrize("precision,scheme", [("FP64", "EULER_FUNCTIONAL"), ("FP32_MIXED", "EULER_FUNCTIONAL"), ("FP64", "EULER")])
+def test_overflow_of_a_fixed_forward(precision, scheme, P):
+    """L_2 starts at 1e6 with a volatility in the step that ends at its fixing, on a factor of its own, that takes its
+    logarithm to the overflow: on about half of the paths it is infinite from then on, and so are the later numeraires.
+    Products on other forwards are worth nothing there and must not become NaN. Bars: those of test_gpu_parity.py
+    (FP64) and 0.1 bp (FP32-mixed)."""
+    say(f"case overflow of a fixed forward {precision} {scheme} P={P}")
+    n = 6
+    wl = workload(n, 2)
+    t = O.ModelTables(wl)
+    t.L0 = t.L0.copy()
+    t.L0[2] = 1.0e6
+    t.vol = np.full_like(t.vol, 0.2)
+    t.vol[:, 2] = 0.0
+    # the drift of the logarithm is sigma^2 dt / 2 at L d >> 1: to ln(1.8e308), or ln(3.4e38), from ln(1e6)
+    t.vol[1, 2] = (4 * ((709.8 if precision == "FP64" else 88.7) - 13.8)) ** 0.5
+    t.factors = np.zeros_like(t.factors)
+    t.factors[:, 0] = 1.0
+    t.factors[2] = [0.0, 1.0]
+    t.lam = t.vol[:, :, None] * t.factors[None]
+    t.var = t.vol * t.vol
+    ctx = _abi.LmmContext(t.times, t.tenor, 2, P, wl.seed, precision=precision, scheme=scheme, libor_cap=np.inf)
+    ctx.set_initial_forwards(t.L0)
+    ctx.set_covariance(t.lam, t.var)
+    v, e = ctx.value_products([_abi.Product.caplet(0.5 * j, 0.5, 0.02) for j in (1, 3, 4, 5)])
+    om = O.OracleModel(t, P, cap=None, with_discount=False, scheme={"EULER": 0, "EULER_FUNCTIONAL": 2}[scheme])
+    over = om.process_value(2, 2) > np.finfo(np.float64 if precision == "FP64" else np.float32).max
+    assert 0.2 < np.mean(over) < 0.8
+    for j, x, y in zip((1, 3, 4, 5), v, e):
+        ov, oe = om.caplet(0.5 * j, 0.5, 0.02)
+        if precision == "FP64":
+            assert x == pytest.approx(ov, rel=1e-10, abs=1e-16) and y == pytest.approx(oe, rel=1e-9, abs=1e-16)
+        else:
+            assert abs(x - ov) < 1e-5 and abs(y - oe) < 1e-5
