@@ -91,13 +91,22 @@ struct Staged {
     std::vector<Piece> pieces;
     size_t total = 0;
     bool pending = false;
+    static size_t piece(size_t n) { return (std::max<size_t>(n, 8) + 255) & ~(size_t)255; }
     void begin() { pieces.clear(); total = 0; }
     // Adds a table, which has to live until send; returns its offset.
     template <class T> size_t add(const std::vector<T>& v) {
         const size_t at = total, bytes = v.size() * sizeof(T);
         pieces.push_back({v.data(), bytes, at});
-        total += (std::max<size_t>(bytes, 8) + 255) & ~(size_t)255;
+        total += piece(bytes);
         return at;
+    }
+    // Memory for a later send of up to `most` bytes.
+    void reserve(hipStream_t s, size_t most) {
+        if (most <= dev.bytes && most <= host.bytes) return;
+        if (pending) HIP_CHECK(hipStreamSynchronize(s));
+        pending = false;
+        (void)dev.get(most);
+        (void)host.get(most);
     }
     char* send(hipStream_t s) {
         if (pending) HIP_CHECK(hipStreamSynchronize(s));
@@ -117,7 +126,7 @@ struct Staged {
 struct ExternalScratch {
     char* base = nullptr;
     size_t bytes = 0, used = 0;
-    static size_t piece(size_t n) { return (std::max<size_t>(n, 8) + 255) & ~(size_t)255; }
+    static size_t piece(size_t n) { return Staged::piece(n); }
     void* take(size_t n) {
         const size_t need = piece(n);
         if (used + need > bytes) throw FmError(FM_ERR_INTERNAL, "scratch carve-up exceeds its checked size");
@@ -196,6 +205,7 @@ struct fm_lmm {
     const void *m_rec = nullptr, *m_lvb = nullptr, *m_walk = nullptr;
     const double *m_L0 = nullptr, *m_Y0 = nullptr, *m_z0 = nullptr, *m_lead = nullptr;
     bool grid_ready = false;            // the tables of times and tenor dates are on the device
+    bool lv_reserved = false;           // the model has been uploaded with a local-volatility table
     DevBuf d_states, d_poly, d_dw, d_row_of, d_paths, d_num;
     DevBuf d_products, d_periods, d_wave_sum, d_wave_m2, d_contrib;
     DevBuf d_ckpt, d_ckpt_first, d_seg, d_adj_num, d_kcur, d_fsig, d_sig, d_cdiag, d_wave_grad, d_grad_out;
@@ -244,6 +254,13 @@ struct fm_lmm {
     // factor capacity of the kernel that runs: the general ones start at three factors
     int fcap() const { return spot64() || spot32() ? fcap_of(F()) : std::max(3, fcap_of(F())); }
     size_t real_size() const { return fp32() ? sizeof(float) : sizeof(double); }
+    // Bytes of the model's tables (prepare_model) under whichever volatility wrappers: the record's size and the
+    // pair table of the FP64 wrappers come and go with them.
+    size_t model_bytes() const {
+        const size_t rows = (size_t)nT() * (size_t)(n() + (n() & 1)), rs = (size_t)rec_size_of(std::max(3, fcap_of(F())));
+        return Staged::piece((rows + 4) * rs * real_size()) + Staged::piece(rows * 2 * sizeof(double)) +
+               2 * Staged::piece((size_t)2 * n() * sizeof(double)) + Staged::piece(80 * sizeof(double));
+    }
     int process_time_index(double t) const { return jsearch(times, round_tick(t)); }
     int libor_index(double t) const { return jsearch(tenor, round_tick(t)); }
 };
@@ -307,6 +324,10 @@ void prepare_model(fm_lmm* c) {
     require(c->has_L0, FM_ERR_STATE, "initial forwards not set");
     require(c->has_cov, FM_ERR_STATE, "covariance tables not set");
     if (!c->tables_dirty) return;
+    // a call without allocation takes any change of the model but a first local-volatility table
+    require(!g_no_alloc || !c->has_lv || c->lv_reserved, FM_ERR_STATE,
+            "the context would have to allocate a local-volatility table: call the allocating entry point once with "
+            "this model first");
     const int n = c->n(), nT = c->nT(), F = c->F();
     hipStream_t s = c->stream;
     std::vector<double> delta((size_t)n);
@@ -439,6 +460,7 @@ void prepare_model(fm_lmm* c) {
     }
     z0.resize(80, 0.0);         // the register array's capacity
     const size_t at_z0 = up.add(z0);
+    if (!g_no_alloc) up.reserve(s, c->model_bytes());
     const char* base = up.send(s);
     c->m_rec = base + at_rec;
     c->m_lvb = base + at_lvb;
@@ -453,6 +475,7 @@ void prepare_model(fm_lmm* c) {
         const double v = c->n0_terminal;
         c->n0_terminal = 1.0 / (c->init_value[(size_t)j] * (delta[(size_t)j] / v) + 1.0 / v);
     }
+    c->lv_reserved = c->lv_reserved || c->has_lv;
     c->tables_dirty = false;
 }
 

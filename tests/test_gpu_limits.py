@@ -100,3 +100,44 @@ def test_overflow_of_a_fixed_forward(precision, scheme, P):
             assert x == pytest.approx(ov, rel=1e-10, abs=1e-16) and y == pytest.approx(oe, rel=1e-9, abs=1e-16)
         else:
             assert abs(x - ov) < 1e-5 and abs(y - oe) < 1e-5
+
+
+# ---- calls without device allocation after a change of the model ------------------------------------
+
+def _sv_driver(t, P):
+    return _abi.LmmContext(t.times, t.tenor, 2, P, 31415)
+
+
+@pytest.mark.parametrize("n,F,precision,state,scheme", [
+    (9, 1, "FP64", "LOGNORMAL", "EULER_FUNCTIONAL"), (9, 3, "FP64", "NORMAL", "EULER_FUNCTIONAL"),
+    (8, 2, "FP64", "LOGNORMAL", "PREDICTOR_CORRECTOR"), (9, 1, "FP32_MIXED", "LOGNORMAL", "EULER_FUNCTIONAL"),
+    (9, 3, "FP32_MIXED", "NORMAL", "EULER_FUNCTIONAL"), (7, 1, "FP64_LOGSTATE", "LOGNORMAL", "EULER_FUNCTIONAL")])
+@pytest.mark.parametrize("first", ["plain", "scaled"])
+def test_noalloc_after_a_stochastic_volatility_comes_or_goes(n, F, precision, state, scheme, first):
+    """A stochastic volatility scaling brings no table of its own, so a call without allocation goes on working after
+    it is set or removed, whichever model the context was first priced with; values and errors are those of the
+    allocating call, bit for bit. A first local-volatility table is still refused."""
+    say(f"case noalloc after a change n={n} F={F} {precision} {state} {scheme} {first}")
+    P = 500
+    wl = workload(n, F)
+    t = O.ModelTables(wl, vol_params=(0.2, 0.0, 0.25, 0.1) if state == "LOGNORMAL" else (0.01, 0.0, 0.25, 0.004))
+    ctx = _abi.LmmContext(t.times, t.tenor, F, P, wl.seed, precision=precision, state_space=state, scheme=scheme)
+    ctx.set_initial_forwards(t.L0)
+    ctx.set_covariance(t.lam, t.var)
+    ctx.set_discount_curve(t.pd)
+    products = to_products([s for s in wl.products if s["type"] == "swaption"])
+    driver = _sv_driver(t, P)
+    order = [False, True, False] if first == "plain" else [True, False, True]
+    for i, scaled in enumerate(order):
+        ctx.set_stochastic_volatility(0.3, -0.3, driver if scaled else None)
+        if i == 0:
+            ctx.value_products(products)
+        v, e = ctx.value_products_noalloc(products)
+        w, f = ctx.value_products(products)
+        assert np.array_equal(v, w) and np.array_equal(e, f)
+    ctx.set_local_volatility(0.5, 0.5 * t.L0[None, :] + 0.0 * t.vol)
+    with pytest.raises(_abi.IllegalStateException):
+        ctx.value_products_noalloc(products)
+    w, f = ctx.value_products(products)
+    v, e = ctx.value_products_noalloc(products)
+    assert np.array_equal(v, w) and np.array_equal(e, f)
