@@ -727,7 +727,6 @@ Lowered lower_products(fm_lmm* c, const fm_product* prods, int count) {
             k.first_j = j0;
             k.num_periods = p.num_periods;
             k.notional = p.notional;
-            k.exercise = Te;
             k.param_off = (int32_t)L.per.size() - p.num_periods;
             k.num_k = numeraire_index(Te);
             check_available(k.eval_index, k.num_k);
@@ -1072,7 +1071,6 @@ size_t external_scratch_bytes(const fm_lmm* c, const Lowered& L) {
     const size_t num_waves = ((size_t)c->P() + 63) / 64, stride = (size_t)L.num_slots + c->n() + 1;
     return 2 * ExternalScratch::piece(num_waves * stride * sizeof(double)) +
            ExternalScratch::piece(L.kp.size() * sizeof(KProduct)) + ExternalScratch::piece(L.per.size() * sizeof(KPeriod)) +
-           ExternalScratch::piece(L.walk.size() * sizeof(double)) + ExternalScratch::piece(L.walk32.size() * sizeof(float)) +
            ExternalScratch::piece(stride * 2 * sizeof(double));
 }
 
@@ -1582,7 +1580,7 @@ int fm_lmm_get_brownian_increment(fm_lmm* c, int32_t t, int32_t k, double* out) 
 }
 
 int fm_lmm_value_products(fm_lmm* c, const fm_product* products, int32_t count, double* values, double* errors) {
-    return fm::value_products_in(c, products, count, values, errors, nullptr, 0);
+    return fm::value_products_in(c, products, count, values, errors, nullptr, 0, 0);
 }
 
 } // extern "C"
@@ -1592,7 +1590,7 @@ namespace fm {
 int context_device(const fm_lmm* c) { return c->device; }
 
 int value_products_in(fm_lmm* c, const fm_product* products, int32_t count, double* values, double* errors,
-                      void* scratch, size_t scratch_bytes) {
+                      void* scratch, size_t scratch_bytes, size_t walk_bytes) {
     FM_TRY
     require(c != nullptr, FM_ERR_INVALID_ARGUMENT, "NULL context");
     require(count >= 0, FM_ERR_INVALID_ARGUMENT, "negative product count");
@@ -1612,8 +1610,14 @@ int value_products_in(fm_lmm* c, const fm_product* products, int32_t count, doub
         require(need <= scratch_bytes, FM_ERR_INVALID_ARGUMENT,
                 "the pass needs " + std::to_string(need) + " bytes of scratch, more than the " +
                 std::to_string(scratch_bytes) + " bytes of the no-allocation entry point (fewer paths or products)");
+        // the walk tables lie beside the counted pieces; swaptions whose tables do not fit take a walk of their own
+        if (ExternalScratch::piece(L.walk.size() * sizeof(double) + L.walk32.size() * sizeof(float)) > walk_bytes) {
+            for (KProduct& k : L.kp) k.walk = -1;
+            L.walk.clear();
+            L.walk32.clear();
+        }
         xs.base = (char*)scratch;
-        xs.bytes = scratch_bytes;
+        xs.bytes = scratch_bytes + walk_bytes;
     }
     std::vector<double> sums, m2s;
     run_pass(c, L, false, sums, m2s, nullptr, 1, nullptr, scratch ? &xs : nullptr);

@@ -73,7 +73,6 @@ struct KProduct {
     int32_t flags;        // bit0: pay fix (swap)
     int32_t num_k;        // tenor index of the numeraire the payoff is divided by
     double  notional;
-    double  exercise;
     double  weight;       // adjoint: objective weight of this (lowered) product per path
     int32_t param_off;    // offset into the per-period parameter table
     int32_t pad2;         // swaption: number of following swaptions valued with it (pricing);
@@ -301,9 +300,10 @@ fm_rv* rv_scale_numeraire(fm_rv* x, double zb, double adj, bool scalar_form);
 // ---- entry points over caller scratch (capi.cpp) -------------------------------------------
 int context_device(const fm_lmm* c);
 // fm_lmm_value_products; with scratch != NULL the per-call device buffers (wave partials, product
-// tables, reduction output) are taken from [scratch, scratch + scratch_bytes) and no context
-// buffer may grow (FM_ERR_STATE), so the call allocates no device memory.
+// tables, reduction output) are taken from [scratch, scratch + scratch_bytes) and the swaptions' walk tables
+// from the walk_bytes after it, and no context buffer may grow (FM_ERR_STATE), so the call allocates no device
+// memory. Without walk tables the values are the same up to rounding.
 int value_products_in(fm_lmm* c, const fm_product* products, int32_t count, double* values, double* errors,
-                      void* scratch, size_t scratch_bytes);
+                      void* scratch, size_t scratch_bytes, size_t walk_bytes);
 
 } // namespace fm

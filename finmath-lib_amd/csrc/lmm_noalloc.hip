@@ -16,9 +16,12 @@ namespace {
 // Maximum scratch of one call: 2 x 8 B x (products + forwards + 1) per 64 paths of partials
 // plus the tables. The 30-swaption strip on 40 forwards fits up to about 3.7M paths.
 constexpr size_t kScratchBytes = (size_t)64 << 20;
+// and the walk tables of swaption groups, which are derived from the tables counted above: at most 80 groups of
+// 80 rows of 64 bytes in FP64, 32 bytes for each period of a group in FP32.
+constexpr size_t kWalkBytes = (size_t)8 << 20;
 
 // Every GPU the library runs on holds its own copy of this array until the process ends.
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kWalkBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_table_mu;
@@ -61,7 +64,8 @@ extern "C" int fm_lmm_value_products_noalloc(fm_lmm* ctx, const fm_product* prod
         const int dev = fm::context_device(ctx);
         void* ptr = scratch_address(dev);
         std::lock_guard<std::mutex> lk(g_call_mu[dev]);
-        return fm::value_products_in(ctx, products, count, values, errors, ptr, kScratchBytes);
+        return fm::value_products_in(ctx, products, count, values, errors, ptr, kScratchBytes,
+                                     kWalkBytes);
     } catch (const fm::FmError& e) {
         fm::set_last_error(e.what());
         return e.code;

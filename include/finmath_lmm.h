@@ -259,9 +259,11 @@ int fm_lmm_value_products(fm_lmm* ctx, const fm_product* products, int32_t count
 /* fm_lmm_value_products without device allocation. No counterpart in the reference: it is
  * for callers that cannot allocate device memory (tight pricing loops, harnesses that forbid
  * hipMalloc). Same inputs, outputs and results as fm_lmm_value_products. The per-call device
- * buffers (wave partials, product tables, reduction output) come from a 64 MiB array that
- * every GPU holds from the library's first use until the process ends; a pass needing more
- * (about 16 B x (products + forwards + 1) per 64 paths) fails with FM_ERR_INVALID_ARGUMENT.
+ * buffers (wave partials, product tables, reduction output) come from an array that every GPU
+ * holds from the library's first use until the process ends: 64 MiB, and 8 MiB for tables derived
+ * from the products; a pass needing more than the 64 MiB (about 16 B x (products + forwards + 1)
+ * per 64 paths) fails with FM_ERR_INVALID_ARGUMENT, one whose derived tables need more than the
+ * 8 MiB (more than 260,000 swaption periods in FP32_MIXED) values them without, equal up to rounding.
  * Only single-date products (swaptions, caplets): swaps and Bermudans need per-path columns
  * (FM_ERR_UNSUPPORTED). The context's own buffers (model tables, generator states, Brownian
  * increments) must already have their size: call fm_lmm_value_products once on the context

@@ -141,3 +141,45 @@ def test_noalloc_after_a_stochastic_volatility_comes_or_goes(n, F, precision, st
     w, f = ctx.value_products(products)
     v, e = ctx.value_products_noalloc(products)
     assert np.array_equal(v, w) and np.array_equal(e, f)
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32_MIXED"])
+def test_noalloc_up_to_its_documented_scratch(precision):
+    """Two partials of 8 bytes per slot, forward and 64 paths, a product table of 64 bytes and periods of 56 bytes (every
+    swaption of a group has a second copy of its own), the averages, all rounded up to 256 bytes: what fits 64 MiB
+    by that count is valued."""
+    n, strikes = 10, np.linspace(0.01, 0.06, 40)
+    wl = workload(n, 1, strikes=strikes)
+    specs = [s for s in wl.products if s["type"] == "swaption"]
+    t = O.ModelTables(wl)
+    def up(b):
+        return (b + 255) // 256 * 256
+    m = len(specs)
+    columns = m + n + 1
+    periods = sum(len(s["fixing"]) for s in specs)
+    fixed = up(64 * m) + up(56 * 2 * periods) + up(16 * columns)
+    waves = ((64 << 20) - fixed) // 2 // 256 * 256 // (8 * columns)
+    assert 2 * up(waves * columns * 8) + fixed <= 64 << 20
+    P = waves * 64
+    say(f"case noalloc at its limit {precision} P={P} products={m}")
+    ctx = make_context(wl, t, P, precision=precision)
+    w, f = ctx.value_products(to_products(specs))
+    v, e = ctx.value_products_noalloc(to_products(specs))
+    assert np.array_equal(v, w) and np.array_equal(e, f)
+
+
+def test_noalloc_beyond_its_derived_tables():
+    """3,400 swaptions of 79 periods that share no walk need 8.6 MB of FP32 walk tables; without them each is valued by
+    a walk over its periods, as one whose group has none. Bar: that of FP32-mixed prices, 0.1 bp."""
+    say("case noalloc beyond its derived tables")
+    n, m = 80, 3400
+    wl = workload(n, 1)
+    t = O.ModelTables(wl)
+    fix, pay = t.tenor[1:n], t.tenor[2:n + 1]
+    products = [_abi.Product.swaption(fix[0], fix, pay, np.full(n - 1, 0.03), period_lengths=(pay - fix) * (1 + 1e-6 * i))
+                for i in range(m)]
+    ctx = make_context(wl, t, 100, precision="FP32_MIXED")
+    w, f = ctx.value_products(products)
+    v, e = ctx.value_products_noalloc(products)
+    assert np.max(np.abs(v - w)) < 1e-5 and np.max(np.abs(e - f)) < 1e-5
+    assert np.all(np.isfinite(w)) and np.min(w) > 1e-4
