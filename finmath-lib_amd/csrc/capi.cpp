@@ -1175,8 +1175,9 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
     } else {
         a.Y0 = c->m_z0;
         a.lead = c->m_lead;
-        if (c->spot64() && !ckpt && !xs && P <= kRowKernelPaths) {
-            a.values = (double*)c->d_values.get((size_t)(L.num_slots + n + 1) * P * sizeof(double));
+        const size_t value_bytes = (size_t)(L.num_slots + n + 1) * P * sizeof(double);
+        if (c->spot64() && !ckpt && !xs && P <= kRowKernelPaths && value_bytes <= kRowKernelBytes) {
+            a.values = (double*)c->d_values.get(value_bytes);
             launch_lmm_rows_fp64(a, s);
         } else if (c->spot64()) launch_lmm_step_fp64(a, s);
         else if (c->wrapped()) launch_lmm_step_lv_fp64(a, s);

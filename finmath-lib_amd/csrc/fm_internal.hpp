@@ -149,6 +149,9 @@ void launch_lmm_step_fp64(const StepArgs& a, void* stream);
 // against 1091, 1188 against 1467, 1623 against 1464; 20 x 3: 257 against 280, 278 against 278, 299 against 277.
 // It does not write checkpoints, and its table of values is not planned for in caller scratch.
 constexpr int kRowKernelPaths = 8192;
+// Its table of values is 32 times the partials' size and stays with the context, so it is bounded: 4,096 products
+// at 8,192 paths.
+constexpr size_t kRowKernelBytes = (size_t)256 << 20;
 void launch_lmm_rows_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_fp32(const StepArgs& a, void* stream);
 // General variant (terminal measure, carried state, predictor-corrector), see lmm_step.hpp.

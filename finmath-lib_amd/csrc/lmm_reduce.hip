@@ -75,8 +75,9 @@ gather_partials_kernel(double* __restrict__ wave_sum, double* __restrict__ wave_
                        int num_slots, int cols, int P)
 {
     __shared__ Acc sh[kReduceThreads];
-    const int col = blockIdx.x * 32 + (threadIdx.x & 31), lane = threadIdx.x >> 5;
-    const int r0 = blockIdx.y * kGatherRows, r1 = min(num_waves, r0 + kGatherRows);
+    const int tiles = (cols + 31) / 32, tile = blockIdx.x % tiles;
+    const int col = tile * 32 + (threadIdx.x & 31), lane = threadIdx.x >> 5;
+    const int r0 = (int)(blockIdx.x / tiles) * kGatherRows, r1 = min(num_waves, r0 + kGatherRows);
     const bool has_m2 = col < num_slots;
     Acc a{0.0, 0.0, 0.0, 0.0};
     if (col < cols) {
@@ -204,7 +205,8 @@ void launch_reduce_partials(double* wave_sum, double* wave_m2, int num_waves, in
     if (num_waves > 8 * kReduceThreads) {
         step = kGatherRows;
         rows = (num_waves + step - 1) / step;
-        hipLaunchKernelGGL(gather_partials_kernel, dim3((unsigned)((cols + 31) / 32), (unsigned)rows), dim3(kReduceThreads), 0,
+        // one grid dimension: the others end at 65,536, 537 million paths; a workgroup stands for 64 KB of partials
+        hipLaunchKernelGGL(gather_partials_kernel, dim3((unsigned)((cols + 31) / 32) * (unsigned)rows), dim3(kReduceThreads), 0,
                            (hipStream_t)stream, wave_sum, wave_m2, num_waves, stride, num_slots, cols, P);
         HIP_CHECK(hipGetLastError());
     }

@@ -234,19 +234,18 @@ __global__ void __launch_bounds__(64) lmm_rows64_kernel(const StepArgs) {
     }
 }
 
-// Partials of 64 paths per wavefront from the table of values: a block row per product (a swaption group at
-// its first member) and one per numeraire.
-static __global__ void __launch_bounds__(kStepThreads) rows64_partials_kernel(const StepArgs a) {
+// Partials of 64 paths per wavefront from the table of values: of product i (a swaption group's at its first
+// member) or, beyond the products, of a numeraire, for the paths of block b.
+__device__ __forceinline__ void rows64_partials(const StepArgs& a, int i, int b) {
     const int lane = threadIdx.x & 63;
-    const int64_t p = (int64_t)blockIdx.x * kStepThreads + threadIdx.x;
-    const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p = (int64_t)b * kStepThreads + threadIdx.x;
+    const int64_t wave = (int64_t)b * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t left = (int64_t)a.P - wave * 64;
     if (left <= 0) return;
     const bool active = p < a.P;
     const int64_t pc = active ? p : (int64_t)a.P - 1;
     const int cnt = left > 64 ? 64 : (int)left;
     const int stride = a.num_slots + a.n + 1;
-    const int i = blockIdx.y;
     if (i >= a.num_products) {
         const int k = i - a.num_products, col = a.num_slots + 1 + k;
         if (a.tenor_time_index[k] > a.nT) return;       // beyond the simulation: no such numeraire
@@ -270,6 +269,13 @@ static __global__ void __launch_bounds__(kStepThreads) rows64_partials_kernel(co
         reduce_slot(a.values[(size_t)pr.out_slot * a.P + pc], active, cnt, lane, wave, a.wave_sum, a.wave_m2, stride,
                     pr.out_slot);
     }
+}
+
+static __global__ void __launch_bounds__(kStepThreads) rows64_partials_kernel(const StepArgs a) {
+    const int blocks = (int)(((int64_t)a.P + kStepThreads - 1) / kStepThreads);
+    const int64_t items = (int64_t)(a.num_products + a.n) * blocks;
+    for (int64_t k = blockIdx.x; k < items; k += gridDim.x)         // uniform over the workgroup
+        rows64_partials(a, (int)(k / blocks), (int)(k % blocks));
 }
 
 template <int R, int FCAP>

@@ -183,3 +183,45 @@ def test_noalloc_beyond_its_derived_tables():
     v, e = ctx.value_products_noalloc(products)
     assert np.max(np.abs(v - w)) < 1e-5 and np.max(np.abs(e - f)) < 1e-5
     assert np.all(np.isfinite(w)) and np.min(w) > 1e-4
+
+
+# ---- grid dimensions --------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("count,P", [(66_000, 64), (4_000, 8192), (4_200, 8192), (70_000, 200)])
+def test_many_products_on_few_paths(count, P):
+    """More lowered products than 65,536, and tables of values on both sides of the size up to which the kernel for few
+    paths runs: values and errors are those of the kernel for many paths, bit for bit."""
+    say(f"case many products {count} P={P}")
+    wl = workload(4, 2)
+    t = O.ModelTables(wl)
+    ctx = make_context(wl, t, P)
+    products = [_abi.Product.caplet(0.5 * (i % 4), 0.5, 0.01 + 1e-7 * i) for i in range(count)]
+    v, e = ctx.value_products(products)
+    w, f = ctx.value_products_noalloc(products)
+    assert np.array_equal(v, w) and np.array_equal(e, f)
+
+
+def test_swaps_of_many_periods_on_few_paths():
+    """66,000 periods of 16,500 swaps: each is worth the same swap's alone."""
+    say("case many swap periods")
+    wl = workload(4, 2)
+    t = O.ModelTables(wl)
+    ctx = make_context(wl, t, 70)
+    products = to_products([wl.products[-1]])
+    v, e = ctx.value_products(products)
+    w, f = ctx.value_products(products * 16_500)
+    assert np.array_equal(w, np.full(16_500, v[0])) and np.array_equal(f, np.full(16_500, e[0]))
+
+
+def test_more_partials_than_a_grid_dimension():
+    """8,388,610 wavefronts, 65,537 groups of them: every path of a forward fixed at time 0 pays the same, so the average
+    is that payoff over 1 + L d, exactly (a sum of 2^29 + 130 equal numbers rounds once), and its error is rounding."""
+    P = (1 << 29) + 130
+    say(f"case partials beyond a grid dimension P={P}")
+    ctx = _abi.LmmContext([0.0, 0.5], [0.0, 0.5], 1, P, 3141, precision="FP32_MIXED")
+    ctx.set_initial_forwards([0.25])
+    ctx.set_covariance(np.full((1, 1, 1), 0.2), np.full((1, 1), 0.04))
+    v, e = ctx.value_products([_abi.Product.caplet(0.0, 0.5, 0.125)])
+    assert v[0] == pytest.approx(0.5 * 0.125 / 1.125, rel=4e-16)
+    assert e[0] < 1e-15
+    ctx.close()
