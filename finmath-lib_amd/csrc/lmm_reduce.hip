@@ -36,18 +36,22 @@ __device__ __forceinline__ void merge(Acc& a, const Acc& b) {
     a.n = nn;
 }
 
+// The partials of every merge_rows-th row: of one wavefront (merge_rows = 1), or of merge_rows of them merged by
+// gather_partials_kernel, with their sum's compensation in the row that follows (if they are more than one).
 __global__ void __launch_bounds__(kReduceThreads)
 reduce_partials_kernel(const double* __restrict__ wave_sum, const double* __restrict__ wave_m2,
-                       int num_rows, int row_paths, int64_t stride, int num_slots, int P,
+                       int num_waves, int merge_rows, int64_t stride, int num_slots, int P,
                        double* __restrict__ out_sum, double* __restrict__ out_m2)
 {
     __shared__ Acc sh[kReduceThreads];
     const int col = blockIdx.x;
     const bool has_m2 = col < num_slots;
+    const int row_paths = 64 * merge_rows;
     Acc a{0.0, 0.0, 0.0, 0.0};
-    for (int w = threadIdx.x; w < num_rows; w += kReduceThreads) {
-        const int64_t left = (int64_t)P - (int64_t)w * row_paths;
-        Acc b{(double)(left > row_paths ? row_paths : left), wave_sum[w * stride + col], 0.0,
+    for (int w = threadIdx.x * merge_rows; w < num_waves; w += kReduceThreads * merge_rows) {
+        const int64_t left = (int64_t)P - (int64_t)w * 64;
+        Acc b{(double)(left > row_paths ? row_paths : left), wave_sum[w * stride + col],
+              merge_rows > 1 && w + 1 < num_waves ? wave_sum[(w + 1) * stride + col] : 0.0,
               has_m2 ? wave_m2[w * stride + col] : 0.0};
         merge(a, b);
     }
@@ -63,11 +67,11 @@ reduce_partials_kernel(const double* __restrict__ wave_sum, const double* __rest
     }
 }
 
-// Merges kGatherRows rows of partials into the first of them, in place: 32 adjacent columns by 8 rows at a time
-// per workgroup. A column's partials are 8 bytes of a line each, so a workgroup per column alone reads
-// every line once per column, and its compute unit's path to the L2 is the bound: 4,000,000 paths, 71
-// columns: 217 us, 30 with the rows merged first; 1,000,000 paths 61 us, 20 with. A workgroup reads and writes
-// only its own rows and columns, and writes after all of it has read.
+// Merges kGatherRows rows of partials into the first of them (the sum's compensation into the second), in place:
+// 32 adjacent columns by 8 rows at a time per workgroup. A column's partials are 8 bytes of a line each, so a
+// workgroup per column alone reads every line once per column, and its compute unit's path to the L2 is the
+// bound: 4,000,000 paths, 71 columns: 217 us, 30 with the rows merged first; 1,000,000 paths 61 us, 20 with.
+// A workgroup reads and writes only its own rows and columns, and writes after all of it has read.
 constexpr int kGatherRows = 128;
 
 __global__ void __launch_bounds__(kReduceThreads)
@@ -95,7 +99,8 @@ gather_partials_kernel(double* __restrict__ wave_sum, double* __restrict__ wave_
         __syncthreads();
     }
     if (lane == 0 && col < cols) {
-        wave_sum[(size_t)r0 * stride + col] = sh[threadIdx.x].s + sh[threadIdx.x].c;
+        wave_sum[(size_t)r0 * stride + col] = sh[threadIdx.x].s;
+        if (r0 + 1 < r1) wave_sum[(size_t)(r0 + 1) * stride + col] = sh[threadIdx.x].c;
         if (has_m2) wave_m2[(size_t)r0 * stride + col] = sh[threadIdx.x].m2;
     }
 }
@@ -200,18 +205,18 @@ void launch_reduce_partials(double* wave_sum, double* wave_m2, int num_waves, in
                             int P, double* out_sum, double* out_m2, void* stream) {
     const int cols = num_slots + num_sums;
     if (cols <= 0) return;
-    int rows = num_waves, step = 1;
+    int merge_rows = 1;
     // worth a launch of its own where a thread of the column's workgroup would merge more than eight rows
     if (num_waves > 8 * kReduceThreads) {
-        step = kGatherRows;
-        rows = (num_waves + step - 1) / step;
+        merge_rows = kGatherRows;
+        const int rows = (num_waves + merge_rows - 1) / merge_rows;
         // one grid dimension: the others end at 65,536, 537 million paths; a workgroup stands for 64 KB of partials
         hipLaunchKernelGGL(gather_partials_kernel, dim3((unsigned)((cols + 31) / 32) * (unsigned)rows), dim3(kReduceThreads), 0,
                            (hipStream_t)stream, wave_sum, wave_m2, num_waves, stride, num_slots, cols, P);
         HIP_CHECK(hipGetLastError());
     }
     hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)cols), dim3(kReduceThreads), 0, (hipStream_t)stream,
-                       wave_sum, wave_m2, rows, 64 * step, (int64_t)stride * step, num_slots, P, out_sum, out_m2);
+                       wave_sum, wave_m2, num_waves, merge_rows, (int64_t)stride, num_slots, P, out_sum, out_m2);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -7,6 +7,7 @@ import pytest
 
 import _oracle as O
 from finmath_hip import _abi
+from finmath_hip.randomvariable import RandomVariable
 from test_gpu_aad_oracle import gpu_context, swaptions
 from test_gpu_parity import make_context, say, to_products
 from test_gpu_spot64 import workload
@@ -225,3 +226,39 @@ def test_more_partials_than_a_grid_dimension():
     assert v[0] == pytest.approx(0.5 * 0.125 / 1.125, rel=4e-16)
     assert e[0] < 1e-15
     ctx.close()
+
+
+# ---- reductions -------------------------------------------------------------------------------------
+
+def test_merged_partials_keep_their_compensation():
+    """Partials whose sum needs more than 53 bits, in rows that are merged 128 at a time first: the compensation of a merged
+    row counts like its sum. Every column holds 2^53 in its first row, -2^53 in a row of another group and ones in
+    between, so its sum is the number of ones, exactly."""
+    say("case compensated merge of partials")
+    lib = _abi.load()
+    launch = lib._ZN2fm22launch_reduce_partialsEPdS0_iiiiiS0_S0_Pv
+    launch.restype = None
+    p, i = ctypes.c_void_p, ctypes.c_int
+    launch.argtypes = [p, p, i, i, i, i, i, p, p, p]
+
+    def pointer(rv):
+        out = ctypes.c_void_p()
+        _abi.check(lib.fm_rv_device_ptr(ctypes.c_void_p(rv.devicePointer()), ctypes.byref(out)))
+        return out
+
+    for rows, slots, sums in ((2049, 3, 2), (2049, 32, 0), (2176, 31, 2), (4100, 64, 5), (2050, 60, 41)):
+        say(f"  rows={rows} slots={slots} sums={sums}")
+        cols = slots + sums
+        part = np.ones((rows, cols))
+        part[0] = 2.0 ** 53
+        part[rows - 1] = -2.0 ** 53
+        P = rows * 64 - 7
+        count = np.full(rows, 64.0)
+        count[-1] = 57.0
+        exact = float(rows + np.sum(count * (part[:, 0] / count - (rows - 2) / P) ** 2))
+        d_part, d_m2, d_sum, d_var = (RandomVariable.from_array(x) for x in (part.ravel(), np.ones(rows * cols), np.zeros(cols + 2),
+                                                                             np.zeros(cols + 2)))
+        launch(pointer(d_part), pointer(d_m2), rows, cols, slots, sums, P, pointer(d_sum), pointer(d_var), None)
+        lib.hipDeviceSynchronize()      # the launch is on the null stream, which the copies below do not wait for
+        assert np.array_equal(d_sum.getRealizations()[:cols], np.full(cols, rows - 2.0))
+        assert np.allclose(d_var.getRealizations()[:slots], exact, rtol=1e-12, atol=0)
