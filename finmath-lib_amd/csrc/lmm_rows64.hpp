@@ -235,11 +235,11 @@ __global__ void __launch_bounds__(64) lmm_rows64_kernel(const StepArgs) {
 }
 
 // Partials of 64 paths per wavefront from the table of values: of product i (a swaption group's at its first
-// member) or, beyond the products, of a numeraire, for the paths of block b.
-__device__ __forceinline__ void rows64_partials(const StepArgs& a, int i, int b) {
+// member) or, beyond the products, of a numeraire.
+__device__ __forceinline__ void rows64_partials(const StepArgs& a, int i) {
     const int lane = threadIdx.x & 63;
-    const int64_t p = (int64_t)b * kStepThreads + threadIdx.x;
-    const int64_t wave = (int64_t)b * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p = (int64_t)blockIdx.x * kStepThreads + threadIdx.x;
+    const int64_t wave = (int64_t)blockIdx.x * (kStepThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t left = (int64_t)a.P - wave * 64;
     if (left <= 0) return;
     const bool active = p < a.P;
@@ -272,10 +272,7 @@ __device__ __forceinline__ void rows64_partials(const StepArgs& a, int i, int b)
 }
 
 static __global__ void __launch_bounds__(kStepThreads) rows64_partials_kernel(const StepArgs a) {
-    const int blocks = (int)(((int64_t)a.P + kStepThreads - 1) / kStepThreads);
-    const int64_t items = (int64_t)(a.num_products + a.n) * blocks;
-    for (int64_t k = blockIdx.x; k < items; k += gridDim.x)         // uniform over the workgroup
-        rows64_partials(a, (int)(k / blocks), (int)(k % blocks));
+    for (int64_t i = blockIdx.y; i < (int64_t)a.num_products + a.n; i += gridDim.y) rows64_partials(a, (int)i);
 }
 
 template <int R, int FCAP>

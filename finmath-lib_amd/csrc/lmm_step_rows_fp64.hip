@@ -13,10 +13,10 @@ void launch_lmm_rows_fp64(const StepArgs& a, void* stream) {
     else if (a.n <= 48) launch_rows64_n<3>(a, s);
     else if (a.n <= 80) launch_rows64_n<5>(a, s);
     else throw FmError(FM_ERR_UNSUPPORTED, "more than 80 forward rates are not supported by the path kernel");
-    // products and numeraires by blocks of paths, in one grid dimension and rounds of at most a million: a swap is
-    // one product per period, so there may be more than the 65,536 of the other dimensions
-    const int64_t items = (((int64_t)a.P + kStepThreads - 1) / kStepThreads) * ((int64_t)a.num_products + a.n);
-    const dim3 grid((unsigned)std::min<int64_t>(items, 1 << 20));
+    // blocks of paths by products and numeraires; a swap is one product per period, so there may be more of them
+    // than the grid's second dimension holds
+    const dim3 grid((unsigned)(((int64_t)a.P + kStepThreads - 1) / kStepThreads),
+                    (unsigned)std::min<int64_t>((int64_t)a.num_products + a.n, 65535));
     hipLaunchKernelGGL(rows64_partials_kernel, grid, dim3(kStepThreads), 0, s, a);
     HIP_CHECK(hipGetLastError());
 }
