@@ -356,8 +356,9 @@ const char* fm_last_error(void);
 
 /* Per-stage device time of the last fm_lmm_value_products / fm_lmm_simulate /
  * fm_lmm_adjoint call, measured with HIP events on the context's stream:
- * ms[0] generator, ms[1] path step, ms[2] reductions, ms[3] adjoint sweep,
- * ms[4] whole call. */
+ * ms[0] generator, ms[1] path step with the clearing of its partials, ms[2] reductions,
+ * ms[3] adjoint sweep, ms[4] whole call from the upload of its product tables on, where they are
+ * 1 MiB or more, and from the first stage on, where they are smaller. */
 int fm_lmm_last_timings(fm_lmm* ctx, double* ms, int32_t count);
 
 /* Library version string and the device it runs on. */

@@ -262,3 +262,19 @@ def test_merged_partials_keep_their_compensation():
         lib.hipDeviceSynchronize()      # the launch is on the null stream, which the copies below do not wait for
         assert np.array_equal(d_sum.getRealizations()[:cols], np.full(cols, rows - 2.0))
         assert np.allclose(d_var.getRealizations()[:slots], exact, rtol=1e-12, atol=0)
+
+
+# ---- timings ----------------------------------------------------------------------------------------
+
+def test_the_whole_call_includes_its_product_tables():
+    """30,000 caplets are 4 MB of tables: at the 64 GB/s of the host link they take 60 us, which belong to the whole call and
+    to none of its stages."""
+    say("case timings with large product tables")
+    wl = workload(4, 1)
+    t = O.ModelTables(wl)
+    ctx = make_context(wl, t, 64)
+    products = [_abi.Product.caplet(0.5, 0.5, 0.01 + 1e-6 * i) for i in range(30_000)]
+    ctx.value_products(products)
+    ctx.value_products(products)
+    ms = ctx.timings()
+    assert ms[0] == 0.0 and ms[4] - ms[1] - ms[2] > 0.02
