@@ -43,20 +43,20 @@ namespace fm {
 
 typedef const double __attribute__((address_space(4)))* RecPtr;
 
-// A record read whole into scalar registers (64-byte pieces).
+// A record read whole into scalar registers (pieces of at most 64 bytes; a record is aligned to its size, or to 64).
 template <int FCAP>
 struct RecVec {
-    typedef double V __attribute__((ext_vector_type(8)));
     static constexpr int size = rec_size_of(FCAP);
-    static constexpr int N = (size + 7) / 8;
+    static constexpr int W = size < 8 ? size : 8, N = size / W;
+    typedef double V __attribute__((ext_vector_type(W)));
     V v[N];
     // record j of a time step whose first record is at rec
     __device__ __forceinline__ RecVec(RecPtr rec, int j) {
         typedef const V __attribute__((address_space(4)))* P;
 #pragma unroll
-        for (int q = 0; q < N; q++) v[q] = *(P)(rec + j * size + 8 * q);
+        for (int q = 0; q < N; q++) v[q] = *(P)(rec + j * size + W * q);
     }
-    __device__ __forceinline__ double at(int e) const { return v[e / 8][e % 8]; }
+    __device__ __forceinline__ double at(int e) const { return v[e / W][e % W]; }
     __device__ __forceinline__ double lam(int k) const { return at(k); }
     __device__ __forceinline__ double h() const { return at(FCAP); }
     __device__ __forceinline__ double zcap() const { return at(FCAP + 1); }
