@@ -438,7 +438,8 @@ void prepare_model(fm_lmm* c) {
     std::vector<double> l0d, y0;
     Staged& up = c->model;
     up.begin();
-    size_t at_lvb = 0, at_L0 = 0, at_Y0 = 0, at_lead = 0, at_rec;
+    constexpr size_t kNone = ~(size_t)0;        // a table of the other precision
+    size_t at_lvb, at_L0 = kNone, at_Y0 = kNone, at_lead = kNone, at_rec;
     if (c->fp32()) {
         // initial state of the carried schemes (LMM.getInitialState:1081-1093): log(max(L_j(0), 0)) or
         // L_j(0), uncapped
@@ -462,12 +463,13 @@ void prepare_model(fm_lmm* c) {
     const size_t at_z0 = up.add(z0);
     if (!g_no_alloc) up.reserve(s, c->model_bytes());
     const char* base = up.send(s);
+    auto table = [&](size_t at) { return at == kNone ? nullptr : (const double*)(base + at); };
     c->m_rec = base + at_rec;
     c->m_lvb = base + at_lvb;
-    c->m_L0 = (const double*)(base + at_L0);
-    c->m_Y0 = (const double*)(base + at_Y0);
-    c->m_lead = (const double*)(base + at_lead);
-    c->m_z0 = (const double*)(base + at_z0);
+    c->m_L0 = table(at_L0);
+    c->m_Y0 = table(at_Y0);
+    c->m_lead = table(at_lead);
+    c->m_z0 = table(at_z0);
     // terminal measure N(T_0): the Scalar chain of the time-0 values (LMM:1028-1042,
     // stochastic/Scalar.java:320-328)
     c->n0_terminal = 1.0;
@@ -1810,7 +1812,7 @@ int fm_lmm_adjoint(fm_lmm* c, const fm_product* products, int32_t count, const d
     a.lognormal = c->cfg.state_space == FM_STATE_SPACE_LOGNORMAL ? 1 : 0;
     a.capped = std::isinf(c->cfg.libor_cap) ? 0 : 1;
     a.delta = c->d_delta.as<double>();
-    a.L0 = c->m_L0; a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
+    a.dw = c->d_dw.p; a.cap = c->cfg.libor_cap; a.scheme = c->cfg.scheme;
     a.rec_n = c->rec_n();
     a.lead = c->m_lead;
     a.walk = c->m_walk;           // uploaded by the pricing pass

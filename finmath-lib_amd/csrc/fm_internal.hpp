@@ -103,15 +103,16 @@ struct StepArgs {
     const void* rec;             // device [nT][rec_n][rec_size_of(factor capacity)] records (double or float)
     const void *model, *tables;  // FP64 kernels: the model's records and the products' tables, whole, and their
     int model_lines, table_lines;   // sizes in lines of 128 bytes
-    int rec_n;                   // records per time step (n, or n rounded up to even for the spot kernels)
+    int rec_n;                   // records per time step: n rounded up to even, n for the FP32 general kernel
     int lognormal, capped;       // state space is LOGNORMAL; the liborCap applies
     const double* delta;         // device n: T_{j+1}-T_j
-    const double* L0;            // device n: initial forwards in value space
+    const double* L0;            // FP32 general kernel, device n: the initial forwards (float-rounded)
     const double* lead;          // FP64 kernels, device [2][n]: the forwards' scales s_j and 1/s_j
     const void* walk;            // spot kernels, device [rows][8]: walk tables of swaption groups (path precision)
-    const double* Y0;            // device n: initial states (log(max(L0, 0)) or L0) of the carried schemes;
-                                 // for the log-forward and spot kernels kept below log(cap)
-                                 // (the spot kernel in the normal state space: the capped forwards)
+    const double* Y0;            // initial states. FP64, device 80: log2(L0 / s_j), -1e9 for zero, capped where the
+                                 // scheme caps the state (normal state space: the forwards). FP32 spot, device 80:
+                                 // the capped forwards. FP32 general, device n: log(max(L0, 0)) or L0, for the
+                                 // carried schemes
     int terminal;                // TERMINAL measure (general kernel)
     int carry;                   // EULER / PREDICTOR_CORRECTOR: the state is carried (general kernel)
     int pc;                      // predictor-corrector (general kernel)

@@ -48,14 +48,12 @@ __host__ __device__ inline double fm_log(double x) {
     return r;
 }
 
-// a / b by the hardware reciprocal estimate refined with two Newton-Raphson steps
-// (r <- r + r (1 - b r)) and one correction of the quotient (q <- q + r (a - b q)). For finite
-// b of moderate exponent (the path kernels divide by 1 + L d or L + 1/d) the result is
-// within one unit in the last place of the correctly rounded quotient and almost always
-// equal to it; b = +-inf gives NaN instead of zero. Seven instructions against the eleven
-// of the scaled IEEE division sequence.
-// fm_rcp_nr(b) is the refined reciprocal, fm_div_nr_r(a, b, r) the quotient from it: divisions of
-// several numerators by one b share the reciprocal and give the same results as fm_div_nr.
+// 1 / b by the hardware reciprocal estimate refined with two Newton-Raphson steps (r <- r + r (1 - b r)),
+// and a / b from it with one correction of the quotient (q <- q + r (a - b q)). For finite b of
+// moderate exponent (the path kernels divide by 1 + L d or L + 1/d) the quotient is within one unit
+// in the last place of the correctly rounded one and almost always equal to it; b = +-inf gives NaN
+// instead of zero. Seven instructions against the eleven of the scaled IEEE division sequence, and
+// numerators with one divisor share the reciprocal.
 __device__ __forceinline__ double fm_rcp_nr(double b) {
     double r = __builtin_amdgcn_rcp(b);
     double e = fma(-b, r, 1.0);
@@ -68,8 +66,6 @@ __device__ __forceinline__ double fm_div_nr_r(double a, double b, double r) {
     const double q = a * r;
     return fma(r, fma(-b, q, a), q);
 }
-
-__device__ __forceinline__ double fm_div_nr(double a, double b) { return fm_div_nr_r(a, b, fm_rcp_nr(b)); }
 
 // The coefficients of fm_exp2 in scalar registers, made once before a kernel's loops (an FP64 operand
 // cannot be a literal on this target). The empty asm hides their values: as known constants the
@@ -89,8 +85,8 @@ struct Exp2Coef {
 };
 
 // 2^x. x = n + r with n the nearest integer (both exact), 2^r = 1 + r q(r) with q the minimax
-// polynomial of degree 10 on [-1/2, 1/2] (relative error below 1.8e-17, Remez exchange in 60-digit
-// arithmetic), scaled by ldexp, which also gives the underflow to zero and the overflow to
+// polynomial of degree 10 on [-1/2, 1/2] (Remez exchange in 60-digit arithmetic; relative error of 2^r below
+// 1.8e-17, below 4.3e-17 with the coefficients rounded to double), scaled by ldexp, which also gives the underflow to zero and the overflow to
 // infinity: within one unit in the last place. NaN propagates; an infinite x gives NaN, so a state
 // that stands for log2(0) is held as the lowest finite number instead.
 __device__ __forceinline__ double fm_exp2(double x, const Exp2Coef& k) {

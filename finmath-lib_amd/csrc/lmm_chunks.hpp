@@ -67,10 +67,7 @@ struct ChunkedForwards {
     }
 };
 
-template <typename real> __device__ __forceinline__ real spot_div(real a, real b);
-template <> __device__ __forceinline__ double spot_div<double>(double a, double b) { return fm_div_nr(a, b); }
-template <> __device__ __forceinline__ float spot_div<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-// spot_div split at the reciprocal of b, for numerators sharing one divisor (same results)
+// a / b by the reciprocal of b, which numerators with one divisor share
 template <typename real> __device__ __forceinline__ real spot_rcp(real b);
 template <> __device__ __forceinline__ double spot_rcp<double>(double b) { return fm_rcp_nr(b); }
 template <> __device__ __forceinline__ float spot_rcp<float>(float b) { return __builtin_amdgcn_rcpf(b); }

@@ -52,7 +52,7 @@ template <int FCAP, typename real, bool TERMINAL, bool LV>
 __device__ __forceinline__ real drift_component(real (&S)[FCAP], const Rec<FCAP, real>& R, real Lj, bool lognormal,
                                                 real f, real sv) {
     auto lam = [&](int k) -> real { return LV ? (R.lam(k) * f) * sv : R.lam(k); };
-    real w = spot_div<real>((real)1.0, Lj * R.c1() + R.c2());
+    real w = spot_rcp<real>(Lj * R.c1() + R.c2());
     if (lognormal) w = w * Lj;
     real mu;
     if (TERMINAL) {

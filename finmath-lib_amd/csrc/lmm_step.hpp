@@ -57,11 +57,9 @@ __device__ __forceinline__ double wave_reduce_sum(double v) {
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// The hardware base-2 exponential and logarithm (about 1 ulp each). FP32 only: the FP64 kernels carry base-2 states.
 template <typename real> __device__ __forceinline__ real dev_exp(real x);
 template <typename real> __device__ __forceinline__ real dev_log(real x);
-template <> __device__ __forceinline__ double dev_exp<double>(double x) { return exp(x); }
-template <> __device__ __forceinline__ double dev_log<double>(double x) { return fm_log(x); }
-// FP32 form: the hardware base-2 exponential and logarithm (about 1 ulp each).
 template <> __device__ __forceinline__ float dev_exp<float>(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 template <> __device__ __forceinline__ float dev_log<float>(float x) { return __builtin_amdgcn_logf(x) * 0.693147180559945309f; }
 
