@@ -1183,7 +1183,7 @@ void run_pass(fm_lmm* c, const Lowered& L, bool store, std::vector<double>& sums
         a.Y0 = c->m_z0;
         a.lead = c->m_lead;
         const size_t value_bytes = (size_t)(L.num_slots + n + 1) * P * sizeof(double);
-        if (c->spot64() && !ckpt && !xs && P <= kRowKernelPaths && value_bytes <= kRowKernelBytes) {
+        if (c->spot64() && !ckpt && !xs && P <= row_kernel_paths(n, c->F()) && value_bytes <= kRowKernelBytes) {
             a.values = (double*)c->d_values.get(value_bytes);
             launch_lmm_rows_fp64(a, s);
         } else if (c->spot64()) launch_lmm_step_fp64(a, s);

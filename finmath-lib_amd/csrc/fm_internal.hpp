@@ -143,15 +143,34 @@ struct StepArgs {
                                  // each checkpoint's segment on (lower rows are neither written nor read)
 };
 void launch_lmm_step_fp64(const StepArgs& a, void* stream);
-// Up to this many paths the row kernel (lmm_rows64.hpp) prices and simulates: two of its wavefronts of four paths
-// for each of the 1,024 SIMDs. Both give the same results. Whole calls when a call took some 150 us more on the
-// host than it does now, row kernel against the other, 40 forwards x 5 factors with 20 swaptions and a swap:
-// 357 us against 425 at 2,000 paths, 404 against 424 at 8,000, 534 against 415 at 12,000; 80 x 10: 640
-// against 1091, 1188 against 1467, 1623 against 1464; 20 x 3: 257 against 280, 278 against 278, 299 against 277.
+// Up to how many paths the row kernel (lmm_rows64.hpp) prices and simulates. Both kernels give the same results.
+// Its time has steps at 4,096 and 8,192 paths, one and two of its wavefronts of four paths for each of the 1,024
+// SIMDs; the other's is that of one wavefront, whatever the paths. Whole calls with new model tables and up to 30
+// swaptions, us, row kernel / other:
+//   forwards x factors   1,000     2,000     4,000     5,000     6,000     8,000     9,000 paths
+//   10 x 1               76/67     77/67     80/68               83/69     88/67
+//   12 x 5               84/79     87/79     93/79     93/79     95/79     100/80
+//   20 x 3               122/125   123/125   127/126             137/125   154/126
+//   24 x 5               126/148   132/149   138/149   146/150   152/150   163/150
+//   28 x 5               136/173   141/174   148/173   164/175   162/174   174/175
+//   40 x 5               192/251   204/253   208/251             238/250   259/251
+//   48 x 5               215/322   227/323   238/325   259/358   268/323   292/324   390/328
+//   60 x 3               270/415   287/415   296/415   460/441   462/414   470/413   633/423
+//   80 x 5               392/653   411/652   421/651   670/708   673/649   682/650   928/696
+//   6 x 6                71/57     63/57     67/57     67/57     68/59     73/58
+//   12 x 10              80/94     85/95     93/95     96/95     96/94     106/95
+//   16 x 10              107/131   110/131   123/132   126/132   129/132   142/132   149/133
+//   28 x 10              151/238   156/237   177/238   189/242   198/238   231/239
+//   48 x 10              244/454   248/458   300/455   459/516   464/456   471/463
+//   80 x 10              483/987   500/989   600/992             950/1046  963/1105  1301/1143 (10,000)
 // It does not write checkpoints, and its table of values is not planned for in caller scratch.
-constexpr int kRowKernelPaths = 8192;
+constexpr int row_kernel_paths(int n, int F) {
+    if (F <= 5) return n < 16 ? 0 : n < 28 || n > 48 ? 4096 : 8192;
+    return n < 8 ? 0 : n < 14 ? 4096 : 8192;
+}
 // Its table of values is 32 times the partials' size and stays with the context, so it is bounded: 4,096 products
-// at 8,192 paths.
+// at 8,192 paths. Products make no difference between the kernels there (20 x 3: 4,000 caplets on 2,000 paths 3.32
+// and 3.33 ms, 16,000 14.0 and 13.3 ms, 4,000 on 8,000 paths 3.7 and 3.3 ms).
 constexpr size_t kRowKernelBytes = (size_t)256 << 20;
 void launch_lmm_rows_fp64(const StepArgs& a, void* stream);
 void launch_lmm_step_fp32(const StepArgs& a, void* stream);

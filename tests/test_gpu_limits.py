@@ -193,7 +193,7 @@ def test_many_products_on_few_paths(count, P):
     """More lowered products than 65,536, and tables of values on both sides of the size up to which the kernel for few
     paths runs: values and errors are those of the kernel for many paths, bit for bit."""
     say(f"case many products {count} P={P}")
-    wl = workload(4, 2)
+    wl = workload(28, 2)
     t = O.ModelTables(wl)
     ctx = make_context(wl, t, P)
     products = [_abi.Product.caplet(0.5 * (i % 4), 0.5, 0.01 + 1e-7 * i) for i in range(count)]
@@ -203,15 +203,15 @@ def test_many_products_on_few_paths(count, P):
 
 
 def test_swaps_of_many_periods_on_few_paths():
-    """66,000 periods of 16,500 swaps: each is worth the same swap's alone."""
+    """67,200 periods of 2,400 swaps: each is worth the same swap's alone."""
     say("case many swap periods")
-    wl = workload(4, 2)
+    wl = workload(28, 2)
     t = O.ModelTables(wl)
     ctx = make_context(wl, t, 70)
     products = to_products([wl.products[-1]])
     v, e = ctx.value_products(products)
-    w, f = ctx.value_products(products * 16_500)
-    assert np.array_equal(w, np.full(16_500, v[0])) and np.array_equal(f, np.full(16_500, e[0]))
+    w, f = ctx.value_products(products * 2_400)
+    assert np.array_equal(w, np.full(2_400, v[0])) and np.array_equal(f, np.full(2_400, e[0]))
 
 
 def test_more_partials_than_a_grid_dimension():
@@ -278,3 +278,20 @@ def test_the_whole_call_includes_its_product_tables():
     ctx.value_products(products)
     ms = ctx.timings()
     assert ms[0] == 0.0 and ms[4] - ms[1] - ms[2] > 0.02
+
+
+# ---- few paths: the line between the two FP64 spot kernels -----------------------------------------
+
+@pytest.mark.parametrize("n,F", [(7, 7), (8, 6), (8, 8), (13, 10), (14, 8), (15, 5), (16, 1), (16, 3), (16, 5), (16, 10), (27, 2),
+                                 (28, 4), (48, 5), (49, 5), (80, 8)])
+@pytest.mark.parametrize("P", [63, 4096, 4097, 8193])
+def test_few_paths_are_priced_as_many(n, F, P):
+    """Values and errors of either kernel are equal bit for bit: a call without allocation takes the one for many paths."""
+    say(f"case few paths n={n} F={F} P={P}")
+    wl = workload(n, F)
+    t = O.ModelTables(wl)
+    ctx = make_context(wl, t, P)
+    products = to_products([s for s in wl.products if s["type"] == "swaption"]) + [_abi.Product.caplet(0.5 * (n // 2), 0.5, 0.025)]
+    v, e = ctx.value_products(products)
+    w, f = ctx.value_products_noalloc(products)
+    assert np.array_equal(v, w) and np.array_equal(e, f)
