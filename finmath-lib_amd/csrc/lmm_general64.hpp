@@ -131,38 +131,31 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
         }
         return zn;
     };
-    const int moved = opaque(first);        // the forwards below are fixed
-    const int special = opaque(WALK && sw->periods > 0 ? n : first);    // pairs below walk or have a fixed forward
-    if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
+    if constexpr (WALK)
+        walk_fixed64<FCAP>(Y, s.recs, first, *sw, [&](double x, int j) -> double {
+            return value(x, s.recs[j * RecVec<FCAP>::size + FCAP + 1]);
+        }, reciprocal);
+    first = opaque(first);
     const unsigned alive = (unsigned)(n - first + 1);
     static_for<0, 4 * NCH>([&](auto Q) {
         constexpr int q = decltype(Q)::value;
         constexpr int j = 2 * (TERMINAL ? 4 * NCH - 1 - q : q);
         if ((unsigned)(j + 1 - first) < alive) {        // j + 1 >= first and j < n
+            // (under the terminal measure the fixed forward comes last)
+            if (WALK && __builtin_expect(j < first, 0)) set_aside_fixed64<lognormal, FCAP, j, false>(Y, s.recs);
             const RecVec<FCAP> R0(s.recs, j), R1(s.recs, j + 1);
             typedef double V4 __attribute__((ext_vector_type(4)));
             typedef const V4 __attribute__((address_space(4)))* P4;
             V4 l = {0.0, 1.0, 0.0, 1.0};
             if constexpr (LV) l = *(P4)(s.lv + 2 * j);
             __builtin_amdgcn_sched_barrier(0);          // the records are requested before the exponentials
-            double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
-            double E0 = value(x0, R0.zcap()), E1 = value(x1, R1.zcap());
-            double r0 = reciprocal(E0 + R0.e()), r1 = reciprocal(E1 + R1.e());
-            if (WALK && j < special) {
-                asm volatile("");       // a branch, not selects
+            const double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
+            const double E0 = value(x0, R0.zcap()), E1 = value(x1, R1.zcap());
+            const double r0 = reciprocal(E0 + R0.e()), r1 = reciprocal(E1 + R1.e());
+            if constexpr (WALK) {
                 if (sw->periods > 0) {
-                    sw->period(j, E0, R0.e(), r0);
+                    if (j >= first) sw->period(j, E0, R0.e(), r0);
                     sw->period(j + 1, E1, R1.e(), r1);
-                }
-                // a fixed forward has no weights: an infinite one times no loading is NaN (under the terminal
-                // measure it comes last)
-                if (j < moved) {
-                    E0 = r0 = 0.0;
-                    if constexpr (PC) x0 = 0.0;
-                    if (j + 1 < moved) {
-                        E1 = r1 = 0.0;
-                        if constexpr (PC) x1 = 0.0;
-                    }
                 }
             }
             double y0, y1;
@@ -178,11 +171,6 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
                 asm volatile("");       // a branch, not selects
                 y0 = jmin(y0, R0.zcap());
                 y1 = jmin(y1, R1.zcap());
-            }
-            if (PC && WALK && j < moved) {
-                asm volatile("");
-                y0 = Y.template at<j>();
-                if (j + 1 < moved) y1 = Y.template at<j + 1>();
             }
             Y.template put<j>(y0);
             Y.template put<j + 1>(y1);

@@ -12,8 +12,8 @@
 // Components are unrolled over the register array in pairs, as in lmm_spot64.hpp: a constant register
 // index needs no indexed move, and two independent chains cover the latency of the transcendental
 // unit and of the record loads. Where the alive range starts or ends at an odd index, the pair's other
-// forward has a record without loadings and, if it is fixed (and may have overflowed), no weight, which adds
-// exact zeros to the sums; it keeps its value.
+// forward has a record without loadings, which adds exact zeros to the sums, and keeps its value (a fixed one
+// that has overflowed is set aside first).
 //
 // The kernel is bound by vector issue: 40 forwards x 5 factors x 4,000,000 paths with 30 swaptions 3.7 ms
 // at 1.0 vector ALU busy (5.53 ms and 0.72 with rolled loops and one record read per component), 80 x 10 x
@@ -106,6 +106,16 @@ __device__ __forceinline__ void spot32_step(Chunks& Y, int n, int rec_n, int i, 
         if ((unsigned)(j + 1 - first) < alive) {        // j + 1 >= first and j < n
             PairRec32<FCAP>& R = (j & 2) ? B : A;
             R.arrive();
+            if (__builtin_expect(j < first, 0)) {
+                // the fixed one of the pair: its weight times no loading is zero unless it is NaN (an infinite forward,
+                // log-normal) or infinite (one of -1/d, normal): then the path's value, used no more, is set to zero
+                const float x = Y.template at<j>();
+                const bool lost = lognormal ? !(x < HUGE_VALF) : fmaf(x, R.c1(0), R.c2(0)) == 0.0f;
+                if (__builtin_amdgcn_ballot_w64(lost) != 0) {
+                    asm volatile("");       // hardly ever
+                    Y.template put<j>(lost ? 0.0f : x);
+                }
+            }
             ((j & 2) ? A : B).read(recs, j + 2);
             __builtin_amdgcn_sched_barrier(0);
             const float L0 = Y.template at<j>(), L1 = Y.template at<j + 1>();
@@ -113,12 +123,7 @@ __device__ __forceinline__ void spot32_step(Chunks& Y, int n, int rec_n, int i, 
             const float l1 = lognormal ? __builtin_amdgcn_logf(L1) : 0.0f;
             const float r0 = __builtin_amdgcn_rcpf(fmaf(L0, R.c1(0), R.c2(0)));
             const float r1 = __builtin_amdgcn_rcpf(fmaf(L1, R.c1(1), R.c2(1)));
-            float w0 = lognormal ? L0 * r0 : r0;
-            if (j < first) {                            // no weight: an infinite one times no loading is NaN
-                asm volatile("");       // a branch, not a select
-                w0 = 0.0f;
-            }
-            float v0 = component(std::integral_constant<int, 0>{}, L0, l0, w0, R);
+            float v0 = component(std::integral_constant<int, 0>{}, L0, l0, lognormal ? L0 * r0 : r0, R);
             float v1 = component(std::integral_constant<int, 1>{}, L1, l1, lognormal ? L1 * r1 : r1, R);
             // the cap seldom binds: one comparison each (min(v, cap) keeps NaN, as a comparison does)
             if (__builtin_amdgcn_ballot_w64(v0 > cap || v1 > cap) != 0) {

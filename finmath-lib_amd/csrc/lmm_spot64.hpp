@@ -20,8 +20,8 @@
 // and reciprocals are independent, which hides the latency of the FP64 pipeline and of the scalar
 // loads of the two records, and a constant register index needs no indexed moves. A pair holds a
 // fixed or absent forward beside an alive one where the alive range starts or ends at an odd
-// index: its record has no loadings, and a fixed one has no weight either (it may have overflowed), so it
-// adds an exact zero to every sum and to its state.
+// index: its record has no loadings, so it adds an exact zero to every sum and to its state (a fixed
+// forward that has overflowed is set aside first).
 //
 // Swaptions that exercise at t_i over consecutive tenor periods are valued by the same walk
 // (SwaptionWalk): it has E_j and the reciprocal at hand, so a period of a swaption costs two
@@ -106,8 +106,36 @@ __device__ __forceinline__ void touch_tables(ArgPtr a) {
 #endif
 }
 
+// The fixed forward J, which shares a pair with the first alive one: its record has no loadings, so a finite weight
+// adds exact zeros, but an infinite one times zero is NaN. Where a path's weight may not be finite, in the log-normal state
+// space where 2^z overflows and in the normal one where L or 1/(L + 1/d) does, the state is set to zero (a fixed
+// forward is used no more). At the start of a pair this splits none of its work; a test of the weight in
+// its midst cost the spot kernel 1 % and the kernels with a corrector 5 to 25 %. BRANCH: without a lost path the
+// state is left alone; the general kernel spills hundreds of scalar registers with that branch, the reverse
+// sweep without it.
+template <bool lognormal, int FCAP, int J, bool BRANCH, typename Chunks>
+__device__ __forceinline__ void set_aside_fixed64(Chunks& Y, RecPtr recs) {
+    const double x = Y.template at<J>();
+    const bool lost = lognormal ? !(x < 1000.0) : !(fabs(x) < 1e300) || x + recs[J * RecVec<FCAP>::size + FCAP + 2] == 0.0;
+    if (BRANCH && __builtin_amdgcn_ballot_w64(lost) == 0) return;
+    if constexpr (BRANCH) asm volatile("");         // hardly ever
+    Y.template put<J>(lost ? 0.0 : x);
+}
+
+// The walk of the fixed forwards [sw.j0, first) before a step; value(x, j) is E_j.
+template <int FCAP, typename Chunks, typename Value, typename Reciprocal>
+__device__ __forceinline__ void walk_fixed64(Chunks& Y, RecPtr recs, int first, SwaptionWalk& sw, Value&& value,
+                                             Reciprocal&& reciprocal) {
+    if (sw.periods == 0) return;
+#pragma unroll 1
+    for (int j = sw.j0; j < first; j++) {
+        const double E = value(Y.get(j), j), e = recs[j * RecVec<FCAP>::size + FCAP + 2];
+        sw.period(j, E, e, reciprocal(E + e));
+    }
+}
+
 // One Euler step of the alive components [first, n), in place. WALK: the walk's swaptions are valued
-// on the states before the step, which also passes over their forwards that are fixed at t_i.
+// on the states before the step, their forwards that are fixed at t_i ahead of it.
 template <int NCH, int FCAP, bool lognormal, bool WALK, typename Chunks>
 __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, int first, double dt,
                                             const double (&dW)[FCAP], const double* rec, const Exp2Coef& ke,
@@ -135,19 +163,20 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
         for (int k = 0; k < FCAP; k++) inc = fma(T[k], R.lam(k), inc);
         return inc;
     };
-    const int moved = opaque(first);        // the forwards below are fixed
-    const int special = opaque(WALK && sw->periods > 0 ? n : first);    // pairs below walk or have a fixed forward
-    if (WALK && sw->periods > 0 && sw->j0 < first) first = sw->j0;
+    if constexpr (WALK)
+        walk_fixed64<FCAP>(Y, recs, first, *sw, [&](double x, int) -> double { return lognormal ? fm_exp2(x, ke) : x; }, reciprocal);
     n = opaque(n);
+    first = opaque(first);
     const unsigned alive = (unsigned)(n - first + 1);
     static_for<0, 4 * NCH>([&](auto Q) {
         constexpr int j = 2 * decltype(Q)::value;
         if ((unsigned)(j + 1 - first) < alive) {        // j + 1 >= first and j < n
+            if (__builtin_expect(j < opaque(first), 0)) set_aside_fixed64<lognormal, FCAP, j, true>(Y, recs);
             const RecVec<FCAP> R0(recs, j), R1(recs, j + 1);
             __builtin_amdgcn_sched_barrier(0);          // both records are requested before the exponentials
             const double x0 = Y.template at<j>(), x1 = Y.template at<j + 1>();
-            double E0 = lognormal ? fm_exp2(x0, ke) : x0;
-            double E1 = lognormal ? fm_exp2(x1, ke) : x1;
+            const double E0 = lognormal ? fm_exp2(x0, ke) : x0;
+            const double E1 = lognormal ? fm_exp2(x1, ke) : x1;
             const double b0 = E0 + R0.e(), b1 = E1 + R1.e();
             // the next pair's records are brought into the scalar cache while this one runs (the table
             // of a model is several times that cache); a pair beyond the last reads its last record
@@ -155,30 +184,19 @@ __device__ __forceinline__ void spot64_step(Chunks& Y, int n, int rec_n, int i, 
             typedef const volatile uint32_t __attribute__((address_space(4)))* WordPtr;
             constexpr int step = RecVec<FCAP>::size;
             uint32_t t0 = *(WordPtr)(recs + (j + 2) * step), t1 = *(WordPtr)(recs + (j + 3) * step);
-            double r0 = reciprocal(b0), r1 = reciprocal(b1);
-            if (WALK && j < special) {
-                asm volatile("");       // a branch, not selects
+            const double r0 = reciprocal(b0), r1 = reciprocal(b1);
+            if constexpr (WALK) {
                 if (sw->periods > 0) {
                     const uint32_t t2 = sw->touch(j + 2), t3 = sw->touch(j + 3);
-                    sw->period(j, E0, R0.e(), r0);
+                    if (j >= opaque(first)) sw->period(j, E0, R0.e(), r0);
                     sw->period(j + 1, E1, R1.e(), r1);
 #if defined(__HIP_DEVICE_COMPILE__)
                     asm volatile("" :: "s"(t2), "s"(t3));
 #endif
                 }
-                if (j < moved) {        // no weight: an infinite one times no loading is NaN
-                    E0 = r0 = 0.0;
-                    if (j + 1 < moved) E1 = r1 = 0.0;
-                }
             }
-            double w0 = (lognormal ? cdt * E0 : cdt) * r0;
-            const double w1 = (lognormal ? cdt * E1 : cdt) * r1;
-            if (!WALK && j < moved) {
-                asm volatile("");
-                w0 = 0.0;
-            }
-            double y0 = x0 + increment(w0, R0);
-            double y1 = x1 + increment(w1, R1);
+            double y0 = x0 + increment((lognormal ? cdt * E0 : cdt) * r0, R0);
+            double y1 = x1 + increment((lognormal ? cdt * E1 : cdt) * r1, R1);
             // the cap seldom binds: one comparison each (min(y, cap) keeps NaN, as a comparison does)
             if (__builtin_amdgcn_ballot_w64(y0 > R0.zcap() || y1 > R1.zcap()) != 0) {
                 asm volatile("");       // a branch, not selects
