@@ -85,10 +85,11 @@ struct Exp2Coef {
 };
 
 // 2^x. x = n + r with n the nearest integer (both exact), 2^r = 1 + r q(r) with q the minimax
-// polynomial of degree 10 on [-1/2, 1/2] (Remez exchange in 60-digit arithmetic; relative error of 2^r below
-// 1.8e-17, below 4.3e-17 with the coefficients rounded to double), scaled by ldexp, which also gives the underflow to zero and the overflow to
-// infinity: within one unit in the last place. NaN propagates; an infinite x gives NaN, so a state
-// that stands for log2(0) is held as the lowest finite number instead.
+// polynomial of degree 10 on [-1/2, 1/2] (Remez exchange in 60-digit arithmetic; relative error of 2^r
+// below 1.8e-17, below 4.3e-17 with the coefficients rounded to double), scaled by ldexp, which also gives
+// the underflow to zero and the overflow to infinity: within one unit in the last place. NaN
+// propagates; an infinite x gives NaN, so a state that stands for log2(0) is held as a finite
+// number whose power underflows instead.
 __device__ __forceinline__ double fm_exp2(double x, const Exp2Coef& k) {
     const double n = __builtin_rint(x);
     const double r = x - n;

@@ -20,9 +20,9 @@
 // Carried schemes cap the value min(2^z, cap/s_j) where it is read; functional ones cap the state.
 //
 // The FP64 vector pipeline bounds it, as it does the spot kernel. 200,000 paths, 40 forwards,
-// 5 factors, 40 steps, terminal measure, PREDICTOR_CORRECTOR: 0.93 ms
+// 5 factors, 40 steps, terminal measure, PREDICTOR_CORRECTOR: 0.86 ms
 // (1.86 ms for the kernel with natural exponentials, divisions and rolled components that this one replaces);
-// 150,000 paths, spot measure, normal, stochastic volatility: 0.34 ms (1.50 ms).
+// 150,000 paths, spot measure, normal, stochastic volatility: 0.31 ms (1.50 ms).
 #pragma once
 
 #include "lmm_spot64.hpp"
@@ -183,7 +183,7 @@ __device__ __forceinline__ void general64_step(Chunks& Y, const General64& s, co
 //
 // Four waves per SIMD where the registers allow them without scratch memory (the spot measure's corrector and
 // the wrappers need up to 167, three waves): at 200,000 paths three are one pass and a nearly empty
-// second one, 1.00 ms against 0.93.
+// second one, 1.00 ms against 0.93 (before the model's tables were touched ahead, which took the four to 0.86).
 template <int NCH, int FCAP, bool TERMINAL, bool PC, bool LV, bool lognormal>
 __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(NCH <= 5 && FCAP <= 5 ? (LV || (PC && !TERMINAL) ? 3 : 4) : 1)))
 lmm_general64_kernel(const StepArgs) {

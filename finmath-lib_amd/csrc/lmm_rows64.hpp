@@ -16,7 +16,8 @@
 // A lane's records of the next step (its own, and column k of the row's sixteen) are requested as soon
 // as this step's are used: with one or two wavefronts per SIMD nothing else hides their latency.
 // It is bound by latency: of a wavefront's time about 0.4 are waits for loads and the LDS and 0.25 vector
-// instructions. 2,000 paths, 40 forwards x 5 factors, 30 swaptions: 112 us (291 us for lmm_spot_kernel).
+// instructions. 2,000 paths, 40 forwards x 5 factors, 30 swaptions: 117 us (187 us for lmm_spot_kernel); 80 x 10 and 4,000
+// paths: 400 us (815 us).
 //
 // Values to be averaged go to a table [column][P], and rows64_partials_kernel forms from it the partials
 // of 64 paths, in the operations of lmm_spot_kernel.

@@ -29,9 +29,9 @@
 // exponential and another reciprocal.
 //
 // The kernel is bound by the FP64 vector pipeline. At 40 forwards x 5 factors x 1,000,000 paths with 30
-// swaptions it issues 38,500 vector instructions per wavefront (80,400 with rolled component loops,
-// a general exponential and separate products and sums) and takes 1.54 ms (3.46 ms), the vector ALUs
-// 0.79 busy (0.67) at four wavefronts per SIMD (three): the registers are held to 128 by reading the
+// swaptions it issues 38,600 vector instructions per wavefront (80,400 with rolled component loops,
+// a general exponential and separate products and sums) and takes 1.55 ms (3.46 ms), the vector ALUs
+// 0.78 busy (0.67) at four wavefronts per SIMD (three): the registers are held to 128 by reading the
 // kernel's arguments where they are used and the increments when the step begins. Bringing the next
 // pair's records into the scalar cache took it from 1.88 to 1.79 ms at three wavefronts; two sets of
 // scalar registers for them instead spilled.

@@ -26,8 +26,8 @@
 //
 // The two register arrays leave two wavefronts per SIMD at 80 FP32 or 40 FP64 forwards, so the sweep
 // waits on scalar loads and on the vector pipeline in turn. 80 forwards x 10 factors x 1,000,000 FP32
-// paths: 20.7 ms (22.2 ms at 0.61 vector ALU busy while the bounds of the unrolled loops were hoisted as masks and
-// spilled; 29.3 ms at 0.49 with rolled loops and every kernel argument held in spilled scalar registers); 40 x 5 x 100,001 FP64 paths with 30 swaptions: 1.21 ms (2.82 ms).
+// paths: 21.2 ms (22.2 ms at 0.61 vector ALU busy while the bounds of the unrolled loops were hoisted as masks and
+// spilled; 29.3 ms at 0.49 with rolled loops and every kernel argument held in spilled scalar registers); 40 x 5 x 100,001 FP64 paths with 30 swaptions: 1.16 ms (2.82 ms).
 //
 // Conventions of the reference's AAD (RandomVariableDifferentiableAAD.java:165-219): averages
 // over paths (the numeraire-adjustment factor) are constants, the floor of the swaption payoff
